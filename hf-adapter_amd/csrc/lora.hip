@@ -167,7 +167,7 @@ __global__ __launch_bounds__(256) void lora_up_kernel(const LoraBatch B, int row
   }
 }
 
-// Many-row form (prefills): one launch, no workspace.  A workgroup owns
+// Many-row form (prefills without a workspace, fp32, ranks above 128): one launch.  A workgroup owns
 // 64 MT rows of one problem; wave w owns rows 16 MT w .. + 16 MT - 1 (MT
 // MFMA row tiles, so every weight operand it loads feeds MT MFMAs) from start
 // to end:
@@ -329,7 +329,8 @@ extern "C" size_t rwkv7mi_lora_workspace_bytes(int64_t nprob, const int64_t* ran
   int64_t sr = 0;
   for (int64_t i = 0; i < nprob; ++i) sr += ranks[i];
   const int64_t nr = rows < LORA_ROWS ? rows : LORA_ROWS;
-  return (size_t)(ks * nr * sr) * sizeof(float);
+  // fp32 split-K partials of one row chunk, or (more rows) the 16-bit mid rows of lora_pair.hip
+  return (size_t)std::max(ks * nr * sr * (int64_t)sizeof(float), rows > LORA_PAIR_MIN ? rows * sr * 2 : (int64_t)0);
 }
 
 static int lora_run(bool up, int64_t nprob, const void* const* xs, const void* const* w_down,
@@ -387,10 +388,15 @@ static int lora_run(bool up, int64_t nprob, const void* const* xs, const void* c
   batch.kr = (int)((D + ks - 1) / ks);
   batch.kr = (batch.kr + 7) / 8 * 8;
   const size_t esz = act_dtype == RWKV7MI_F32 ? 4 : 2;
+  if (up && rows > LORA_PREFILL_ROWS &&
+      (rows * std::max(D, A) * (int64_t)esz > INT32_MAX || A * LORA_MAXR * (int64_t)esz > INT32_MAX))
+    return fail(RWKV7MI_EINVAL, "lora_multi: too large");
+  const bool full = act_dtype == RWKV7MI_F16 && (rows + 255) / 256 * nprob >= LORA_SEQ_WGS &&
+                    lora_seq_supported(batch, rows);
+  if (up && rows > LORA_PAIR_MIN && !full && lora_pair_supported(batch, rows, act_dtype, workspace, workspace_bytes))
+    return lora_pair_run(batch, rows, act_dtype, workspace, stream);
   if (up && rows > LORA_PREFILL_ROWS) {
     // many rows: the fused per-row-tile kernel, one launch, no partials
-    if (rows * std::max(D, A) * (int64_t)esz > INT32_MAX || A * LORA_MAXR * (int64_t)esz > INT32_MAX)
-      return fail(RWKV7MI_EINVAL, "lora_multi: too large");
     const int rt = (rmax + 15) / 16;
     // fp16 with ranks that are multiples of 32: weights shared through LDS, 256 rows per workgroup
     if (act_dtype == RWKV7MI_F16 && lora_seq_supported(batch, rows)) return lora_seq_run(batch, rows, stream);

@@ -8,6 +8,8 @@ namespace rwkv7mi {
 
 enum { LORA_ACT_NONE = 0, LORA_ACT_TANH = 1, LORA_ACT_SIGMOID = 2 };
 constexpr int LORA_MAXR = 256;   // largest rank
+constexpr int LORA_PAIR_MIN = 64;         // above: the two-launch pair of lora_pair.hip (fp16 / bf16)
+constexpr int LORA_SEQ_WGS = 160;         // fp16: from this many of its workgroups on, lora_seq.hip instead
 constexpr int LORA_PREFILL_ROWS = 256;  // above: the fused many-row kernel (no workspace)
 
 struct LoraProb {
@@ -25,6 +27,10 @@ struct LoraBatch {
   int tpw;  // up kernel: output tiles of 16 columns per workgroup
 };
 
+// fp16 / bf16 pair over all rows (lora_pair.hip): whether it takes these shapes
+// with this workspace (rows x the ranks' sum activations), and its launches.
+bool lora_pair_supported(const LoraBatch& b, int64_t rows, int act_dtype, const void* ws, size_t ws_bytes);
+int lora_pair_run(const LoraBatch& b, int64_t rows, int act_dtype, void* ws, void* stream);
 // Many-row fp16 form (lora_seq.hip): whether it takes these shapes, and its launch.
 bool lora_seq_supported(const LoraBatch& b, int64_t rows);
 int lora_seq_run(const LoraBatch& b, int64_t rows, void* stream);

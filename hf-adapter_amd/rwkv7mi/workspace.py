@@ -40,13 +40,18 @@ def _key(device, slot):
     return (idx, slot)
 
 
-def reserve(device: torch.device, nbytes: int, slot: str = "mm8") -> torch.Tensor:
-    """Return the device's buffer for ``slot``, growing it (zero-filled) to ``nbytes``."""
+def reserve(device: torch.device, nbytes: int, slot: str = "mm8", *, floor: int | None = None) -> torch.Tensor:
+    """Return the device's buffer for ``slot``, growing it (zero-filled) to ``nbytes``.
+
+    ``floor``: the least the call can run with.  Under graph capture a buffer
+    of at least ``floor`` bytes is returned as it is instead of raising."""
     key = _key(device, slot)
     with _lock:
         buf = _buffers.get(key)
         if buf is None or buf.numel() < nbytes:
             if torch.cuda.is_current_stream_capturing():
+                if floor is not None and buf is not None and buf.numel() >= floor:
+                    return buf
                 raise RuntimeError(
                     f"rwkv7mi workspace '{slot}' must be reserved before graph capture "
                     f"(need {nbytes} bytes on cuda:{key[0]})"

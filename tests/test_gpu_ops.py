@@ -259,6 +259,50 @@ def test_wag_lora_dtypes(oracle, dt, rows, D):
         _ok(got[q], ref, tol=1e-2 if dt == torch.bfloat16 else 1e-4)
 
 
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,D,A,ranks", [(65, 512, 264, (64, 72, 128, 8)), (257, 72, 100, (32, 96, 40, 16)),
+                                            (400, 1088, 520, (64, 64, 128, 32)), (2100, 264, 256, (24, 128, 56, 32))])
+def test_lora_row_pair_edges(oracle, dt, rows, D, A, ranks):
+    """The down / up pair over all rows: row counts that end inside a 16-, 32-
+    and 64-row tile, K that ends inside a 64-input step, ranks that end inside
+    a 16- and a 64-column block, output widths that end inside a wave's 64
+    columns and (100) inside an 8-column store; a call whose workspace is too
+    small for it runs on the other kernels and agrees with it."""
+    from rwkv7mi import _lib
+    from rwkv7mi.fused_lora import lora_multi
+    import ctypes
+
+    rng = np.random.default_rng(rows)
+    xs = [_t(rng.standard_normal((rows, D)), dt) for _ in range(4)]
+    downs = [_t(rng.standard_normal((r, D)) * 0.05, dt) for r in ranks]
+    ups = [_t(rng.standard_normal((A, r)) * 0.1, dt) for r in ranks]
+    biases = [_t(rng.standard_normal(A) * 0.1, dt), None, None, _t(rng.standard_normal(A) * 0.1, dt)]
+    acts_d, acts_u = [1, 0, 2, 0], [0, 2, 0, 2]
+    outs = [torch.full((rows, A), float("nan"), device="cuda", dtype=dt) for _ in range(4)]
+    lora_multi(xs, downs, ups, biases, outs, acts_d, acts_u)
+    alt = [torch.empty(rows, A, device="cuda", dtype=dt) for _ in range(4)]
+    small = torch.zeros(16 * min(rows, 64) * sum(ranks) * 4, device="cuda", dtype=torch.uint8)
+    small = small[: max(0, rows * sum(ranks) * 2 - 16)]
+    k64 = lambda v: (ctypes.c_int64 * 4)(*v)
+    k32 = lambda v: (ctypes.c_int * 4)(*v)
+    if rows > 256:
+        _lib.call("rwkv7mi_lora_multi", 4, _lib.ptr_array(xs), _lib.ptr_array(downs), _lib.ptr_array(ups),
+                  _lib.ptr_array(biases), _lib.ptr_array(alt), k64(ranks), k32(acts_d), k32(acts_u), rows, D, A,
+                  _lib.dtype_code(xs[0]), _lib.ptr(small), int(small.numel()), _lib.stream_of(xs[0]))
+    torch.cuda.synchronize()
+    act = {0: lambda v: v, 1: np.tanh, 2: lambda v: 1 / (1 + np.exp(-v))}
+    # one rounding of the intermediate (its ties may fall the other way: one
+    # step on some of its r values) and one of the output
+    step = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8
+    for q in range(4):
+        mid = act[acts_d[q]](_f(xs[q]) @ _f(downs[q]).T)
+        ref = act[acts_u[q]](mid @ _f(ups[q]).T + (0 if biases[q] is None else _f(biases[q])))
+        bound = step * (np.abs(ref) + np.abs(mid) @ np.abs(_f(ups[q])).T) + 1e-6
+        assert np.all(np.abs(_f(outs[q]) - ref) <= bound), q
+        if rows > 256:
+            assert np.all(np.abs(_f(alt[q]) - ref) <= bound), q
+
+
 @pytest.mark.parametrize("rows", [20, 70])
 def test_lora_rank_above_128(oracle, rows):
     """Ranks above 128 take 32-row launch pairs (64-row pairs hold ranks up to 128)."""
