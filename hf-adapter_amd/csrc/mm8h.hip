@@ -73,6 +73,9 @@ struct MhBatch {
   int rows, I, O, SB;  // SB = ceil(I / 64) steps
   int mt, nt;          // row / column tiles
   int gm, gn;          // XCD tile group: gm row tiles x gn column tiles
+  int S, sps;          // K splits and the steps of each (S > 1: fp32 partial tiles)
+  int64_t ldp;         // partials [problem][split][row][ldp]: O padded to whole 32-column pairs
+  float* part;
 };
 
 __device__ __forceinline__ int mh_key(int r) { return (r & 7) ^ ((r >> 3) & 1); }
@@ -95,10 +98,9 @@ struct MhDeqProb {
 struct MhDeqBatch {
   MhDeqProb p[MM8T_MAXPROB];
   int I, O, SB, KB;
+  int vec;  // every my / ry 16-byte aligned
 };
 
-// one thread per (column group, step, lane): the lane's 16 MM8 bytes ->
-// its two 8-half records
 // The same operand order for an fp16 nn.Linear weight W [O, I] (W_hat[k, o]
 // = W[o, k]): one thread per (column group, step, lane) copies the 16
 // inputs 16 kg .. +15 of its column into its two records.
@@ -133,6 +135,10 @@ __global__ __launch_bounds__(256) void mm8h_relayout_kernel(const MhRelBatch R) 
   }
 }
 
+// one thread per (column group, step, lane): the lane's 16 MM8 bytes -> its
+// two 8-value records.  Bound by its 3 bytes a weight; with ry / my as 16-byte
+// runs (32 two-byte loads a thread before) 67 MB of weights took 57 -> 42 us,
+// 4.8 TB/s.
 template <typename TA>
 __global__ __launch_bounds__(256) void mm8h_dequant_kernel(const MhDeqBatch D) {
   using E = typename MhTypes<TA>::E;
@@ -158,6 +164,18 @@ __global__ __launch_bounds__(256) void mm8h_dequant_kernel(const MhDeqBatch D) {
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     V v;
+    float ry8[8], my8[8];
+    if (D.vec && k0 < D.I) {  // I % 16 == 0: the lane's 16 inputs are all inside or all outside
+      ld8(ry + k0 + 8 * h, ry8);
+      ld8(my + k0 + 8 * h, my8);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int k = k0 + 8 * h + j;
+        ry8[j] = k < D.I ? to_f32(ry[k]) : 0.f;
+        my8[j] = k < D.I ? to_f32(my[k]) : 0.f;
+      }
+    }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int k = k0 + 8 * h + j;
@@ -165,7 +183,7 @@ __global__ __launch_bounds__(256) void mm8h_dequant_kernel(const MhDeqBatch D) {
       float x = 0.f;
       if (ocol && k < D.I) {
         const float wq = (float)byte + 0.5f;
-        x = wq * to_f32(ry[k]) * rxo + to_f32(my[k]) + mxo;
+        x = wq * ry8[j] * rxo + my8[j] + mxo;
       }
       v[j] = (E)x;
     }
@@ -173,8 +191,77 @@ __global__ __launch_bounds__(256) void mm8h_dequant_kernel(const MhDeqBatch D) {
   }
 }
 
-// FULLK: I is a multiple of 64 (no step ends inside a 16-byte chunk's range)
-template <bool FULLK, typename TA>
+// The tail of a column vector run: y = epilogue(v + bias), 8 columns from c0
+template <typename TA>
+__device__ __forceinline__ void mh_store8(const MhProb& P, int64_t row, int c0, int O, float (&v)[8]) {
+  using E = typename MhTypes<TA>::E;
+  using V = typename MhTypes<TA>::V;
+  const int64_t oi = row * O + c0;
+  if (P.vec && c0 + 8 <= O) {
+    if (P.epilogue == RWKV7MI_EPI_RESIDUAL) {
+      const V r = *reinterpret_cast<const V*>(reinterpret_cast<const TA*>(P.residual) + oi);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] += (float)r[e];
+    }
+    V o8;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float w = v[e];
+      if (P.epilogue == RWKV7MI_EPI_RELU2) {
+        w = fmaxf(w, 0.f);
+        w = w * w;
+      }
+      o8[e] = (E)w;
+    }
+    *reinterpret_cast<V*>(reinterpret_cast<TA*>(P.y) + oi) = o8;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      if (c0 + e >= O) continue;
+      float w = v[e];
+      if (P.epilogue == RWKV7MI_EPI_RELU2) {
+        w = fmaxf(w, 0.f);
+        w = w * w;
+      } else if (P.epilogue == RWKV7MI_EPI_RESIDUAL) {
+        w += ld(reinterpret_cast<const TA*>(P.residual), oi + e);
+      }
+      reinterpret_cast<TA*>(P.y)[oi + e] = from_f32<TA>(w);
+    }
+  }
+}
+
+// S > 1: one thread adds the S fp32 partials of 8 columns of a row in split
+// order and applies the epilogue.  Memory-bound: 4 S + 2 (+ 2) bytes a value.
+template <typename TA>
+__global__ __launch_bounds__(256) void mm8h_reduce_kernel(const MhBatch B) {
+  const MhProb& P = B.p[blockIdx.y];
+  const int cols = (int)(B.ldp / 8);
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (t >= (int64_t)B.rows * cols) return;
+  const int64_t row = t / cols;
+  const int c0 = 8 * (int)(t % cols);
+  if (c0 >= B.O) return;
+  const int64_t zs = (int64_t)B.rows * B.ldp;
+  const float* p = B.part + (int64_t)blockIdx.y * B.S * zs + row * B.ldp + c0;
+  float v[8];
+  ld8(p, v);
+  for (int z = 1; z < B.S; ++z) {
+    float a[8];
+    ld8(p + z * zs, a);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] += a[e];
+  }
+  const TA* bp = reinterpret_cast<const TA*>(P.bias);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] += bp && c0 + e < B.O ? to_f32(bp[c0 + e]) : 0.f;
+  mh_store8<TA>(P, row, c0, B.O, v);
+}
+
+// FULLK: I is a multiple of 64 (no step ends inside a 16-byte chunk's range).
+// SPLIT: blockIdx.z takes B.sps of the steps and leaves fp32 partial tiles (an
+// instance of its own: the bounds and the second epilogue cost the unsplit
+// kernel 4%)
+template <bool FULLK, bool SPLIT, typename TA>
 __global__ __launch_bounds__(MH_THREADS, 1) void mm8h_gemm_kernel(const MhBatch B) {
   using E = typename MhTypes<TA>::E;
   using V = typename MhTypes<TA>::V;
@@ -202,7 +289,9 @@ __global__ __launch_bounds__(MH_THREADS, 1) void mm8h_gemm_kernel(const MhBatch 
   const int lane = tid & 63;
   const int n = lane & 15, kg = lane >> 4;
   const int SB = B.SB;
-  const int nsteps = SB + (SB & 1);  // whole step pairs; a padding step reads zeros
+  const int sb0 = SPLIT ? (int)blockIdx.z * B.sps : 0;  // this split's steps
+  const int sb1 = SPLIT ? min(SB, sb0 + B.sps) : SB;
+  const int nsteps = (sb1 - sb0 + 1) & ~1;  // whole step pairs; a padding step reads zeros
 
   // ---- global sources (raw buffer loads; out-of-range offsets read zeros)
   const __amdgpu_buffer_rsrc_t xr = mm8t_rsrc(P.x, (uint32_t)((int64_t)M * I * 2));
@@ -234,14 +323,14 @@ __global__ __launch_bounds__(MH_THREADS, 1) void mm8h_gemm_kernel(const MhBatch 
   auto issue_x = [&](int s, int u) {
     const int st = s % MH_NST;
     const int r0 = 32 * u + 8 * wave;
-    const int so = s < SB ? 128 * s : (int)MM8T_OOB;
-    const int vo = FULLK ? xo[u] : (s == SB - 1 ? xl[u] : xo[u]);
+    const int so = sb0 + s < sb1 ? 128 * (sb0 + s) : (int)MM8T_OOB;
+    const int vo = FULLK ? xo[u] : (sb0 + s == SB - 1 ? xl[u] : xo[u]);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_ptr)(xs(st) + r0 * MH_XS), 16, vo, so, 0, 0);
   };
   // W_hat of step s for the wave's group j = 0..3, sub-step h (load 2 j + h
   // of 8): lane offset 16 lane, the rest a scalar offset
   auto issue_w = [&](int s, int j, int h, V (&bw)[4][2]) {
-    const int so = s < SB ? (j * SB + s) * (int)MH_REC + h * 1024 : (int)MM8T_OOB;
+    const int so = sb0 + s < sb1 ? (j * SB + sb0 + s) * (int)MH_REC + h * 1024 : (int)MM8T_OOB;
     bw[j][h] = __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(wr, 16 * lane, so, 0));
   };
 
@@ -322,6 +411,22 @@ __global__ __launch_bounds__(MH_THREADS, 1) void mm8h_gemm_kernel(const MhBatch 
 
   // ---- epilogue: lane holds row 16 i + n and, in groups 2 p and 2 p + 1,
   // columns c0 = 32 p + 8 kg .. +3 and c0 + 4 .. +7 of the wave's 64
+  if constexpr (SPLIT) {
+    float* part = B.part + ((int64_t)blockIdx.y * B.S + blockIdx.z) * M * B.ldp;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int c0 = n0 + 64 * wave + 32 * p + 8 * kg;
+      if (c0 >= O) continue;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int64_t row = m0 + 16 * i + n;
+        if (row >= M) continue;
+        *reinterpret_cast<f32x4*>(part + row * B.ldp + c0) = acc[i][2 * p];
+        *reinterpret_cast<f32x4*>(part + row * B.ldp + c0 + 4) = acc[i][2 * p + 1];
+      }
+    }
+    return;
+  }
   const TA* bp = reinterpret_cast<const TA*>(P.bias);
   const bool vec = P.vec;
 #pragma unroll
@@ -381,16 +486,47 @@ __global__ __launch_bounds__(MH_THREADS, 1) void mm8h_gemm_kernel(const MhBatch 
 
 using namespace rwkv7mi;
 
+// W_hat records of nprob problems
+static int64_t mh_weight_bytes(int64_t nprob, int64_t I, int64_t O) {
+  return nprob * (2 * ((O + 31) / 32)) * ((I + 63) / 64) * MH_REC;
+}
 extern "C" int64_t rwkv7mi_mm8t_gemm_prefill_ws_bytes(int nprob, int64_t I, int64_t O) {
   if (nprob < 1 || I <= 0 || O <= 0) return 0;
-  return (int64_t)nprob * (2 * ((O + 31) / 32)) * ((I + 63) / 64) * MH_REC;
+  return mh_weight_bytes(nprob, I, O);
 }
 
 namespace rwkv7mi {
+// K splits of a launch of `tiles` 256 x 256 tiles (over all problems) with SB
+// steps: fewer than one tile per CU leaves CUs idle, so K is cut into equal
+// ranges while tiles x splits <= 256.  The estimate, in us: 1.1 per step with
+// the chip nearly idle, 1.66 with every CU streaming (measured: 16384 -> 4096
+// at 1000 rows, 64 tiles, 289 us for 256 steps; 4096 -> 16384, 256 tiles, 107
+// us for 64), and the fp32 partials (part_bytes a split) written and read back
+// at about 4 TB/s plus a launch.
+static int mh_splits(int64_t tiles, int64_t I, int64_t part_bytes) {
+  if (I % 64) return 1;
+  const int64_t SB = I / 64;
+  int best = 1;
+  double cost = 1e30;
+  for (int S = 1; S <= 16 && (S == 1 || tiles * S <= 256); ++S) {
+    const int64_t sps = (SB + S - 1) / S;
+    if (S > 1 && (sps < 4 || (SB + sps - 1) / sps != S)) continue;  // no empty split
+    const double t = (sps + 6) * (1.1 + 0.56 * std::min<double>(1.0, tiles * S / 256.0)) +
+                     (S > 1 ? 5.0 + 2.0 * part_bytes * S / 4e6 : 0.0);
+    if (t < cost) cost = t, best = S;
+  }
+  return best;
+}
+static int64_t mh_tiles(int64_t nprob, int64_t rows, int64_t O) {
+  return nprob * ((rows + MH_M - 1) / MH_M) * ((O + MH_N - 1) / MH_N);
+}
+static int64_t mh_part_bytes(int64_t nprob, int64_t rows, int64_t O) {
+  return nprob * rows * ((O + 31) / 32 * 32) * 4;
+}
 // the GEMM over prepared W_hat records (b.p[i].wt), with the tile grid set here
 template <typename TA>
-static int mh_gemm_launch(MhBatch& b, int nprob, int64_t rows, int64_t I, int64_t O, void* stream,
-                          const std::string& w) {
+static int mh_gemm_launch(MhBatch& b, int nprob, int64_t rows, int64_t I, int64_t O, void* ws, int64_t ws_bytes,
+                          void* stream, const std::string& w) {
   b.rows = (int)rows;
   b.I = (int)I;
   b.O = (int)O;
@@ -402,18 +538,41 @@ static int mh_gemm_launch(MhBatch& b, int nprob, int64_t rows, int64_t I, int64_
   const int64_t T = (int64_t)((b.mt + b.gm - 1) / b.gm) * b.gm * ((b.nt + b.gn - 1) / b.gn) * b.gn;
   if (T > (int64_t)INT32_MAX / 2) return fail(RWKV7MI_EINVAL, w + ": too many tiles");
   const int64_t per = (T + 7) / 8;
+  // partials follow the weights in the workspace (a caller that gave only the
+  // weights' bytes gets no splits)
+  b.ldp = (O + 31) / 32 * 32;
+  const int64_t wb = mh_weight_bytes(nprob, I, O), pb = mh_part_bytes(nprob, rows, O);
+  b.S = mh_splits(mh_tiles(nprob, rows, O), I, pb);
+  if (ws_bytes < wb + (b.S > 1 ? b.S * pb : 0)) b.S = 1;
+  b.sps = (b.SB + b.S - 1) / b.S;
+  b.part = reinterpret_cast<float*>(static_cast<char*>(ws) + wb);
   auto launch = [&](auto kern, std::atomic<uint64_t>& raised) {
     if (int rc = raise_dynamic_lds(reinterpret_cast<const void*>(kern), MH_LDS, raised, "mm8h_gemm_kernel"))
       return rc;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(per * 8), (unsigned)nprob), dim3(MH_THREADS), MH_LDS,
+    hipLaunchKernelGGL(kern, dim3((unsigned)(per * 8), (unsigned)nprob, (unsigned)b.S), dim3(MH_THREADS), MH_LDS,
                        as_stream(stream), b);
-    return check_launch("mm8h_gemm_kernel");
+    if (int rc = check_launch("mm8h_gemm_kernel")) return rc;
+    if (b.S == 1) return (int)RWKV7MI_OK;
+    hipLaunchKernelGGL(mm8h_reduce_kernel<TA>, dim3((unsigned)((rows * (b.ldp / 8) + 255) / 256), (unsigned)nprob),
+                       dim3(256), 0, as_stream(stream), b);
+    return check_launch("mm8h_reduce_kernel");
   };
-  static std::atomic<uint64_t> raised_full{0}, raised_part{0};
-  return I % 64 == 0 ? launch(&mm8h_gemm_kernel<true, TA>, raised_full)
-                      : launch(&mm8h_gemm_kernel<false, TA>, raised_part);
+  static std::atomic<uint64_t> raised[3];
+  if (b.S > 1) return launch(&mm8h_gemm_kernel<true, true, TA>, raised[0]);
+  return I % 64 == 0 ? launch(&mm8h_gemm_kernel<true, false, TA>, raised[1])
+                     : launch(&mm8h_gemm_kernel<false, false, TA>, raised[2]);
 }
 
+}  // namespace rwkv7mi
+
+extern "C" int64_t rwkv7mi_mm8t_gemm_prefill_split_ws_bytes(int nprob, int64_t rows, int64_t I, int64_t O) {
+  if (nprob < 1 || rows <= 0 || I <= 0 || O <= 0) return 0;
+  const int64_t pb = mh_part_bytes(nprob, rows, O);
+  const int S = mh_splits(mh_tiles(nprob, rows, O), I, pb);
+  return mh_weight_bytes(nprob, I, O) + (S > 1 ? S * pb : 0);
+}
+
+namespace rwkv7mi {
 // shape, workspace and per-problem checks shared by the two entries
 static int mh_check(const std::string& w, int nprob, int64_t rows, int64_t I, int64_t O, void* ws, int64_t ws_bytes) {
   if (nprob < 1 || nprob > MM8T_MAXPROB) return fail(RWKV7MI_EINVAL, w + ": 1..4 problems per launch");
@@ -425,8 +584,7 @@ static int mh_check(const std::string& w, int nprob, int64_t rows, int64_t I, in
       rows * O > ((int64_t)1 << 40))
     return fail(RWKV7MI_EINVAL, w + ": too large (split the rows)");
   if (rows == 0) return RWKV7MI_OK;
-  const int64_t per_prob = (2 * ((O + 31) / 32)) * ((I + 63) / 64) * MH_REC;
-  if (!ws || ws_bytes < per_prob * nprob)
+  if (!ws || ws_bytes < mh_weight_bytes(nprob, I, O))
     return fail(RWKV7MI_EINVAL, w + ": workspace too small (rwkv7mi_mm8t_gemm_prefill_ws_bytes)");
   if (reinterpret_cast<uintptr_t>(ws) & 15) return fail(RWKV7MI_EINVAL, w + ": workspace must be 16-byte aligned");
   return RWKV7MI_OK;
@@ -457,7 +615,7 @@ extern "C" int rwkv7mi_mm8t_gemm_prefill_ws(int nprob, const void* const* x, con
     return fail(RWKV7MI_EINVAL, w + ": fp16 or bf16 activations with metadata of the same type");
   if (int rc = mh_check(w, nprob, rows, I, O, ws, ws_bytes)) return rc;
   if (rows == 0) return RWKV7MI_OK;
-  const int64_t per_prob = rwkv7mi_mm8t_gemm_prefill_ws_bytes(1, I, O);
+  const int64_t per_prob = mh_weight_bytes(1, I, O);
   MhBatch b{};
   MhDeqBatch d{};
   for (int i = 0; i < nprob; ++i) {
@@ -473,16 +631,19 @@ extern "C" int rwkv7mi_mm8t_gemm_prefill_ws(int nprob, const void* const* x, con
   d.O = (int)O;
   d.SB = (int)((I + 63) / 64);
   d.KB = (int)((I + 127) / 128);
+  d.vec = 1;
+  for (int i = 0; i < nprob; ++i)
+    if ((reinterpret_cast<uintptr_t>(my[i]) | reinterpret_cast<uintptr_t>(ry[i])) & 15) d.vec = 0;
   const int64_t recs = (2 * ((O + 31) / 32)) * (int64_t)d.SB * 64;
   const dim3 dgrid((unsigned)((recs + 255) / 256), (unsigned)nprob);
   if (act_dtype == RWKV7MI_BF16) {
     hipLaunchKernelGGL(mm8h_dequant_kernel<__hip_bfloat16>, dgrid, dim3(256), 0, as_stream(stream), d);
     if (int rc = check_launch("mm8h_dequant_kernel")) return rc;
-    return mh_gemm_launch<__hip_bfloat16>(b, nprob, rows, I, O, stream, w);
+    return mh_gemm_launch<__hip_bfloat16>(b, nprob, rows, I, O, ws, ws_bytes, stream, w);
   }
   hipLaunchKernelGGL(mm8h_dequant_kernel<__half>, dgrid, dim3(256), 0, as_stream(stream), d);
   if (int rc = check_launch("mm8h_dequant_kernel")) return rc;
-  return mh_gemm_launch<__half>(b, nprob, rows, I, O, stream, w);
+  return mh_gemm_launch<__half>(b, nprob, rows, I, O, ws, ws_bytes, stream, w);
 }
 
 extern "C" int rwkv7mi_dense_gemm_prefill_ws(int nprob, const void* const* x, const void* const* W,
@@ -495,7 +656,7 @@ extern "C" int rwkv7mi_dense_gemm_prefill_ws(int nprob, const void* const* x, co
     return fail(RWKV7MI_EINVAL, w + ": fp16 or bf16 activations and weights");
   if (int rc = mh_check(w, nprob, rows, I, O, ws, ws_bytes)) return rc;
   if (rows == 0) return RWKV7MI_OK;
-  const int64_t per_prob = rwkv7mi_mm8t_gemm_prefill_ws_bytes(1, I, O);
+  const int64_t per_prob = mh_weight_bytes(1, I, O);
   MhBatch b{};
   MhRelBatch r{};
   for (int i = 0; i < nprob; ++i) {
@@ -515,9 +676,9 @@ extern "C" int rwkv7mi_dense_gemm_prefill_ws(int nprob, const void* const* x, co
   if (act_dtype == RWKV7MI_BF16) {
     hipLaunchKernelGGL(mm8h_relayout_kernel<__hip_bfloat16>, rgrid, dim3(256), 0, as_stream(stream), r);
     if (int rc = check_launch("mm8h_relayout_kernel")) return rc;
-    return mh_gemm_launch<__hip_bfloat16>(b, nprob, rows, I, O, stream, w);
+    return mh_gemm_launch<__hip_bfloat16>(b, nprob, rows, I, O, ws, ws_bytes, stream, w);
   }
   hipLaunchKernelGGL(mm8h_relayout_kernel<__half>, rgrid, dim3(256), 0, as_stream(stream), r);
   if (int rc = check_launch("mm8h_relayout_kernel")) return rc;
-  return mh_gemm_launch<__half>(b, nprob, rows, I, O, stream, w);
+  return mh_gemm_launch<__half>(b, nprob, rows, I, O, ws, ws_bytes, stream, w);
 }

@@ -1031,9 +1031,11 @@ class NativeRWKV7ForCausalLM(_PreTrainedModel, _GenerationMixin):
             pneed = 0
             for L in self.layers:
                 if isinstance(L.r_proj, QuantLinear):
-                    pneed = max(pneed, mm8_prefill_workspace_bytes(3, L.r_proj.in_features, L.r_proj.out_features))
+                    pneed = max(pneed, mm8_prefill_workspace_bytes(3, L.r_proj.in_features, L.r_proj.out_features, rows))
             for lin in self._linears():
-                if isinstance(lin, QuantLinear) or (isinstance(lin, DenseLinear) and lin.weight.dtype != torch.float32):
+                if isinstance(lin, QuantLinear):
+                    pneed = max(pneed, mm8_prefill_workspace_bytes(1, lin.in_features, lin.out_features, rows))
+                elif isinstance(lin, DenseLinear) and lin.weight.dtype != torch.float32:
                     pneed = max(pneed, mm8_prefill_workspace_bytes(1, lin.in_features, lin.out_features))
             if pneed:
                 _ws.reserve(self.device, pneed, slot="mm8p")

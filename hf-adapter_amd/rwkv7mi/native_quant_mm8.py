@@ -131,9 +131,12 @@ def mm8_workspace_bytes(rows: int, n: int, m: int) -> int:
     return int(_lib.load().rwkv7mi_mm8_workspace_bytes(int(rows), int(n), int(m)))
 
 
-def mm8_prefill_workspace_bytes(nprob: int, n: int, m: int) -> int:
+def mm8_prefill_workspace_bytes(nprob: int, n: int, m: int, rows: int | None = None) -> int:
     """Bytes of the ``"mm8p"`` slot a prefill GEMM of ``nprob`` ``[n -> m]``
-    problems needs: their fp16 dequantised weights in MFMA operand order."""
+    problems needs: their fp16 dequantised weights in MFMA operand order, and
+    with ``rows`` also the partials of the K splits that call runs with."""
+    if rows is not None:
+        return int(_lib.load().rwkv7mi_mm8t_gemm_prefill_split_ws_bytes(int(nprob), int(rows), int(n), int(m)))
     return int(_lib.load().rwkv7mi_mm8t_gemm_prefill_ws_bytes(int(nprob), int(n), int(m)))
 
 
@@ -401,8 +404,10 @@ def mm8_gemm_prefill_multi_into(xs, mods, outs, *, residuals=None, epilogues=Non
             else:
                 mm8_matmul_multi_into(xc, mods, oc, residuals=rc, epilogues=epilogues)
             continue
-        need = mm8_prefill_workspace_bytes(k, n, m)
-        ws = _ws.reserve(xs[0].device, need, "mm8p")
+        need = mm8_prefill_workspace_bytes(k, n, m, r1 - r0)
+        # (a graph captured over a slot without the partials runs unsplit)
+        ws = _ws.reserve(xs[0].device, need, "mm8p", floor=mm8_prefill_workspace_bytes(k, n, m))
+        need = min(need, int(ws.numel()))
         _lib.call(
             "rwkv7mi_mm8t_gemm_prefill_ws", k, arr(xc), arr([md.w_blk for md in mods]), arr([md.mx for md in mods]),
             arr([md.rx for md in mods]), arr([md.my for md in mods]), arr([md.ry for md in mods]),

@@ -423,6 +423,10 @@ int rwkv7mi_mm8t_gemm_prefill(int nprob, const void* const* x,
  * in_features I, out_features O: nprob * ceil(O / 16) * ceil(I / 64) * 2048
  * (each problem's fp16 dequantised weight); 0 for a bad shape. */
 int64_t rwkv7mi_mm8t_gemm_prefill_ws_bytes(int nprob, int64_t I, int64_t O);
+/* The same plus the fp32 partials of the K splits that `rows` rows run with
+ * when their 256 x 256 tiles do not fill the chip.  A call with a workspace of
+ * only rwkv7mi_mm8t_gemm_prefill_ws_bytes runs unsplit. */
+int64_t rwkv7mi_mm8t_gemm_prefill_split_ws_bytes(int nprob, int64_t rows, int64_t I, int64_t O);
 
 /* The prefill GEMM as the reference computes it, the faster form on gfx950:
  * the dequantised weight W_hat = (w + 0.5) ry rx + my + mx, rounded once to

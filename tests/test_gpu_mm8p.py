@@ -235,6 +235,44 @@ def test_dense_prefill_gemm_matches_fp64(IO, rows, epi, dt):
     assert torch.equal(y2, y)
 
 
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("I,O,rows,epi", [(2048, 264, 257, 0), (2112, 520, 300, 1), (4096, 40, 700, 2),
+                                          (8192, 256, 1030, 2)])
+def test_mm8p_k_splits(oracle, I, O, rows, epi, dt):
+    """Few 256 x 256 tiles: K cut into ranges whose fp32 partials a second
+    launch adds (uneven ranges: 33 steps; columns that end inside a wave and
+    inside an 8-column store), against the oracle and against the unsplit form
+    that a workspace of only the weights gives."""
+    import ctypes
+
+    from rwkv7mi import _lib
+    from rwkv7mi.native_quant_mm8 import mm8_gemm_prefill_multi_into, mm8_prefill_workspace_bytes
+
+    tdt = torch.float16 if dt == "f16" else torch.bfloat16
+    rng = np.random.default_rng(I + O + rows)
+    mod = _packed(rng, I, O, tdt, bias=True)
+    x = _cuda(rng.standard_normal((rows, I)), tdt)
+    res = _cuda(rng.standard_normal((rows, O)), tdt) if epi == 2 else None
+    y, one = (torch.full((rows, O), float("nan"), device="cuda", dtype=tdt) for _ in range(2))
+    need = mm8_prefill_workspace_bytes(1, I, O)
+    assert mm8_prefill_workspace_bytes(1, I, O, rows) > need, "the shape must split"
+    mm8_gemm_prefill_multi_into([x], [mod], [y], residuals=[res], epilogues=[epi])
+    ws = torch.empty(need, device="cuda", dtype=torch.uint8)
+    arr = _lib.ptr_array
+    _lib.call("rwkv7mi_mm8t_gemm_prefill_ws", 1, arr([x]), arr([mod.w_blk]), arr([mod.mx]), arr([mod.rx]),
+              arr([mod.my]), arr([mod.ry]), arr([mod.bias]), arr([res]), arr([one]), (ctypes.c_int * 1)(epi),
+              rows, I, O, _lib.dtype_code(x), _lib.dtype_code(x), _lib.ptr(ws), need, _lib.stream_of(x))
+    torch.cuda.synchronize()
+    f64 = lambda t: _np(t.float()).astype(np.float64)
+    # fp32 sums in another order, each rounded once: one step of the result
+    step = 2.0 ** -10 if dt == "f16" else 2.0 ** -7
+    assert np.all(np.abs(f64(y) - f64(one)) <= step * np.abs(f64(one)) + 1e-4)
+    ref = _ref(oracle, x, mod) if dt == "f16" else None
+    if ref is not None:
+        ref = np.maximum(ref, 0.0) ** 2 if epi == 1 else ref + f64(res) if epi == 2 else ref
+        assert _rel_err(f64(y), ref) <= TOL
+
+
 def test_mm8p_rejects():
     from rwkv7mi import _lib
 
