@@ -23,7 +23,7 @@
 //   sum_i W x = s sum (q - 8) x + (8 s + b) sum_i x,
 // and the group sums of x come from one more MFMA per step against a B
 // operand of ones, which lands them in the accumulator layout directly.
-#include "mm8t_common.h"
+#include "w4_common.h"
 
 namespace rwkv7mi {
 
@@ -53,25 +53,6 @@ __device__ __forceinline__ void w4_load_a(const TA* __restrict__ xrow, bool ok, 
     hi[p] = h;
     lo[p] = (_Float16)(f - (float)h);
   }
-}
-
-__device__ __forceinline__ f16x8 w4_nibbles_to_f16(uint32_t d) {
-  // d = 8 nibbles n0..n7 (n_{2j} low nibble of byte j); out = [n0,n4,n1,n5,n2,n6,n3,n7] - 8.
-  // fp16 pairs with exponent 0x64 hold 1024 + n (nibble in bits 0-3) or
-  // 1024 + 16 n (bits 4-7): one packed add of -1032 or one packed fma by
-  // 1/16 with -72 gives n - 8 exactly.  9 VALU ops per dword.
-  const uint32_t d8 = d >> 8;
-  const f16x2 a = __builtin_bit_cast(f16x2, and_or(d, 0x000F000Fu, 0x64006400u));
-  const f16x2 b = __builtin_bit_cast(f16x2, and_or(d, 0x00F000F0u, 0x64006400u));
-  const f16x2 c = __builtin_bit_cast(f16x2, and_or(d8, 0x000F000Fu, 0x64006400u));
-  const f16x2 e = __builtin_bit_cast(f16x2, and_or(d8, 0x00F000F0u, 0x64006400u));
-  const f16x2 off = {(_Float16)-1032.0f, (_Float16)-1032.0f};
-  const f16x2 sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f};
-  const f16x2 off16 = {(_Float16)-72.0f, (_Float16)-72.0f};
-  const f16x2 p0 = a + off, p2 = c + off;
-  const f16x2 p1 = __builtin_elementwise_fma(b, sixteenth, off16);
-  const f16x2 p3 = __builtin_elementwise_fma(e, sixteenth, off16);
-  return (f16x8){p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
 }
 
 template <int MT, typename TA, typename TS, bool AFF>
@@ -616,9 +597,26 @@ static int w4t_go(int nw, int csw, dim3 grid, size_t lds, void* stream, const W4
   return w4t_launch<TA, TS, 8, 8, AFF>(grid, lds, stream, a);
 }
 
+// The many-row product (w4m.hip) from 17 rows on, and below that where the
+// rows' x does not fit the GEMV's LDS at once (it would re-stage x for every
+// column group).  Measured, GEMV -> many-row kernel: 17 rows 4096 x 4096 15 ->
+// 14 us (w4g_kernel there); staged once: 16 rows 4096 x 65536 54 -> 57, 9 rows
+// 4096 x 4096 8 -> 14; in chunks: bf16 16 rows 4096 x 65536 affine 246 -> 67,
+// 9 rows 16384 x 4096 48 -> 25, fp16 12 rows 29 -> 22.
+static bool w4_many(int64_t rows, int64_t O, int64_t I, int64_t group, int act_dtype, bool aff) {
+  if (!w4m_supported(rows, O, I, group, act_dtype)) return false;
+  if (rows > 16) return true;
+  // (7 rows bf16 16384 x 4096 in chunks: 27 us, 16 rows bf16 4096 x 4096: 15,
+  // about the many-row kernel and its reduce there)
+  if (rows <= 8 || O * I < ((int64_t)1 << 25)) return false;
+  int nw = 0, csw = 0;
+  return !w4t_plan(rows, I, O, act_dtype != RWKV7MI_F16, aff, &nw, &csw) || 256 * nw * csw < I;
+}
+
 static int w4_matmul(const char* who, const void* x, const uint8_t* packed, const void* scales, const void* gbias,
                      const void* bias, const void* residual, void* y, int64_t rows, int64_t O, int64_t I,
-                     int64_t group, int epilogue, int act_dtype, int scale_dtype, void* stream) {
+                     int64_t group, int epilogue, int act_dtype, int scale_dtype, void* ws, int64_t ws_bytes,
+                     void* stream) {
   const std::string w(who);
   if (group != 128 && group != 256) return fail(RWKV7MI_EINVAL, w + ": group must be 128 or 256");
   if (rows < 0 || O <= 0 || I <= 0 || I % group) return fail(RWKV7MI_EINVAL, w + ": bad shape");
@@ -631,7 +629,8 @@ static int w4_matmul(const char* who, const void* x, const uint8_t* packed, cons
     return fail(RWKV7MI_EINVAL, w + ": x and packed must be 16-byte aligned");
   if (!valid_dtype(act_dtype) || !valid_dtype(scale_dtype)) return fail(RWKV7MI_EINVAL, w + ": bad dtype");
   const size_t esz = act_dtype == RWKV7MI_F32 ? 4 : 2;
-  if (rows <= 16 && I <= (1 << 22) && (int64_t)rows * I * (int64_t)esz <= INT32_MAX &&
+  const bool many = w4_many(rows, O, I, group, act_dtype, gbias != nullptr);
+  if (!many && rows <= 16 && I <= (1 << 22) && (int64_t)rows * I * (int64_t)esz <= INT32_MAX &&
       16 * (I / 2) <= INT32_MAX) {
     int nw = 4, csw = 4;
     const bool hl = act_dtype != RWKV7MI_F16, aff = gbias != nullptr;
@@ -659,8 +658,13 @@ static int w4_matmul(const char* who, const void* x, const uint8_t* packed, cons
       });
     }
   }
-  for (int64_t r0 = 0; r0 < rows; r0 += 64) {
-    const int64_t nr = rows - r0 > 64 ? 64 : rows - r0;
+  if (many)
+    return w4m_run(x, packed, scales, gbias, bias, residual, y, rows, O, I, group, epilogue, act_dtype, scale_dtype,
+                   ws, ws_bytes, stream);
+  // fp32 (and 16-bit inputs too wide for the kernels above, 16 rows a launch)
+  const int64_t step = act_dtype == RWKV7MI_F32 ? 64 : 16;
+  for (int64_t r0 = 0; r0 < rows; r0 += step) {
+    const int64_t nr = rows - r0 > step ? step : rows - r0;
     const int mt = nr <= 16 ? 1 : nr <= 32 ? 2 : 4;
     const char* xr = reinterpret_cast<const char*>(x) + r0 * I * esz;
     char* yr = reinterpret_cast<char*>(y) + r0 * O * esz;
@@ -674,14 +678,18 @@ static int w4_matmul(const char* who, const void* x, const uint8_t* packed, cons
   hipLaunchKernelGGL((w4g_kernel<MT_, TA, TS, AFF_>), grid, dim3(256), 0, as_stream(stream), (const TA*)xr, \
                      packed, (const TS*)scales, (const TS*)gbias, (const TS*)bias, (const TA*)rr, (TA*)yr,   \
                      (int)nr, (int)O, (int)I, (int)group, epilogue)
-        if (gbias) {
-          if (mt == 1) W4_LAUNCH(1, true);
-          else if (mt == 2) W4_LAUNCH(2, true);
-          else W4_LAUNCH(4, true);
-        } else {
-          if (mt == 1) W4_LAUNCH(1, false);
-          else if (mt == 2) W4_LAUNCH(2, false);
-          else W4_LAUNCH(4, false);
+        if constexpr (std::is_same<TA, float>::value) {
+          if (mt == 2) {
+            if (gbias) W4_LAUNCH(2, true);
+            else W4_LAUNCH(2, false);
+          } else if (mt == 4) {
+            if (gbias) W4_LAUNCH(4, true);
+            else W4_LAUNCH(4, false);
+          }
+        }
+        if (mt == 1) {
+          if (gbias) W4_LAUNCH(1, true);
+          else W4_LAUNCH(1, false);
         }
 #undef W4_LAUNCH
         return check_launch("w4g_kernel");
@@ -696,7 +704,7 @@ extern "C" int rwkv7mi_w4g_matmul(const void* x, const uint8_t* packed, const vo
                                   const void* residual, void* y, int64_t rows, int64_t O, int64_t I,
                                   int64_t group, int epilogue, int act_dtype, int scale_dtype, void* stream) {
   return w4_matmul("w4g_matmul", x, packed, scales, nullptr, bias, residual, y, rows, O, I, group, epilogue,
-                   act_dtype, scale_dtype, stream);
+                   act_dtype, scale_dtype, nullptr, 0, stream);
 }
 
 extern "C" int rwkv7mi_w4a_matmul(const void* x, const uint8_t* packed, const void* scales, const void* biases,
@@ -705,5 +713,19 @@ extern "C" int rwkv7mi_w4a_matmul(const void* x, const uint8_t* packed, const vo
                                   void* stream) {
   if (!biases) return fail(RWKV7MI_EINVAL, "w4a_matmul: null group biases");
   return w4_matmul("w4a_matmul", x, packed, scales, biases, bias, residual, y, rows, O, I, group, epilogue,
-                   act_dtype, scale_dtype, stream);
+                   act_dtype, scale_dtype, nullptr, 0, stream);
+}
+
+extern "C" int64_t rwkv7mi_w4_workspace_bytes(int64_t rows, int64_t O, int64_t I, int64_t group, int affine,
+                                              int act_dtype) {
+  if (rows <= 0 || O <= 0 || I <= 0 || (group != 128 && group != 256) || I % group) return 0;
+  return w4_many(rows, O, I, group, act_dtype, affine != 0) ? w4m_workspace_bytes(rows, O, I, group) : 0;
+}
+
+extern "C" int rwkv7mi_w4_matmul_ws(const void* x, const uint8_t* packed, const void* scales, const void* biases,
+                                    const void* bias, const void* residual, void* y, int64_t rows, int64_t O,
+                                    int64_t I, int64_t group, int epilogue, int act_dtype, int scale_dtype,
+                                    void* ws, int64_t ws_bytes, void* stream) {
+  return w4_matmul("w4_matmul_ws", x, packed, scales, biases, bias, residual, y, rows, O, I, group, epilogue,
+                   act_dtype, scale_dtype, ws, ws_bytes, stream);
 }

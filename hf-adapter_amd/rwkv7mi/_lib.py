@@ -115,6 +115,8 @@ SIGNATURES = {
     "rwkv7mi_w4g_pack": (_i32, [_c_p, _i64, _i64, _i64, _i32, _c_p, _c_p, _c_p]),
     "rwkv7mi_w4a_pack": (_i32, [_c_p, _i64, _i64, _i64, _i32, _c_p, _c_p, _c_p, _c_p]),
     "rwkv7mi_w4a_matmul": (_i32, [_c_p] * 7 + [_i64, _i64, _i64, _i64, _i32, _i32, _i32, _c_p]),
+    "rwkv7mi_w4_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _i32, _i32]),
+    "rwkv7mi_w4_matmul_ws": (_i32, [_c_p] * 7 + [_i64, _i64, _i64, _i64, _i32, _i32, _i32, _c_p, _i64, _c_p]),
     "rwkv7mi_w4g_matmul": (
         _i32,
         [_c_p] * 6 + [_i64, _i64, _i64, _i64, _i32, _i32, _i32, _c_p],

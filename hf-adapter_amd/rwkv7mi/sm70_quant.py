@@ -11,6 +11,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
+from . import workspace as _ws
 
 
 def quantize_w4_groupwise(weight: torch.Tensor, group_size: int = 128):
@@ -35,6 +36,18 @@ def quantize_w4_groupwise(weight: torch.Tensor, group_size: int = 128):
     return packed, scales, in_features
 
 
+def _w4_call(x2, q, scales, biases, bias, residual, out2, rows, out_features, in_features, group_size, epilogue):
+    """The W4 product (``biases`` None: symmetric) over the ``"w4"`` slot's
+    workspace (many rows; a graph captured without one runs unsplit)."""
+    dt = _lib.dtype_code(x2)
+    need = int(_lib.load().rwkv7mi_w4_workspace_bytes(rows, out_features, in_features, group_size,
+                                                      int(biases is not None), dt))
+    ws = _ws.reserve(x2.device, need, slot="w4", floor=0) if need else None
+    _lib.call("rwkv7mi_w4_matmul_ws", _lib.ptr(x2), _lib.ptr(q), _lib.ptr(scales), _lib.ptr(biases), _lib.ptr(bias),
+              _lib.ptr(residual), _lib.ptr(out2), rows, out_features, in_features, group_size, int(epilogue), dt,
+              _lib.dtype_code(scales), _lib.ptr(ws), 0 if ws is None else int(ws.numel()), _lib.stream_of(x2))
+
+
 def w4_groupwise_linear_into(x2, q, scales, out2, *, group_size=128, bias=None, residual=None,
                              epilogue=_lib.EPI_NONE):
     rows, in_features = (int(s) for s in x2.shape)
@@ -48,11 +61,7 @@ def w4_groupwise_linear_into(x2, q, scales, out2, *, group_size=128, bias=None, 
         residual = residual.reshape(rows, out_features)
         if not residual.is_contiguous() or residual.dtype != x2.dtype:
             raise ValueError("w4: residual must be contiguous with x's dtype")
-    _lib.call(
-        "rwkv7mi_w4g_matmul", _lib.ptr(x2), _lib.ptr(q), _lib.ptr(scales), _lib.ptr(bias),
-        _lib.ptr(residual), _lib.ptr(out2), rows, out_features, in_features, int(group_size),
-        int(epilogue), _lib.dtype_code(x2), _lib.dtype_code(scales), _lib.stream_of(x2),
-    )
+    _w4_call(x2, q, scales, None, bias, residual, out2, rows, out_features, in_features, int(group_size), epilogue)
     return out2
 
 
@@ -120,10 +129,8 @@ def w4_affine_groupwise_linear(x, q, scales, biases, out_features, in_features, 
     out2 = out.reshape(rows, int(out_features)) if out is not None else torch.empty(
         (rows, int(out_features)), device=x.device, dtype=x.dtype)
     _lib.require_gpu(x2, q, scales, biases, out2, name="w4_affine_groupwise_linear")
-    _lib.call("rwkv7mi_w4a_matmul", _lib.ptr(x2), _lib.ptr(q), _lib.ptr(scales.contiguous()),
-              _lib.ptr(biases.contiguous()), _lib.ptr(bias), None, _lib.ptr(out2), rows, int(out_features),
-              int(in_features), group_size, int(_lib.EPI_NONE), _lib.dtype_code(x2), _lib.dtype_code(scales),
-              _lib.stream_of(x2))
+    _w4_call(x2, q, scales.contiguous(), biases.contiguous(), bias, None, out2, rows, int(out_features),
+             int(in_features), group_size, _lib.EPI_NONE)
     if out is not None:
         return out
     return out2.reshape(*x.shape[:-1], int(out_features))

@@ -7,7 +7,8 @@ on one stream.  Slot ``"mm8t"`` holds the blocked GEMV's split-K partials
 (written before they are read).  Slot ``"mm8g"`` holds the many-row MM8 GEMM's x', row sums and
 split partials (each call writes them before reading).  Slot ``"lora"`` holds
 the LoRA kernels' fp32 partials.  Slot ``"mm8p"`` holds the prefill GEMM's
-fp16 dequantised weights (each call writes them before reading).  Slots never share memory, so one kernel
+fp16 dequantised weights and split partials, slot ``"w4"`` the many-row W4
+product's split partials (each call writes them before reading).  Slots never share memory, so one kernel
 family cannot disturb another's counters.  Calls that run concurrently on
 different streams of the same device must not share a slot (the decode step
 issues all of them on one stream).
@@ -44,13 +45,14 @@ def reserve(device: torch.device, nbytes: int, slot: str = "mm8", *, floor: int 
     """Return the device's buffer for ``slot``, growing it (zero-filled) to ``nbytes``.
 
     ``floor``: the least the call can run with.  Under graph capture a buffer
-    of at least ``floor`` bytes is returned as it is instead of raising."""
+    of at least ``floor`` bytes (with 0 also no buffer: None) is returned as it
+    is instead of raising."""
     key = _key(device, slot)
     with _lock:
         buf = _buffers.get(key)
         if buf is None or buf.numel() < nbytes:
             if torch.cuda.is_current_stream_capturing():
-                if floor is not None and buf is not None and buf.numel() >= floor:
+                if floor is not None and (0 if buf is None else buf.numel()) >= floor:
                     return buf
                 raise RuntimeError(
                     f"rwkv7mi workspace '{slot}' must be reserved before graph capture "

@@ -703,6 +703,17 @@ int rwkv7mi_w4a_matmul(const void* x, const uint8_t* packed,
                        int64_t rows, int64_t O, int64_t I, int64_t group,
                        int epilogue, int act_dtype, int scale_dtype,
                        void* stream);
+/* Both with a workspace (biases NULL: the symmetric form).  Many fp16 / bf16
+ * rows whose tiles do not fill the chip split K over workgroups through it;
+ * rwkv7mi_w4_workspace_bytes says how much that takes (0: no split), and with
+ * less, or with NULL, the call runs unsplit. */
+int64_t rwkv7mi_w4_workspace_bytes(int64_t rows, int64_t O, int64_t I, int64_t group, int affine, int act_dtype);
+int rwkv7mi_w4_matmul_ws(const void* x, const uint8_t* packed,
+                         const void* scales, const void* biases,
+                         const void* bias, const void* residual, void* y,
+                         int64_t rows, int64_t O, int64_t I, int64_t group,
+                         int epilogue, int act_dtype, int scale_dtype,
+                         void* ws, int64_t ws_bytes, void* stream);
 
 /* ------------------------------------------------ LayerNorm + token shift */
 

@@ -225,6 +225,54 @@ def test_w4_stream_gemv_edges(oracle, case):
     assert err <= tol, (case, err)
 
 
+@pytest.mark.parametrize("case", [
+    # (O, I, group, rows, act dtype, affine, epilogue)
+    (200, 384, 128, 17, torch.float16, False, 0),     # three K blocks, one ragged column tile
+    (260, 256, 256, 33, torch.bfloat16, False, 1),    # two blocks of one group; 260 ends inside an 8-column store
+    (1040, 2048, 256, 65, torch.float16, False, 2),   # 65 rows: a second row tile of one row; K splits
+    (520, 4096, 128, 100, torch.bfloat16, True, 0),
+    (264, 16384, 128, 32, torch.float16, True, 0),
+    (4100, 1152, 128, 131, torch.float16, False, 2),  # 9 blocks: uneven K ranges
+])
+def test_w4_many_rows(oracle, case):
+    """More than 16 rows: row, column and K edges of the 32- and 64-row tiles,
+    both groups, the epilogues, the K splits and (through the entry without a
+    workspace) the unsplit form."""
+    from rwkv7mi import _lib
+    from rwkv7mi import quantize_w4_groupwise
+    from rwkv7mi.sm70_quant import (quantize_w4_affine_groupwise, w4_affine_groupwise_linear,
+                                    w4_groupwise_linear_into)
+
+    O, I, group, rows, act, aff, epi = case
+    rng = np.random.default_rng(O + I + rows + group)
+    W = _cuda(rng.standard_normal((O, I)) * 0.02, torch.float16)
+    x = _cuda(rng.standard_normal((rows, I)), act)
+    f64 = lambda t: _np(t.float()).astype(np.float64)
+    one = torch.full((rows, O), float("nan"), device="cuda", dtype=act)
+    if aff:
+        q, s, b, _ = quantize_w4_affine_groupwise(W, group_size=group)
+        y = w4_affine_groupwise_linear(x, q, s, b, O, I, group_size=group)
+        _lib.call("rwkv7mi_w4a_matmul", _lib.ptr(x), _lib.ptr(q), _lib.ptr(s), _lib.ptr(b), None, None, _lib.ptr(one),
+                  rows, O, I, group, 0, _lib.dtype_code(x), _lib.dtype_code(s), _lib.stream_of(x))
+        ref = oracle.w4a_linear(f64(x), _np(q), _np(s), _np(b), group)
+    else:
+        q, s, _ = quantize_w4_groupwise(W, group_size=group)
+        bias = _cuda(rng.standard_normal(O) * 0.1, torch.float16)
+        res = _cuda(rng.standard_normal((rows, O)), act) if epi == 2 else None
+        y = res.clone() if epi == 2 else torch.empty((rows, O), device="cuda", dtype=act)
+        w4_groupwise_linear_into(x, q, s, y, group_size=group, bias=bias, residual=y if epi == 2 else None,
+                                 epilogue=epi)
+        _lib.call("rwkv7mi_w4g_matmul", _lib.ptr(x), _lib.ptr(q), _lib.ptr(s), _lib.ptr(bias), _lib.ptr(res),
+                  _lib.ptr(one), rows, O, I, group, epi, _lib.dtype_code(x), _lib.dtype_code(s), _lib.stream_of(x))
+        ref = oracle.w4g_linear(f64(x), _np(q), _np(s), group) + f64(bias)
+        ref = np.maximum(ref, 0.0) ** 2 if epi == 1 else ref + f64(res) if epi == 2 else ref
+    torch.cuda.synchronize()
+    # exact products and fp32 sums: the output's rounding
+    tol = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[act]
+    for got in (y, one):
+        assert np.all(np.abs(f64(got) - ref) <= tol * np.abs(ref) + 2e-5 * np.abs(ref).max()), case
+
+
 @pytest.mark.parametrize("rows", [1, 6])
 def test_w4_stream_gemv_epilogues(oracle, rows):
     """Bias, residual (in place: out aliases the residual) and relu^2 epilogues
