@@ -11,24 +11,13 @@
 // 16-feature tile; its 4 waves take interleaved 32-wide k-steps and are
 // reduced through LDS.  fp16 operands are used as-is; fp32 / bf16 operands are
 // split into fp16 hi + lo (three MFMAs) so accuracy stays fp32-class.
-// One to four rows take a GEMV form instead (dense_gemv_kernel below).
-#include "common.h"
+// One to four rows take a GEMV form instead (dense_gemv_kernel below), more
+// fp16 / bf16 rows the tile kernel of dense_tile.hip; this form is fp32's.
+#include <algorithm>
+
+#include "dense_common.h"
 
 namespace rwkv7mi {
-
-enum { ACT_NONE = 0, ACT_TANH = 1, ACT_SIGMOID = 2, ACT_RELU2 = 3 };
-
-struct DenseProb {
-  const void* x;
-  const void* W;
-  const void* bias;
-  void* y;
-  int N, K, act, tile0;
-};
-struct DenseBatch {
-  DenseProb p[4];
-  int nprob;
-};
 
 template <typename T>
 __device__ __forceinline__ void load8_split(const T* src, bool ok, f16x8& hi, f16x8& lo) {
@@ -49,16 +38,6 @@ __device__ __forceinline__ void load8_split(const T* src, bool ok, f16x8& hi, f1
       lo[e] = (_Float16)(f - (float)h);
     }
   }
-}
-
-__device__ __forceinline__ float apply_act(float v, int act) {
-  if (act == ACT_TANH) return tanhf(v);
-  if (act == ACT_SIGMOID) return 1.0f / (1.0f + expf(-v));
-  if (act == ACT_RELU2) {
-    v = fmaxf(v, 0.f);
-    return v * v;
-  }
-  return v;
 }
 
 template <int MT, typename TA>
@@ -118,7 +97,9 @@ __global__ __launch_bounds__(256) void dense_kernel(DenseBatch batch, int rows) 
     if (o >= P.N) continue;
     float v = s_red[r][nn];
     if (bias) v += to_f32(bias[o]);
-    y[(int64_t)r * P.N + o] = from_f32<TA>(apply_act(v, P.act));
+    v = apply_act(v, P.act);
+    if (P.residual) v += to_f32(reinterpret_cast<const TA*>(P.residual)[(int64_t)r * P.N + o]);
+    y[(int64_t)r * P.N + o] = from_f32<TA>(v);
   }
 }
 
@@ -211,10 +192,13 @@ __global__ __launch_bounds__(256) void dense_gemv_kernel(DenseBatch batch, int r
   const TA* bias = reinterpret_cast<const TA*>(P.bias);
   const float b = bias ? to_f32(bias[n]) : 0.f;
   TA* y = reinterpret_cast<TA*>(P.y);
+  // lane r finishes row r; its residual is on its way during the sums
+  const TA* res = reinterpret_cast<const TA*>(P.residual);
+  const float rv = res && lane < R && lane < rows ? to_f32(res[(int64_t)lane * P.N + n]) : 0.f;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const float v = wave_sum(acc[r]);
-    if (lane == r && r < rows) y[(int64_t)r * P.N + n] = from_f32<TA>(apply_act(v + b, P.act));
+    if (lane == r && r < rows) y[(int64_t)r * P.N + n] = from_f32<TA>(apply_act(v + b, P.act) + rv);
   }
 }
 
@@ -227,6 +211,14 @@ using namespace rwkv7mi;
 extern "C" int rwkv7mi_dense_multi(const void* const* xs, const void* const* Ws, const void* const* biases,
                                    void* const* ys, const int64_t* Ns, const int64_t* Ks, const int* acts,
                                    int64_t nprob, int64_t rows, int act_dtype, void* stream) {
+  return rwkv7mi_dense_multi_residual(xs, Ws, biases, nullptr, ys, Ns, Ks, acts, nprob, rows, act_dtype, stream);
+}
+
+extern "C" int rwkv7mi_dense_multi_residual(const void* const* xs, const void* const* Ws,
+                                            const void* const* biases, const void* const* residuals,
+                                            void* const* ys, const int64_t* Ns, const int64_t* Ks,
+                                            const int* acts, int64_t nprob, int64_t rows, int act_dtype,
+                                            void* stream) {
   if (nprob < 1 || nprob > 4) return fail(RWKV7MI_EINVAL, "dense_multi: 1..4 problems");
   if (rows < 0) return fail(RWKV7MI_EINVAL, "dense_multi: bad rows");
   if (rows == 0) return RWKV7MI_OK;
@@ -239,12 +231,22 @@ extern "C" int rwkv7mi_dense_multi(const void* const* xs, const void* const* Ws,
     if (acts[i] < 0 || acts[i] > 3) return fail(RWKV7MI_EINVAL, "dense_multi: bad activation");
     if ((reinterpret_cast<uintptr_t>(xs[i]) | reinterpret_cast<uintptr_t>(Ws[i])) & 15)
       return fail(RWKV7MI_EINVAL, "dense_multi: x and W must be 16-byte aligned");
-    batch.p[i] = DenseProb{xs[i], Ws[i], biases[i], ys[i], (int)Ns[i], (int)Ks[i], acts[i], tiles};
+    batch.p[i] = DenseProb{xs[i], Ws[i], biases[i], residuals ? residuals[i] : nullptr, ys[i], (int)Ns[i], (int)Ks[i],
+                           acts[i], tiles};
     tiles += (int)((Ns[i] + 15) / 16);
   }
   batch.nprob = (int)nprob;
   const size_t esz = act_dtype == RWKV7MI_F32 ? 4 : 2;
-  if (rows <= 4) {  // the GEMV form: tiles of four features, one wave each
+  // Two to four 16-bit rows with many short outputs: the GEMV's per-feature
+  // reduction outweighs its loads there, and the tile kernel is faster (GEMV ->
+  // tile, us: 4 rows 768 -> 65536 80 -> 26, 768 -> 3072 5.2 -> 3.2, 2048 -> 8192
+  // 10.8 -> 9.3; 2 rows 768 -> 65536 39 -> 26, but 2048 -> 65536 51 -> 61; the
+  // other way 4 rows 2048 -> 2048 3.8 -> 5.0, 3072 -> 768 3.9 -> 5.8).
+  int64_t nsum = 0, kmax = 0;
+  for (int i = 0; i < nprob; ++i) nsum += Ns[i], kmax = std::max(kmax, Ks[i]);
+  const bool wide = nsum >= 2 * kmax && (rows >= 3 || (rows == 2 && kmax <= 1024)) &&
+                    dense_tile_supported(batch, rows, act_dtype);
+  if (rows <= 4 && !wide) {  // the GEMV form: tiles of four features, one wave each
     DenseBatch gb = batch;
     int gt = 0;
     for (int i = 0; i < nprob; ++i) {
@@ -265,19 +267,25 @@ extern "C" int rwkv7mi_dense_multi(const void* const* xs, const void* const* Ws,
       return check_launch("dense_gemv_kernel");
     });
   }
-  for (int64_t r0 = 0; r0 < rows; r0 += 64) {
-    const int64_t nr = rows - r0 > 64 ? 64 : rows - r0;
+  if (dense_tile_supported(batch, rows, act_dtype)) return dense_tile_run(batch, rows, act_dtype, 1, nullptr, 0, stream);
+  // fp32 (and 16-bit inputs too wide for the tile kernel, 16 rows a launch)
+  const int64_t step = act_dtype == RWKV7MI_F32 ? 64 : 16;
+  for (int64_t r0 = 0; r0 < rows; r0 += step) {
+    const int64_t nr = rows - r0 > step ? step : rows - r0;
     DenseBatch bb = batch;
     for (int i = 0; i < nprob; ++i) {
       bb.p[i].x = reinterpret_cast<const char*>(batch.p[i].x) + r0 * Ks[i] * esz;
       bb.p[i].y = reinterpret_cast<char*>(batch.p[i].y) + r0 * Ns[i] * esz;
+      if (batch.p[i].residual) bb.p[i].residual = reinterpret_cast<const char*>(batch.p[i].residual) + r0 * Ns[i] * esz;
     }
     const int mt = nr <= 16 ? 1 : nr <= 32 ? 2 : 4;
     int rc = dispatch_dtype(act_dtype, [&](auto ta) {
       using TA = decltype(ta);
       if (mt == 1) hipLaunchKernelGGL((dense_kernel<1, TA>), dim3(tiles), dim3(256), 0, as_stream(stream), bb, (int)nr);
-      else if (mt == 2) hipLaunchKernelGGL((dense_kernel<2, TA>), dim3(tiles), dim3(256), 0, as_stream(stream), bb, (int)nr);
-      else hipLaunchKernelGGL((dense_kernel<4, TA>), dim3(tiles), dim3(256), 0, as_stream(stream), bb, (int)nr);
+      if constexpr (std::is_same<TA, float>::value) {
+        if (mt == 2) hipLaunchKernelGGL((dense_kernel<2, TA>), dim3(tiles), dim3(256), 0, as_stream(stream), bb, (int)nr);
+        if (mt == 4) hipLaunchKernelGGL((dense_kernel<4, TA>), dim3(tiles), dim3(256), 0, as_stream(stream), bb, (int)nr);
+      }
       return check_launch("dense_kernel");
     });
     if (rc) return rc;

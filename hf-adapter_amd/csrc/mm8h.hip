@@ -47,6 +47,7 @@
 //    8 column tiles (their x rows and weight columns stay in that XCD's L2).
 #include <string>
 
+#include "dense_common.h"
 #include "mm8t_common.h"
 
 namespace rwkv7mi {
@@ -646,6 +647,36 @@ extern "C" int rwkv7mi_mm8t_gemm_prefill_ws(int nprob, const void* const* x, con
   return mh_gemm_launch<__half>(b, nprob, rows, I, O, ws, ws_bytes, stream, w);
 }
 
+namespace rwkv7mi {
+// Whether a dense prefill product runs on the tile kernel (dense_tile.hip), which
+// reads W where it is, instead of the W copy and the 256 x 256 tiles: its K
+// splits (fp32 partials in the room the copy would take), 0 for the latter.
+static int mh_dense_tile(int nprob, const void* const* x, const void* const* W, int64_t rows, int64_t I, int64_t O,
+                         int act_dtype) {
+  DenseBatch d{};
+  d.nprob = nprob;
+  for (int i = 0; i < nprob; ++i) {
+    if ((reinterpret_cast<uintptr_t>(x[i]) | reinterpret_cast<uintptr_t>(W[i])) & 15) return 0;
+    d.p[i].N = (int)O;
+    d.p[i].K = (int)I;
+  }
+  if (!dense_tile_supported(d, rows, act_dtype)) return 0;
+  const int64_t tiles = mh_tiles(nprob, rows, O), SB = (I + 63) / 64, pb = mh_part_bytes(nprob, rows, O);
+  // the 256 x 256 form: copy W (read and written) and a launch, then rounds of tiles
+  const double big = 8.0 + mh_weight_bytes(nprob, I, O) * 2 / 3e6 +
+                     (tiles + 255) / 256 * (SB + 8) * (1.1 + 0.56 * std::min<double>(1.0, tiles / 256.0));
+  int best = 0;
+  double cost = big;
+  for (int S = 1; S <= 8; ++S) {
+    const int64_t sps = (SB + S - 1) / S;
+    if (S > 1 && (sps < 4 || (SB + sps - 1) / sps != S || S * pb > mh_weight_bytes(nprob, I, O))) continue;
+    const double t = dense_tile_us(d, rows, S) + (S > 1 ? 5.0 + 2.0 * S * pb / 4e6 : 0.0);
+    if (t < cost) cost = t, best = S;
+  }
+  return best;
+}
+}  // namespace rwkv7mi
+
 extern "C" int rwkv7mi_dense_gemm_prefill_ws(int nprob, const void* const* x, const void* const* W,
                                              const void* const* bias, const void* const* residual, void* const* y,
                                              const int* epilogue, int64_t rows, int64_t I, int64_t O, int act_dtype,
@@ -656,6 +687,32 @@ extern "C" int rwkv7mi_dense_gemm_prefill_ws(int nprob, const void* const* x, co
     return fail(RWKV7MI_EINVAL, w + ": fp16 or bf16 activations and weights");
   if (int rc = mh_check(w, nprob, rows, I, O, ws, ws_bytes)) return rc;
   if (rows == 0) return RWKV7MI_OK;
+  if (const int S = mh_dense_tile(nprob, x, W, rows, I, O, act_dtype)) {
+    MhBatch t{};
+    DenseBatch d{};
+    d.nprob = nprob;
+    for (int i = 0; i < nprob; ++i) {
+      if (!W[i]) return fail(RWKV7MI_EINVAL, w + ": null pointer");
+      if (int rc = mh_prob(w, t.p[i], x[i], W[i], bias ? bias[i] : nullptr, residual ? residual[i] : nullptr, y[i],
+                           epilogue[i], O))
+        return rc;
+      d.p[i] = DenseProb{x[i], W[i], t.p[i].bias, epilogue[i] == RWKV7MI_EPI_RESIDUAL ? t.p[i].residual : nullptr, y[i],
+                         (int)O, (int)I, epilogue[i] == RWKV7MI_EPI_RELU2 ? ACT_RELU2 : ACT_NONE, 0};
+    }
+    t.rows = (int)rows;
+    t.O = (int)O;
+    t.S = S;
+    t.ldp = (O + 31) / 32 * 32;
+    t.part = S > 1 ? static_cast<float*>(ws) : nullptr;
+    if (int rc = dense_tile_run(d, rows, act_dtype, S, t.part, t.ldp, stream)) return rc;
+    if (S == 1) return RWKV7MI_OK;
+    const dim3 rgrid((unsigned)((rows * (t.ldp / 8) + 255) / 256), (unsigned)nprob);
+    if (act_dtype == RWKV7MI_BF16)
+      hipLaunchKernelGGL(mm8h_reduce_kernel<__hip_bfloat16>, rgrid, dim3(256), 0, as_stream(stream), t);
+    else
+      hipLaunchKernelGGL(mm8h_reduce_kernel<__half>, rgrid, dim3(256), 0, as_stream(stream), t);
+    return check_launch("mm8h_reduce_kernel");
+  }
   const int64_t per_prob = mh_weight_bytes(1, I, O);
   MhBatch b{};
   MhRelBatch r{};

@@ -128,6 +128,7 @@ SIGNATURES = {
     "rwkv7mi_seq_norm_mix": (_i32, [_c_p] * 7 + [_i64, _i64, _i64, _i64, _f32, _i32, _i32, _c_p]),
     "rwkv7mi_layer_norm": (_i32, [_c_p] * 4 + [_i64, _i64, _f32, _i32, _i32, _c_p]),
     "rwkv7mi_dense_multi": (_i32, [_c_p] * 7 + [_i64, _i64, _i32, _c_p]),
+    "rwkv7mi_dense_multi_residual": (_i32, [_c_p] * 8 + [_i64, _i64, _i32, _c_p]),
     "rwkv7mi_state_prep": (_i32, [_c_p] * 12 + [_i64, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _c_p]),
     "rwkv7mi_output_prepare": (_i32, [_c_p] * 9 + [_i64, _i64, _i64, _f32, _i32, _i32, _c_p]),
 }

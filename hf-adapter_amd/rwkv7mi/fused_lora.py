@@ -18,8 +18,9 @@ from . import workspace as _ws
 ACT_NONE, ACT_TANH, ACT_SIGMOID, ACT_RELU2 = 0, 1, 2, 3
 
 
-def dense_multi(problems, rows: int):
-    """problems: list of (x2 [rows,K], W [N,K], bias or None, y [rows,N], act)."""
+def dense_multi(problems, rows: int, residuals=None):
+    """problems: list of (x2 [rows,K], W [N,K], bias or None, y [rows,N], act);
+    ``residuals`` (one ``[rows, N]`` tensor or None each) are added after the activation."""
     xs = [p[0] for p in problems]
     Ws = [p[1] for p in problems]
     bs = [p[2] for p in problems]
@@ -29,8 +30,9 @@ def dense_multi(problems, rows: int):
     Ks = (ctypes.c_int64 * k)(*[int(p[1].shape[1]) for p in problems])
     acts = (ctypes.c_int * k)(*[int(p[4]) for p in problems])
     _lib.require_gpu(*xs, *Ws, *ys, name="dense_multi")
-    _lib.call("rwkv7mi_dense_multi", _lib.ptr_array(xs), _lib.ptr_array(Ws), _lib.ptr_array(bs), _lib.ptr_array(ys),
-              Ns, Ks, acts, len(problems), int(rows), _lib.dtype_code(xs[0]), _lib.stream_of(xs[0]))
+    _lib.call("rwkv7mi_dense_multi_residual", _lib.ptr_array(xs), _lib.ptr_array(Ws), _lib.ptr_array(bs),
+              _lib.ptr_array(list(residuals) if residuals is not None else [None] * k), _lib.ptr_array(ys), Ns, Ks, acts,
+              len(problems), int(rows), _lib.dtype_code(xs[0]), _lib.stream_of(xs[0]))
 
 
 def lora_workspace_bytes(ranks, rows: int, D: int) -> int:

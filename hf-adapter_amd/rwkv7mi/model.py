@@ -195,11 +195,11 @@ def random_weights(cfg: NativeRWKV7Config, *, seed: int = 0, device="cpu", dtype
 class DenseLinear:
     """Unquantised Linear ``y = x W^T`` (projections below the MM8 size
     threshold, and every projection of an unquantised model such as the fp32
-    0.1B one): the HIP dense kernel up to 256 rows; above that, for fp16 and
-    bf16, the prefill MFMA GEMM (``rwkv7mi_dense_gemm_prefill_ws``: W copied
-    into the ``"mm8p"`` workspace in operand order, relu^2 / residual fused),
-    and for fp32 weights a plain library GEMM (hipBLASLt through torch) with
-    the epilogue as torch elementwise ops."""
+    0.1B one): the HIP dense kernels up to 256 rows; above that, for fp16 and
+    bf16, the prefill entry (``rwkv7mi_dense_gemm_prefill_ws``: the tile kernel,
+    or W copied into the ``"mm8p"`` workspace in operand order and the 256 x 256
+    MFMA GEMM; relu^2 / residual fused), and for fp32 weights a plain library
+    GEMM (hipBLASLt through torch) with the epilogue as torch elementwise ops."""
 
     def __init__(self, weight: torch.Tensor, bias: torch.Tensor | None = None):
         self.weight = weight.contiguous()
@@ -208,17 +208,8 @@ class DenseLinear:
 
     def apply(self, x2, out, *, act=ACT_NONE, residual=None):
         rows = int(x2.shape[0])
-        if (rows > 256 and x2.dtype in (torch.float16, torch.bfloat16) and self.weight.dtype == x2.dtype
-                and self.in_features % 16 == 0 and act in (0, 3) and not (act == 3 and residual is not None)
-                and x2.is_contiguous() and out.is_contiguous()):
-            epi = _lib.EPI_RELU2 if act == 3 else (_lib.EPI_RESIDUAL if residual is not None else _lib.EPI_NONE)
-            need = mm8_prefill_workspace_bytes(1, self.in_features, self.out_features)
-            ws = _ws.reserve(x2.device, need, "mm8p")
-            res = None if residual is None else residual.reshape(out.shape).contiguous()
-            arr = _lib.ptr_array
-            _lib.call("rwkv7mi_dense_gemm_prefill_ws", 1, arr([x2]), arr([self.weight]), arr([self.bias]), arr([res]),
-                      arr([out]), (ctypes.c_int * 1)(epi), rows, self.in_features, self.out_features, _lib.dtype_code(x2),
-                      _lib.ptr(ws), need, _lib.stream_of(x2))
+        if self._prefill_gemm(x2, out) and act in (0, 3) and not (act == 3 and residual is not None):
+            self._gemm([self], [x2], [out], act, [None if residual is None else residual.reshape(out.shape).contiguous()])
             return out
         if rows > 256:
             y = torch.nn.functional.linear(x2, self.weight, self.bias)
@@ -229,12 +220,51 @@ class DenseLinear:
             out.copy_(y)
             return out
         if residual is not None:
-            tmp = torch.empty_like(out)
-            dense_multi([(x2, self.weight, self.bias, tmp, act)], rows)
-            torch.add(residual, tmp, out=out)
-            return out
-        dense_multi([(x2, self.weight, self.bias, out, act)], rows)
+            if residual.dtype != out.dtype or residual.numel() != out.numel():  # torch's promotion / broadcasting
+                tmp = torch.empty_like(out)
+                dense_multi([(x2, self.weight, self.bias, tmp, act)], rows)
+                torch.add(residual, tmp, out=out)
+                return out
+            residual = residual.reshape(out.shape).contiguous()
+        dense_multi([(x2, self.weight, self.bias, out, act)], rows, [residual])
         return out
+
+    def _prefill_gemm(self, x2, out) -> bool:
+        return (int(x2.shape[0]) > 256 and x2.dtype in (torch.float16, torch.bfloat16)
+                and self.weight.dtype == x2.dtype and self.in_features % 16 == 0 and x2.is_contiguous()
+                and out.is_contiguous())
+
+    @staticmethod
+    def _gemm(lins, xs, outs, act, residuals):
+        """Up to four products of one shape above 256 rows, one launch."""
+        l, k = lins[0], len(lins)
+        need = mm8_prefill_workspace_bytes(k, l.in_features, l.out_features)
+        ws = _ws.reserve(xs[0].device, need, "mm8p")
+        arr = _lib.ptr_array
+        epis = [_lib.EPI_RELU2 if act == 3 else (_lib.EPI_RESIDUAL if r is not None else _lib.EPI_NONE)
+                for r in residuals]
+        _lib.call("rwkv7mi_dense_gemm_prefill_ws", k, arr(xs), arr([q.weight for q in lins]),
+                  arr([q.bias for q in lins]), arr(residuals), arr(outs), (ctypes.c_int * k)(*epis),
+                  int(xs[0].shape[0]), l.in_features, l.out_features, _lib.dtype_code(xs[0]), _lib.ptr(ws), need,
+                  _lib.stream_of(xs[0]))
+
+    @staticmethod
+    def apply_group(lins, xs, outs) -> bool:
+        """``[l.apply(x, o) for ...]`` as one launch; False (nothing run) when
+        the products do not share a shape and dtype."""
+        x = xs[0]
+        rows = int(x.shape[0])
+        if (len(lins) > 4 or len({(l.in_features, l.out_features, l.weight.dtype) for l in lins}) != 1
+                or any(q.dtype != x.dtype or tuple(q.shape) != tuple(x.shape) for q in xs)
+                or lins[0].weight.dtype != x.dtype):
+            return False
+        if rows <= 256:
+            dense_multi([(q, l.weight, l.bias, o, ACT_NONE) for l, q, o in zip(lins, xs, outs)], rows)
+            return True
+        if not all(l._prefill_gemm(q, o) for l, q, o in zip(lins, xs, outs)):
+            return False
+        DenseLinear._gemm(lins, list(xs), list(outs), ACT_NONE, [None] * len(lins))
+        return True
 
 
 class QuantLinear:
@@ -281,6 +311,8 @@ class QuantLinear:
                 mm8_gemm_multi_into(list(xs), [l.m for l in lins], list(outs))
             else:
                 mm8_gemm_prefill_multi_into(list(xs), [l.m for l in lins], list(outs))
+            return outs
+        if all(isinstance(l, DenseLinear) for l in lins) and DenseLinear.apply_group(lins, xs, outs):
             return outs
         for l, x2, o in zip(lins, xs, outs):
             l.apply(x2, o)
@@ -1032,6 +1064,8 @@ class NativeRWKV7ForCausalLM(_PreTrainedModel, _GenerationMixin):
             for L in self.layers:
                 if isinstance(L.r_proj, QuantLinear):
                     pneed = max(pneed, mm8_prefill_workspace_bytes(3, L.r_proj.in_features, L.r_proj.out_features, rows))
+                elif L.r_proj.weight.dtype != torch.float32:
+                    pneed = max(pneed, mm8_prefill_workspace_bytes(3, L.r_proj.in_features, L.r_proj.out_features))
             for lin in self._linears():
                 if isinstance(lin, QuantLinear):
                     pneed = max(pneed, mm8_prefill_workspace_bytes(1, lin.in_features, lin.out_features, rows))

@@ -781,6 +781,14 @@ int rwkv7mi_dense_multi(const void* const* xs, const void* const* Ws,
                         const int64_t* Ns, const int64_t* Ks, const int* acts,
                         int64_t nprob, int64_t rows, int act_dtype,
                         void* stream);
+/* The same with y_i += residual_i [rows, N_i] after the activation (residuals
+ * or single entries may be NULL; y_i may be residual_i). */
+int rwkv7mi_dense_multi_residual(const void* const* xs, const void* const* Ws,
+                                 const void* const* biases,
+                                 const void* const* residuals, void* const* ys,
+                                 const int64_t* Ns, const int64_t* Ks,
+                                 const int* acts, int64_t nprob, int64_t rows,
+                                 int act_dtype, void* stream);
 
 /* ------------------------------------------- scan input / output prep */
 

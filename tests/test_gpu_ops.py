@@ -260,6 +260,60 @@ def test_wag_lora_dtypes(oracle, dt, rows, D):
 
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,K,Ns", [(2, 72, (200,)), (3, 768, (1544, 8, 33)), (5, 1096, (16, 17, 300)),
+                                       (17, 264, (130,)), (33, 64, (65, 64)), (130, 776, (260,)),
+                                       (256, 2048, (768, 768, 768, 100))])
+def test_dense_tile_edges(dt, rows, K, Ns):
+    """The tile kernel and its rule at the edges of its tiles: row, column and
+    K remainders, one to four problems of different widths, bias, activation
+    and a residual that is the output itself, against fp64."""
+    from rwkv7mi.fused_lora import dense_multi
+
+    rng = np.random.default_rng(rows + K)
+    xs = [_t(rng.standard_normal((rows, K)), dt) for _ in Ns]
+    Ws = [_t(rng.standard_normal((n, K)) * 0.05, dt) for n in Ns]
+    bs = [_t(rng.standard_normal(n) * 0.1, dt) if i != 1 else None for i, n in enumerate(Ns)]
+    res = [_t(rng.standard_normal((rows, n)), dt) if i % 2 == 0 else None for i, n in enumerate(Ns)]
+    acts = [0, 2, 3, 1][: len(Ns)]
+    ys = [torch.full((rows, n), float("nan"), device="cuda", dtype=dt) if r is None else r.clone()
+          for n, r in zip(Ns, res)]
+    dense_multi(list(zip(xs, Ws, bs, ys, acts)), rows, [None if r is None else y for r, y in zip(res, ys)])
+    torch.cuda.synchronize()
+    act = {0: lambda v: v, 1: np.tanh, 2: lambda v: 1 / (1 + np.exp(-v)), 3: lambda v: np.maximum(v, 0) ** 2}
+    step = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8  # one rounding of the output, fp32 sums
+    for x, W, b, r, y, a in zip(xs, Ws, bs, res, ys, acts):
+        ref = act[a](_f(x) @ _f(W).T + (0 if b is None else _f(b))) + (0 if r is None else _f(r))
+        assert np.all(np.abs(_f(y) - ref) <= step * np.abs(ref) + 2e-5 * max(1.0, np.abs(ref).max()))
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,K,N,epi", [(257, 768, 768, 2), (300, 3072, 104, 1), (520, 784, 3072, 0),
+                                          (700, 4096, 264, 2), (1500, 2048, 2048, 0)])
+def test_dense_prefill_routes(dt, rows, K, N, epi):
+    """Above 256 rows: the tile kernel, its K splits (whose partials take the
+    place of W's copy) and the 256 x 256 form, one and three products a call."""
+    from rwkv7mi.model import DenseLinear
+
+    rng = np.random.default_rng(rows + K + N)
+    lins = [DenseLinear(_t(rng.standard_normal((N, K)) * 0.05, dt), _t(rng.standard_normal(N) * 0.1, dt))
+            for _ in range(3)]
+    xs = [_t(rng.standard_normal((rows, K)), dt) for _ in range(3)]
+    step = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8
+    refs = [_f(x) @ _f(l.weight).T + _f(l.bias) for x, l in zip(xs, lins)]
+    tol = lambda r: step * np.abs(r) + 2e-5 * np.abs(r).max()
+    outs = [torch.full((rows, N), float("nan"), device="cuda", dtype=dt) for _ in range(3)]
+    assert DenseLinear.apply_group(lins, xs, outs)
+    res = _t(rng.standard_normal((rows, N)), dt)
+    y = res.clone()
+    lins[0].apply(xs[0], y, act=3 if epi == 1 else 0, residual=y if epi == 2 else None)
+    torch.cuda.synchronize()
+    for o, r in zip(outs, refs):
+        assert np.all(np.abs(_f(o) - r) <= tol(r))
+    ref = np.maximum(refs[0], 0) ** 2 if epi == 1 else refs[0] + (_f(res) if epi == 2 else 0)
+    assert np.all(np.abs(_f(y) - ref) <= tol(ref))
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rows,D,A,ranks", [(65, 512, 264, (64, 72, 128, 8)), (257, 72, 100, (32, 96, 40, 16)),
                                             (400, 1088, 520, (64, 64, 128, 32)), (2100, 264, 256, (24, 128, 56, 32))])
 def test_lora_row_pair_edges(oracle, dt, rows, D, A, ranks):
