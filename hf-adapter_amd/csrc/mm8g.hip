@@ -39,6 +39,7 @@ namespace rwkv7mi {
 constexpr int MM8G_ROWS = 64;   // rows per workgroup tile
 constexpr int MM8G_GPW = 2;     // 16-column groups per wave
 constexpr int MM8G_COLS = 4 * MM8G_GPW * MM8T_COLS;  // 128 columns per workgroup
+constexpr int MM8R_COLS = 256;  // middle-row kernel: columns per workgroup
 constexpr int MM8G_MAXKB = 8;   // K blocks (128 inputs) staged per workgroup
 constexpr int MM8G_DEPTH = 4;   // weight ring depth (steps): ~1.5 us of HBM latency at the loop's pace
 
@@ -48,6 +49,7 @@ struct Mm8gBatch {
   _Float16* xl;  // same shape: fp16(x ry - xp), written and read for fp32 activations only
   float* rsum;   // [nprob][rows][3] sum x, sum x my, sum x ry
   float* part;   // [S][nprob][rows][O] fp32 partial products (S > 1)
+  float* rscale; // [nprob][rows] (mm8r_kernel, else null) 2^-e of a row whose xp is x ry 2^e
   int rows, I, O, KB, S, ctiles, nprob;
   int cw;  // workgroups per (problem, split, row tile): column-tile stride
   // Tail workgroups x >= cw S: the decode LoRA down projections (inputs ready
@@ -99,8 +101,10 @@ __device__ __forceinline__ float mm8g_finish(const Mm8tProb& P, float acc, float
 
 // x' = fp16(x ry) for one (problem, row) per workgroup, zero past I up to the
 // whole-block width KB 128, and the row's fp32 sums (lanes in a fixed DPP
-// order, then the four waves in order)
-template <typename TA, typename TM>
+// order, then the four waves in order).  SCALE: x' = fp16(x ry 2^e) with e
+// putting the row's largest value just below 2^15, so neither large bf16 rows
+// overflow nor small rows fall into fp16's subnormals; 2^-e goes to rscale.
+template <typename TA, typename TM, bool SCALE>
 __global__ __launch_bounds__(256) void mm8g_prep_kernel(const Mm8gBatch B) {
   const int p = blockIdx.y;
   const int64_t row = blockIdx.x;
@@ -115,6 +119,36 @@ __global__ __launch_bounds__(256) void mm8g_prep_kernel(const Mm8gBatch B) {
   _Float16* xlo = B.xl + ((int64_t)p * B.rows + row) * KBK;
   float a = 0.f, b = 0.f, c = 0.f;
   constexpr int PB = 4;  // passes whose loads are in flight together
+  float scale = 1.f;
+  if constexpr (SCALE) {
+    float m = 0.f;
+    for (int k0 = 8 * tid; k0 < I; k0 += 8 * 256 * PB) {
+      Raw8<TA> xv[PB];
+      Raw8<TM> rr[PB];
+#pragma unroll
+      for (int u = 0; u < PB; ++u) {
+        const int k = k0 + 8 * 256 * u;
+        xv[u] = mm8t_ld8<TA>(xr, (uint32_t)k, k < I);
+        rr[u] = mm8t_ld8<TM>(ryr, (uint32_t)k, k < I);
+      }
+#pragma unroll
+      for (int u = 0; u < PB; ++u) {
+        float x[8], rv[8];
+        mm8t_cvt8(xv[u], x);
+        mm8t_cvt8(rr[u], rv);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(x[e] * rv[e]));
+      }
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+    __shared__ float wmax[4];
+    if (lane == 0) wmax[wave] = m;
+    __syncthreads();
+    m = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+    if (m > 0.f && m < INFINITY) scale = ldexpf(1.f, min(max(14 - ilogbf(m), -100), 100));
+    if (tid == 0) B.rscale[(int64_t)p * B.rows + row] = 1.f / scale;  // (a power of two: exact)
+  }
   for (int k0 = 8 * tid; k0 < KBK; k0 += 8 * 256 * PB) {
     Raw8<TA> xv[PB];
     Raw8<TM> rr[PB], mr[PB];
@@ -137,7 +171,7 @@ __global__ __launch_bounds__(256) void mm8g_prep_kernel(const Mm8gBatch B) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const float xp = x[e] * rv[e];
-        h[e] = (_Float16)xp;
+        h[e] = (_Float16)(SCALE ? xp * scale : xp);
         l[e] = (_Float16)(xp - (float)h[e]);
         a += x[e];
         b += x[e] * mv[e];
@@ -380,9 +414,204 @@ __global__ __launch_bounds__(256) void mm8g_reduce_kernel(const Mm8gBatch B) {
   }
   const float* rsum = B.rsum + ((int64_t)p * B.rows + row) * 3;
   const float s0 = rsum[0], s1 = rsum[1], s2 = rsum[2];
+  const float sc = B.rscale ? B.rscale[(int64_t)p * B.rows + row] : 1.f;
 #pragma unroll
   for (int v = 0; v < V; ++v)
-    reinterpret_cast<TA*>(P.y)[idx + v] = from_f32<TA>(mm8g_finish<TA, TM>(P, a[v], s0, s1, s2, row, o + v, O));
+    reinterpret_cast<TA*>(P.y)[idx + v] = from_f32<TA>(mm8g_finish<TA, TM>(P, a[v] * sc, s0, s1, s2, row, o + v, O));
+}
+
+// ---- middle row counts: 128 rows x 256 columns a workgroup over a K range.
+// What a CU pulls through its L1 bounds these products (35-50 GB/s a CU): a
+// tile of 64 rows x 128 or 256 columns that every wave loads for itself spends
+// most of its time there.  Here eight waves share one tile, every byte of x' and
+// of the packed weights comes in once, by DMA straight into LDS:
+//  * a step is 64 inputs: 16 KB of x' (fp16, from the pre-pass) and 16 KB of
+//    weight bytes, four stages, three steps ahead, one barrier a step;
+//  * x': chunk 2 kg + u of a row at position (2 kg + u) ^ key(row) of its 128
+//    bytes, which leaves the operand reads free of bank conflicts on gfx950;
+//  * weights: a 16-column group's 64 inputs are 1 KB in the order of the lanes
+//    that use them, so both the DMA and the reads are linear; a lane's 16 bytes
+//    are two operands, exact w - 128 in fp16, built for the next step between
+//    this step's MFMAs;
+//  * wave w: rows 64 (w / 4) .. +63, columns 64 (w % 4) .. +63; W is the A
+//    operand, so a lane holds one row and 4 consecutive columns of a group.
+constexpr int MM8R_ROWS = 128;
+constexpr int MM8R_NST = 4;                                // stages
+constexpr int MM8R_XB = MM8R_ROWS * 128;                   // x' bytes of a stage
+constexpr int MM8R_STAGE = MM8R_XB + MM8R_COLS * 64;       // + weight bytes
+__device__ __forceinline__ int mm8r_key(int r) { return (r & 7) ^ ((r >> 3) & 1); }
+
+template <typename TA, typename TM>
+__global__ __launch_bounds__(512, 1) void mm8r_kernel(const Mm8gBatch B) {
+  extern __shared__ __align__(16) char smem[];
+  typedef __attribute__((address_space(3))) void* lds_ptr;
+  const int p = blockIdx.y;
+  const Mm8tProb& P = B.p[p];
+  const int O = B.O, KB = B.KB, KBK = KB * 128;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, kg = lane >> 4;
+  const int o0 = MM8R_COLS * ((int)blockIdx.x % B.ctiles), row0 = MM8R_ROWS * ((int)blockIdx.x / B.ctiles);
+  const int nrow = min(MM8R_ROWS, B.rows - row0);
+  const int ngroups = min(MM8R_COLS / MM8T_COLS, (O + MM8T_COLS - 1) / MM8T_COLS - o0 / MM8T_COLS);
+  const int s0 = blockIdx.z * B.cw, s1 = min(2 * KB, s0 + B.cw);  // cw: steps of a split (even)
+
+  // descriptors end at the tile's last row / column group: past them zeros
+  const __amdgpu_buffer_rsrc_t xr =
+      mm8t_rsrc(B.xp + ((int64_t)p * B.rows + row0) * KBK, (uint32_t)nrow * (uint32_t)KBK * 2u);
+  const __amdgpu_buffer_rsrc_t wr =
+      mm8t_rsrc(P.w + (int64_t)(o0 / MM8T_COLS) * KB * 2048, (uint32_t)ngroups * (uint32_t)KB * 2048u);
+  // this wave's share of a step: x' rows 8 (wave + 8 u) .. +7 (lane l: row l /
+  // 8, position l % 8) and column groups wave + 8 u
+  int xo[2], wo[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int r = 8 * (wave + 8 * u) + (lane >> 3);
+    xo[u] = (r * KBK + 8 * ((lane & 7) ^ mm8r_key(r))) * 2;
+    wo[u] = (wave + 8 * u) * KB * 2048 + 16 * lane;
+  }
+  auto issue = [&](int s) {
+    char* st = smem + (s & (MM8R_NST - 1)) * MM8R_STAGE;
+    const int k = s0 + s;
+    const bool ok = k < s1;  // (uniform) past the range: zeros
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_ptr)(st + 1024 * (wave + 8 * u)), 16,
+                                               ok ? xo[u] : (int)MM8T_OOB, ok ? 128 * k : 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_ptr)(st + MM8R_XB + 1024 * (wave + 8 * u)), 16,
+                                               ok ? wo[u] : (int)MM8T_OOB, ok ? 1024 * k : 0, 0, 0);
+    }
+  };
+  f32x4 acc[4][4];
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) acc[m][g] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  const int rs = 64 * (wave >> 2), cq = 4 * (wave & 3);
+  const int key = mm8r_key(n);
+  auto raw_w = [&](int s, int g) {
+    const char* st = smem + (s & (MM8R_NST - 1)) * MM8R_STAGE;
+    return *reinterpret_cast<const u32x4*>(st + MM8R_XB + 1024 * (cq + g) + 16 * lane);
+  };
+  auto dequant = [&](const u32x4& v, f16x8 (&w)[2]) {
+    const uint32_t d0 = v[0], d1 = v[1], d2 = v[2], d3 = v[3];
+    w[0] = mm8g_b_operand(d0, d1);
+    w[1] = mm8g_b_operand(d2, d3);
+  };
+  auto read_x = [&](int s, f16x8 (&xa)[4][2]) {
+    const char* st = smem + (s & (MM8R_NST - 1)) * MM8R_STAGE;
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        xa[m][u] = *reinterpret_cast<const f16x8*>(st + (rs + 16 * m + n) * 128 + 16 * ((2 * kg + u) ^ key));
+  };
+  // Step s: its operands are in xa, wb; step s + 1 landed (only step s + 2's
+  // four loads may be pending) and visible; step s + 3 into the stage of step s
+  // - 1, which every wave has left.  All of step s + 1's LDS reads go out first,
+  // so they have half of the step's MFMAs to land; its weights are dequantised
+  // between the other half.
+  auto step = [&](int s, const f16x8 (&xa)[4][2], const f16x8 (&wb)[4][2], f16x8 (&xn)[4][2], f16x8 (&wn)[4][2]) {
+    __builtin_amdgcn_s_waitcnt(0x0F74);  // vmcnt(4)
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    issue(s + 3);
+    u32x4 rw[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) rw[g] = raw_w(s + 1, g);
+    read_x(s + 1, xn);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) acc[0][g] = mfma16x16x32(wb[g][u], xa[0][u], acc[0][g]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int m = 1; m < 4; ++m)
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) acc[m][g] = mfma16x16x32(wb[g][u], xa[m][u], acc[m][g]);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) dequant(rw[g], wn[g]);
+#pragma unroll
+    for (int i = 0; i < 24; ++i) {  // the 64 dequantising VALU spread over the 24 MFMAs
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  f16x8 x0[4][2], x1[4][2], w0[4][2], w1[4][2];
+#pragma unroll
+  for (int s = 0; s < 3; ++s) issue(s);
+  __builtin_amdgcn_s_waitcnt(0x0F78);  // vmcnt(8): step 0 landed
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int g = 0; g < 4; ++g) dequant(raw_w(0, g), w0[g]);
+  read_x(0, x0);
+  for (int s = 0; s < s1 - s0; s += 2) {
+    step(s, x0, w0, x1, w1);
+    step(s + 1, x1, w1, x0, w0);
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the trailing loads have landed before the waves exit
+
+  // lane: row 16 m + n, columns c .. +3 of each group
+  float* part = B.S > 1 ? B.part + ((int64_t)blockIdx.z * B.nprob + p) * B.rows * O : nullptr;
+  const bool vec = O % 4 == 0;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int c = o0 + 16 * (cq + g) + 4 * kg;
+    if (c >= O) continue;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const int64_t row = row0 + rs + 16 * m + n;
+      if (row >= B.rows) continue;
+      if (part) {
+        if (vec) {
+          *reinterpret_cast<f32x4*>(part + row * O + c) = acc[m][g];
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (c + e < O) part[row * O + c + e] = acc[m][g][e];
+        }
+      } else {
+        const float* q = B.rsum + ((int64_t)p * B.rows + row) * 3;
+        const float sc = B.rscale[(int64_t)p * B.rows + row];
+        TA o4[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (c + e < O) o4[e] = from_f32<TA>(mm8g_finish<TA, TM>(P, acc[m][g][e] * sc, q[0], q[1], q[2], row, c + e, O));
+        TA* y = reinterpret_cast<TA*>(P.y) + row * O + c;
+        if (vec && !(reinterpret_cast<uintptr_t>(y) & 7)) {
+          *reinterpret_cast<uint2*>(y) = make_uint2(
+              (uint32_t)__builtin_bit_cast(uint16_t, o4[0]) | ((uint32_t)__builtin_bit_cast(uint16_t, o4[1]) << 16),
+              (uint32_t)__builtin_bit_cast(uint16_t, o4[2]) | ((uint32_t)__builtin_bit_cast(uint16_t, o4[3]) << 16));
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (c + e < O) y[e] = o4[e];
+        }
+      }
+    }
+  }
+}
+
+// K splits of the middle-row kernel: rounds of 256 workgroups (one a CU) against
+// the partials' traffic
+static int mm8r_splits(int nprob, int64_t rows, int64_t I, int64_t O, double* us = nullptr) {
+  const int64_t KB = (I + 127) / 128;  // two steps each
+  const int64_t tiles = nprob * ((rows + MM8R_ROWS - 1) / MM8R_ROWS) * ((O + MM8R_COLS - 1) / MM8R_COLS);
+  const double pb = 4.0 * nprob * rows * O;
+  int best = 1;
+  double cost = 1e30;
+  for (int S = 1; S <= 32 && (S == 1 || tiles * S <= 256); ++S) {
+    const int64_t bps = (KB + S - 1) / S;
+    if (S > 1 && (bps < 2 || (KB + bps - 1) / bps != S)) continue;  // no empty split
+    const double t = ((tiles * S + 255) / 256) * (4.0 + 2.2 * bps) + (S > 1 ? 4.0 + 2.0 * pb * S / 4e6 : 0.0);
+    if (t < cost) cost = t, best = S;
+  }
+  if (us) *us = cost;
+  return best;
 }
 
 // Split count: explicit, or the fewest (a power of two) that keep every
@@ -425,23 +654,18 @@ extern "C" size_t rwkv7mi_mm8t_gemm_workspace_bytes(int nprob, int64_t rows, int
   return mm8g_ws_layout(mm8g_splits(rows, I, O, nprob, splits), nprob, rows, I, O).total;
 }
 
-static int mm8g_run(const char* who, int nprob, const void* const* x, const uint8_t* const* w_blk,
-                    const void* const* mx, const void* const* rx, const void* const* my, const void* const* ry,
-                    const void* const* bias, const void* const* residual, void* const* y, const int* epilogue,
-                    int64_t rows, int64_t I, int64_t O, int act_dtype, int meta_dtype, int splits, void* workspace,
-                    size_t workspace_bytes, void* stream, const LoraBatch* tl = nullptr, float* tl_part = nullptr,
-                    int tl_tiles = 0) {
-  const std::string w(who);
+// argument checks shared by the entries; fills b's problems and shape
+static int mm8g_problems(const std::string& w, Mm8gBatch& b, int nprob, const void* const* x,
+                         const uint8_t* const* w_blk, const void* const* mx, const void* const* rx,
+                         const void* const* my, const void* const* ry, const void* const* bias,
+                         const void* const* residual, void* const* y, const int* epilogue, int64_t rows, int64_t I,
+                         int64_t O, int act_dtype, int meta_dtype) {
   if (nprob < 1 || nprob > MM8T_MAXPROB) return fail(RWKV7MI_EINVAL, w + ": 1..4 problems per launch");
   if (!x || !w_blk || !mx || !rx || !my || !ry || !y || !epilogue) return fail(RWKV7MI_EINVAL, w + ": null array");
-  if (rows < 0 || I <= 0 || O <= 0 || splits < 0) return fail(RWKV7MI_EINVAL, w + ": bad shape");
+  if (rows < 0 || I <= 0 || O <= 0) return fail(RWKV7MI_EINVAL, w + ": bad shape");
   if (rows == 0) return RWKV7MI_OK;
   if (I % 16) return fail(RWKV7MI_EINVAL, w + ": in_features must be a multiple of 16");
-  const int trows = act_dtype == RWKV7MI_F32 ? MM8G_ROWS / 2 : MM8G_ROWS;  // rows per tile (fp32: hi + lo)
-  if (I > (1 << 24) || O > (1 << 24) || rows > 65535LL * trows || rows * std::max(I, O) > INT32_MAX)
-    return fail(RWKV7MI_EINVAL, w + ": too large");
   if (!valid_dtype(act_dtype) || !valid_dtype(meta_dtype)) return fail(RWKV7MI_EINVAL, w + ": bad dtype");
-  Mm8gBatch b{};
   for (int i = 0; i < nprob; ++i) {
     Mm8tProb q{x[i], nullptr, w_blk[i], mx[i], rx[i], my[i], ry[i], bias ? bias[i] : nullptr,
                residual ? residual[i] : nullptr, y[i], epilogue[i]};
@@ -453,6 +677,44 @@ static int mm8g_run(const char* who, int nprob, const void* const* x, const uint
     if (q.epilogue == RWKV7MI_EPI_RESIDUAL && !q.residual) return fail(RWKV7MI_EINVAL, w + ": residual missing");
     b.p[i] = q;
   }
+  b.rows = (int)std::min<int64_t>(rows, INT32_MAX);
+  b.I = (int)std::min<int64_t>(I, INT32_MAX);
+  b.O = (int)std::min<int64_t>(O, INT32_MAX);
+  b.KB = (int)std::min<int64_t>((I + 127) / 128, INT32_MAX);
+  b.nprob = nprob;
+  return RWKV7MI_OK;
+}
+
+// the split reduce of b's partials
+template <typename TA, typename TM>
+static int mm8g_reduce(const Mm8gBatch& b, void* stream) {
+  const int64_t n = (int64_t)b.rows * b.O;
+  if (b.O % 4 == 0) {
+    const dim3 rgrid((unsigned)((n / 4 + 255) / 256), (unsigned)b.nprob);
+    hipLaunchKernelGGL((mm8g_reduce_kernel<TA, TM, 4>), rgrid, dim3(256), 0, as_stream(stream), b);
+  } else {
+    const dim3 rgrid((unsigned)((n + 255) / 256), (unsigned)b.nprob);
+    hipLaunchKernelGGL((mm8g_reduce_kernel<TA, TM, 1>), rgrid, dim3(256), 0, as_stream(stream), b);
+  }
+  return check_launch("mm8g_reduce_kernel");
+}
+
+static int mm8g_run(const char* who, int nprob, const void* const* x, const uint8_t* const* w_blk,
+                    const void* const* mx, const void* const* rx, const void* const* my, const void* const* ry,
+                    const void* const* bias, const void* const* residual, void* const* y, const int* epilogue,
+                    int64_t rows, int64_t I, int64_t O, int act_dtype, int meta_dtype, int splits, void* workspace,
+                    size_t workspace_bytes, void* stream, const LoraBatch* tl = nullptr, float* tl_part = nullptr,
+                    int tl_tiles = 0) {
+  const std::string w(who);
+  Mm8gBatch b{};
+  if (int rc = mm8g_problems(w, b, nprob, x, w_blk, mx, rx, my, ry, bias, residual, y, epilogue, rows, I, O, act_dtype,
+                             meta_dtype))
+    return rc;
+  if (splits < 0) return fail(RWKV7MI_EINVAL, w + ": bad shape");
+  if (rows == 0) return RWKV7MI_OK;
+  const int trows = act_dtype == RWKV7MI_F32 ? MM8G_ROWS / 2 : MM8G_ROWS;  // rows per tile (fp32: hi + lo)
+  if (I > (1 << 24) || O > (1 << 24) || rows > 65535LL * trows || rows * std::max(I, O) > INT32_MAX)
+    return fail(RWKV7MI_EINVAL, w + ": too large");
   const int S = mm8g_splits(rows, I, O, nprob, splits);
   const int64_t KB = (I + 127) / 128;
   if ((int64_t)MM8G_ROWS * KB * 128 * 2 > INT32_MAX) return fail(RWKV7MI_EINVAL, w + ": too large");
@@ -462,12 +724,7 @@ static int mm8g_run(const char* who, int nprob, const void* const* x, const uint
   if (!workspace || workspace_bytes < lay.total || (reinterpret_cast<uintptr_t>(workspace) & 255))
     return fail(RWKV7MI_ESIZE, w + ": workspace missing, unaligned or smaller than "
                                    "rwkv7mi_mm8t_gemm_workspace_bytes");
-  b.rows = (int)rows;
-  b.I = (int)I;
-  b.O = (int)O;
-  b.KB = (int)KB;
   b.S = S;
-  b.nprob = nprob;
   b.ctiles = (int)((O + MM8G_COLS - 1) / MM8G_COLS);
   char* wsb = reinterpret_cast<char*>(workspace);
   b.xp = reinterpret_cast<_Float16*>(wsb + lay.xp);
@@ -508,7 +765,7 @@ static int mm8g_run(const char* who, int nprob, const void* const* x, const uint
       if (int rc = raise_dynamic_lds(reinterpret_cast<const void*>(&mm8g_kernel<TA, TM, MM8G_DEPTH, 4>),
                                      MM8G_ROWS * (128 * 4 + 8) * 2, raised_4, "mm8g_kernel"))
         return rc;
-      hipLaunchKernelGGL((mm8g_prep_kernel<TA, TM>), dim3((unsigned)rows, (unsigned)nprob), dim3(256), 0,
+      hipLaunchKernelGGL((mm8g_prep_kernel<TA, TM, false>), dim3((unsigned)rows, (unsigned)nprob), dim3(256), 0,
                          as_stream(stream), b);
       int rc = check_launch("mm8g_prep_kernel");
       if (rc != RWKV7MI_OK) return rc;
@@ -518,14 +775,7 @@ static int mm8g_run(const char* who, int nprob, const void* const* x, const uint
         hipLaunchKernelGGL((mm8g_kernel<TA, TM, MM8G_DEPTH, MM8G_MAXKB>), grid, dim3(256), lds, as_stream(stream), b);
       rc = check_launch("mm8g_kernel");
       if (rc != RWKV7MI_OK || S == 1) return rc;
-      if (O % 4 == 0) {
-        const dim3 rgrid((unsigned)((rows * O / 4 + 255) / 256), (unsigned)nprob);
-        hipLaunchKernelGGL((mm8g_reduce_kernel<TA, TM, 4>), rgrid, dim3(256), 0, as_stream(stream), b);
-      } else {
-        const dim3 rgrid((unsigned)((rows * O + 255) / 256), (unsigned)nprob);
-        hipLaunchKernelGGL((mm8g_reduce_kernel<TA, TM, 1>), rgrid, dim3(256), 0, as_stream(stream), b);
-      }
-      return check_launch("mm8g_reduce_kernel");
+      return mm8g_reduce<TA, TM>(b, stream);
     });
   });
 }
@@ -564,6 +814,92 @@ extern "C" int rwkv7mi_mm8t_gemm_multi_lora(int nprob, const void* const* x, con
     return fail(RWKV7MI_ESIZE, std::string(who) + ": LoRA partial buffer missing, unaligned or too small");
   return mm8g_run(who, nprob, x, w_blk, mx, rx, my, ry, bias, residual, y, epilogue, rows, I, O, act_dtype,
                   meta_dtype, splits, workspace, workspace_bytes, stream, &lb, lora_part, tiles);
+}
+
+// ---- middle rows (mm8r_kernel), fp16 / bf16 activations
+// Whether these rows run faster on it.  Measured (key + value of an FFN, kernel
+// time, us): against mm8g_kernel at 7.2B widths (4096 / 16384) 64 rows 64 -> 66,
+// 100 rows 88 -> 76, 200 rows 147 -> 101; at 2048 / 8192 100 rows 45 -> 50, 200
+// rows 61 -> 61, so only where one product has 2^25 weights.  Against the
+// dequantise + GEMM form (300 / 600 / 1000 / 1500 / 2500 rows): 232 -> 149, 287
+// -> 247, 353 -> 312, 536 -> 526, 770 -> 875 at 7.2B widths, 107 -> 87, 128 ->
+// 100, 142 -> 116, 167 -> 186, 292 -> 309 at 2048; there by the two estimates
+// (that form's runs about a tenth high) up to 1024 rows.
+extern "C" int rwkv7mi_mm8t_rows_pays(int nprob, int64_t rows, int64_t I, int64_t O, int act_dtype) {
+  if (nprob < 1 || nprob > MM8T_MAXPROB || rows <= 64 || I <= 0 || O <= 0 || act_dtype == RWKV7MI_F32) return 0;
+  if (I % 16 || I > (1 << 22) || O > (1 << 24) || rows * std::max(I, O) > INT32_MAX) return 0;
+  if (rows <= 256) return I * O >= ((int64_t)1 << 25);
+  if (rows > 1024) return 0;
+  double us = 0;
+  mm8r_splits(nprob, rows, I, O, &us);
+  return us + 5.0 < 0.9 * mm8h_estimate_us(nprob, rows, I, O);
+}
+// workspace: x' | row sums | row scales | partials, each part 256-byte aligned
+struct Mm8rWs {
+  size_t rsum, rscale, part, total;
+};
+static Mm8rWs mm8r_ws_layout(int S, int nprob, int64_t rows, int64_t I, int64_t O) {
+  auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
+  Mm8rWs w{};
+  w.rsum = up((size_t)nprob * rows * (size_t)((I + 127) / 128) * 128u * 2u);
+  w.rscale = w.rsum + up((size_t)nprob * rows * 3u * 4u);
+  w.part = w.rscale + up((size_t)nprob * rows * 4u);
+  w.total = w.part + (S > 1 ? up((size_t)S * nprob * rows * O * 4u) : 0);
+  return w;
+}
+extern "C" int64_t rwkv7mi_mm8t_rows_workspace_bytes(int nprob, int64_t rows, int64_t I, int64_t O) {
+  if (nprob < 1 || nprob > MM8T_MAXPROB || rows <= 0 || I <= 0 || O <= 0) return 0;
+  return (int64_t)mm8r_ws_layout(mm8r_splits(nprob, rows, I, O), nprob, rows, I, O).total;
+}
+
+extern "C" int rwkv7mi_mm8t_rows_multi(int nprob, const void* const* x, const uint8_t* const* w_blk,
+                                       const void* const* mx, const void* const* rx, const void* const* my,
+                                       const void* const* ry, const void* const* bias, const void* const* residual,
+                                       void* const* y, const int* epilogue, int64_t rows, int64_t I, int64_t O,
+                                       int act_dtype, int meta_dtype, void* workspace, int64_t workspace_bytes,
+                                       void* stream) {
+  const std::string w("mm8t_rows_multi");
+  Mm8gBatch b{};
+  if (int rc = mm8g_problems(w, b, nprob, x, w_blk, mx, rx, my, ry, bias, residual, y, epilogue, rows, I, O, act_dtype,
+                             meta_dtype))
+    return rc;
+  if (rows == 0) return RWKV7MI_OK;
+  if (act_dtype == RWKV7MI_F32) return fail(RWKV7MI_EINVAL, w + ": fp16 or bf16 activations");
+  const int64_t KB = (I + 127) / 128;
+  // 32-bit offsets: 128 rows of x', 16 column groups of weights
+  if (I > (1 << 24) || O > (1 << 24) || (int64_t)MM8R_ROWS * KB * 256 >= (int64_t)MM8T_OOB ||
+      16 * KB * 2048 >= (int64_t)MM8T_OOB || rows * std::max(I, O) > INT32_MAX)
+    return fail(RWKV7MI_EINVAL, w + ": too large");
+  const int S = mm8r_splits(nprob, rows, I, O);
+  const Mm8rWs lay = mm8r_ws_layout(S, nprob, rows, I, O);
+  if (!workspace || workspace_bytes < (int64_t)lay.total || (reinterpret_cast<uintptr_t>(workspace) & 255))
+    return fail(RWKV7MI_ESIZE, w + ": workspace missing, unaligned or smaller than rwkv7mi_mm8t_rows_workspace_bytes");
+  b.S = S;
+  b.ctiles = (int)((O + MM8R_COLS - 1) / MM8R_COLS);
+  b.cw = 2 * (int)((KB + S - 1) / S);
+  char* wsb = static_cast<char*>(workspace);
+  b.xp = reinterpret_cast<_Float16*>(wsb);
+  b.rsum = reinterpret_cast<float*>(wsb + lay.rsum);
+  b.rscale = reinterpret_cast<float*>(wsb + lay.rscale);
+  b.part = S > 1 ? reinterpret_cast<float*>(wsb + lay.part) : nullptr;
+  const dim3 grid((unsigned)((rows + MM8R_ROWS - 1) / MM8R_ROWS * b.ctiles), (unsigned)nprob, (unsigned)S);
+  const auto go = [&](auto ta, auto tm) {
+    using TA = decltype(ta);
+    using TM = decltype(tm);
+    hipLaunchKernelGGL((mm8g_prep_kernel<TA, TM, true>), dim3((unsigned)rows, (unsigned)nprob), dim3(256), 0,
+                       as_stream(stream), b);
+    if (int rc = check_launch("mm8g_prep_kernel")) return rc;
+    static std::atomic<uint64_t> raised{0};  // devices whose dynamic LDS limit is raised for this instance
+    if (int rc = raise_dynamic_lds(reinterpret_cast<const void*>(&mm8r_kernel<TA, TM>), MM8R_NST * MM8R_STAGE, raised,
+                                   "mm8r_kernel"))
+      return rc;
+    hipLaunchKernelGGL((mm8r_kernel<TA, TM>), grid, dim3(512), MM8R_NST * MM8R_STAGE, as_stream(stream), b);
+    if (int rc = check_launch("mm8r_kernel")) return rc;
+    return S > 1 ? mm8g_reduce<TA, TM>(b, stream) : (int)RWKV7MI_OK;
+  };
+  return dispatch_dtype(meta_dtype, [&](auto tm) {
+    return act_dtype == RWKV7MI_BF16 ? go(__hip_bfloat16{}, tm) : go(__half{}, tm);
+  });
 }
 
 // ---- allocation-free form: the scratch lives in this file's device array

@@ -504,18 +504,18 @@ namespace rwkv7mi {
 // at 1000 rows, 64 tiles, 289 us for 256 steps; 4096 -> 16384, 256 tiles, 107
 // us for 64), and the fp32 partials (part_bytes a split) written and read back
 // at about 4 TB/s plus a launch.
-static int mh_splits(int64_t tiles, int64_t I, int64_t part_bytes) {
-  if (I % 64) return 1;
-  const int64_t SB = I / 64;
+static int mh_splits(int64_t tiles, int64_t I, int64_t part_bytes, double* us = nullptr) {
+  const int64_t SB = (I + 63) / 64;
   int best = 1;
   double cost = 1e30;
   for (int S = 1; S <= 16 && (S == 1 || tiles * S <= 256); ++S) {
     const int64_t sps = (SB + S - 1) / S;
-    if (S > 1 && (sps < 4 || (SB + sps - 1) / sps != S)) continue;  // no empty split
-    const double t = (sps + 6) * (1.1 + 0.56 * std::min<double>(1.0, tiles * S / 256.0)) +
+    if (S > 1 && (I % 64 || sps < 4 || (SB + sps - 1) / sps != S)) continue;  // no empty split
+    const double t = (tiles * S + 255) / 256 * (sps + 6) * (1.1 + 0.56 * std::min<double>(1.0, tiles * S / 256.0)) +
                      (S > 1 ? 5.0 + 2.0 * part_bytes * S / 4e6 : 0.0);
     if (t < cost) cost = t, best = S;
   }
+  if (us) *us = cost;
   return best;
 }
 static int64_t mh_tiles(int64_t nprob, int64_t rows, int64_t O) {
@@ -562,6 +562,12 @@ static int mh_gemm_launch(MhBatch& b, int nprob, int64_t rows, int64_t I, int64_
   if (b.S > 1) return launch(&mm8h_gemm_kernel<true, true, TA>, raised[0]);
   return I % 64 == 0 ? launch(&mm8h_gemm_kernel<true, false, TA>, raised[1])
                      : launch(&mm8h_gemm_kernel<false, false, TA>, raised[2]);
+}
+
+double mm8h_estimate_us(int64_t nprob, int64_t rows, int64_t I, int64_t O) {
+  double us = 0;
+  mh_splits(mh_tiles(nprob, rows, O), I, mh_part_bytes(nprob, rows, O), &us);
+  return us + 4.0 + 3.0 * nprob * I * O / 4.8e6;  // + the dequantisation
 }
 
 }  // namespace rwkv7mi

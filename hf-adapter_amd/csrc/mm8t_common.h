@@ -84,6 +84,10 @@ __device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t mask, uint32_t b
   return r;
 }
 
+// Estimated time (us) of the dequantise + 256 x 256 GEMM form (mm8h.hip), K
+// splits included, for the choice between it and the middle-row kernel.
+double mm8h_estimate_us(int64_t nprob, int64_t rows, int64_t I, int64_t O);
+
 // Compute units of the current device (cached per device).
 int64_t mm8t_cus();
 

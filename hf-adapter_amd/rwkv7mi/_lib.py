@@ -79,6 +79,9 @@ SIGNATURES = {
     "rwkv7mi_mm8t_gemm_multi_noalloc": (_i32, [_i32] + [_c_p] * 10 + [_i64, _i64, _i64, _i32, _i32, _i32, _c_p]),
     "rwkv7mi_mm8t_gemm_prefill": (_i32, [_i32] + [_c_p] * 10 + [_i64, _i64, _i64, _i32, _i32, _c_p]),
     "rwkv7mi_mm8t_gemm_prefill_ws": (_i32, [_i32] + [_c_p] * 10 + [_i64, _i64, _i64, _i32, _i32, _c_p, _i64, _c_p]),
+    "rwkv7mi_mm8t_rows_workspace_bytes": (_i64, [_i32, _i64, _i64, _i64]),
+    "rwkv7mi_mm8t_rows_pays": (_i32, [_i32, _i64, _i64, _i64, _i32]),
+    "rwkv7mi_mm8t_rows_multi": (_i32, [_i32] + [_c_p] * 10 + [_i64, _i64, _i64, _i32, _i32, _c_p, _i64, _c_p]),
     "rwkv7mi_mm8t_gemm_prefill_ws_bytes": (_i64, [_i32, _i64, _i64]),
     "rwkv7mi_mm8t_gemm_prefill_split_ws_bytes": (_i64, [_i32, _i64, _i64, _i64]),
     "rwkv7mi_dense_gemm_prefill_ws": (_i32, [_i32] + [_c_p] * 6 + [_i64, _i64, _i64, _i32, _c_p, _i64, _c_p]),

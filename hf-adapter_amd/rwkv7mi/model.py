@@ -37,10 +37,9 @@ from .native_wkv_fp16 import (native_fp16_recurrent_output_prepare_raw, native_f
                               native_fp16_sequence)
 from .fused_time_mix import fused_attn_sequence_shift_mix, fused_ffn_sequence_shift_mix
 from .sampling import argmax_rows, argmax_workspace_bytes
-from .native_quant_mm8 import (GEMM_ROWS, GEMV_ROWS, MM8Linear, is_blocked, mm8_gemm_multi_into, mm8_gemm_prefill_multi_into,
-                               mm8_gemm_workspace_bytes, mm8_prefill_workspace_bytes, mm8_lnmix_multi_into, mm8_matmul_multi_into,
-                               mm8_matmul_multi_lora_into,
-                               mm8_matmul_partials, mm8t_workspace_bytes)
+from .native_quant_mm8 import (GEMM_ROWS, GEMV_ROWS, MM8Linear, is_blocked, mm8_gemm_workspace_bytes, mm8_lnmix_multi_into,
+                               mm8_many_rows_into, mm8_matmul_multi_into, mm8_matmul_multi_lora_into,
+                               mm8_matmul_partials, mm8_prefill_workspace_bytes, mm8_rows_reserve_bytes, mm8t_workspace_bytes)
 from .native_quant_policy import should_quantize_linear
 from .self_chunk_rwkv7 import _run_chunk, check_wkv7_chunk_status
 
@@ -271,7 +270,7 @@ class QuantLinear:
     """MM8 Linear, all on HIP kernels: the fused blocked dequant GEMV for up to
     ``GEMV_ROWS`` rows, the 64-row MFMA tile GEMM (split K) up to ``GEMM_ROWS``
     rows, and above that the prefill GEMM over the materialised fp16
-    dequantised weight (``mm8_gemm_prefill_multi_into``).  Modules whose bytes are not blocked
+    dequantised weight (``mm8_many_rows_into``).  Modules whose bytes are not blocked
     take MM8Linear's own route."""
 
     GEMV_ROWS = GEMV_ROWS
@@ -283,17 +282,11 @@ class QuantLinear:
 
     def apply(self, x2, out, *, act=ACT_NONE, residual=None):
         rows = int(x2.shape[0])
-        if self.GEMV_ROWS < rows <= self.GEMM_ROWS and is_blocked(self.m.w_blk):
-            epi = _lib.EPI_RELU2 if act == 3 else (_lib.EPI_RESIDUAL if residual is not None else _lib.EPI_NONE)
-            if act not in (0, 3) or (act == 3 and residual is not None):
-                raise ValueError("QuantLinear: unsupported activation / residual combination")
-            mm8_gemm_multi_into([x2], [self.m], [out], residuals=[residual], epilogues=[epi])
-            return out
         if act not in (0, 3) or (act == 3 and residual is not None):
             raise ValueError("QuantLinear: unsupported activation / residual combination")
         epi = _lib.EPI_RELU2 if act == 3 else (_lib.EPI_RESIDUAL if residual is not None else _lib.EPI_NONE)
-        if rows > self.GEMM_ROWS and is_blocked(self.m.w_blk):
-            mm8_gemm_prefill_multi_into([x2], [self.m], [out], residuals=[residual], epilogues=[epi])
+        if rows > self.GEMV_ROWS and is_blocked(self.m.w_blk):
+            mm8_many_rows_into([x2], [self.m], [out], residuals=[residual], epilogues=[epi])
             return out
         return self.m._run(x2, out=out, residual=residual, epilogue=epi)
 
@@ -307,10 +300,8 @@ class QuantLinear:
                 and all(is_blocked(l.m.w_blk) for l in lins)):
             if rows <= QuantLinear.GEMV_ROWS:
                 mm8_matmul_multi_into(list(xs), [l.m for l in lins], list(outs))
-            elif rows <= QuantLinear.GEMM_ROWS:
-                mm8_gemm_multi_into(list(xs), [l.m for l in lins], list(outs))
             else:
-                mm8_gemm_prefill_multi_into(list(xs), [l.m for l in lins], list(outs))
+                mm8_many_rows_into(list(xs), [l.m for l in lins], list(outs))
             return outs
         if all(isinstance(l, DenseLinear) for l in lins) and DenseLinear.apply_group(lins, xs, outs):
             return outs
@@ -1059,6 +1050,13 @@ class NativeRWKV7ForCausalLM(_PreTrainedModel, _GenerationMixin):
                     gneed = max(gneed, mm8_gemm_workspace_bytes(1, rows, lin.in_features, lin.out_features))
             if gneed:
                 _ws.reserve(self.device, gneed, slot="mm8g")
+        rneed = 0  # the middle-row products
+        for lins in [(L.r_proj, L.k_proj, L.v_proj) for L in self.layers] + [(lin,) for lin in self._linears()]:
+            if all(isinstance(lin, QuantLinear) for lin in lins):
+                rneed = max(rneed, mm8_rows_reserve_bytes(len(lins), rows, lins[0].in_features, lins[0].out_features,
+                                                          self.dtype))
+        if rneed:
+            _ws.reserve(self.device, rneed, slot="mm8r")
         if rows > QuantLinear.GEMM_ROWS:  # prefill: the fp16 dequantised weights of the widest launch
             pneed = 0
             for L in self.layers:

@@ -158,7 +158,8 @@ def _check_out(x2, m, out, residual):
 
 
 # Blocked-weight routes by row count: the fused GEMV up to GEMV_ROWS rows, the
-# 64-row MFMA tile GEMM up to GEMM_ROWS, the 256 x 256 prefill GEMM above.
+# 64-row MFMA tile GEMM up to GEMM_ROWS, the 256 x 256 prefill GEMM above; in the
+# middle (65 to about 1000 rows) the 128 x 256 tile kernel where it is faster.
 GEMV_ROWS = 16
 GEMM_ROWS = 256
 
@@ -183,10 +184,8 @@ def mm8_matmul_into(x2, w_u8, mx, rx, my, ry, out, *, bias=None, residual=None, 
             raise ValueError(f"mm8: blocked weights {tuple(w_u8.shape)} do not match [{n}, {m}]")
         residual = _check_out(x2, m, out, residual)
         mod = types.SimpleNamespace(w_blk=w_u8, mx=mx, rx=rx, my=my, ry=ry, bias=bias, in_features=n, out_features=m)
-        if rows > GEMM_ROWS:
-            mm8_gemm_prefill_multi_into([x2], [mod], [out], residuals=[residual], epilogues=[epilogue])
-        elif rows > GEMV_ROWS:
-            mm8_gemm_multi_into([x2], [mod], [out], residuals=[residual], epilogues=[epilogue])
+        if rows > GEMV_ROWS:
+            mm8_many_rows_into([x2], [mod], [out], residuals=[residual], epilogues=[epilogue])
         else:
             mm8_matmul_multi_into([x2], [mod], [out], residuals=[residual], epilogues=[epilogue])
         return out
@@ -357,6 +356,68 @@ def mm8_gemm_multi_into(xs, mods, outs, *, residuals=None, epilogues=None, split
         _lib.stream_of(xs[0]),
     )
     return outs
+
+
+def mm8_rows_workspace_bytes(nprob: int, rows: int, n: int, m: int) -> int:
+    """Scratch bytes of :func:`mm8_rows_multi_into` (the ``"mm8r"`` slot)."""
+    return int(_lib.load().rwkv7mi_mm8t_rows_workspace_bytes(int(nprob), int(rows), int(n), int(m)))
+
+
+_DTYPE_CODES = {torch.float32: _lib.F32, torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}
+
+
+def mm8_rows_reserve_bytes(nprob: int, rows: int, n: int, m: int, dtype: torch.dtype) -> int:
+    """What :func:`mm8_many_rows_into` takes of the ``"mm8r"`` slot (0 when it runs another form)."""
+    if not _lib.load().rwkv7mi_mm8t_rows_pays(int(nprob), int(rows), int(n), int(m), _DTYPE_CODES[dtype]):
+        return 0
+    return mm8_rows_workspace_bytes(nprob, rows, n, m)
+
+
+def mm8_rows_multi_into(xs, mods, outs, *, residuals=None, epilogues=None) -> bool:
+    """:func:`mm8_gemm_multi_into` for middle row counts (fp16 / bf16): the
+    128-row x 256-column tile kernel.  False, with nothing run, when a graph is
+    being captured and the ``"mm8r"`` slot is smaller than the call needs, or an
+    operand is not 16-byte aligned."""
+    k = len(mods)
+    rows, n = (int(s) for s in xs[0].shape)
+    m = int(mods[0].out_features)
+    residuals = list(residuals) if residuals is not None else [None] * k
+    epilogues = list(epilogues) if epilogues is not None else [_lib.EPI_NONE] * k
+    for x2, mod, out, r in zip(xs, mods, outs, residuals):
+        if tuple(x2.shape) != (rows, n) or not x2.is_contiguous() or x2.dtype != xs[0].dtype:
+            raise ValueError("mm8_rows_multi_into: inputs must share one contiguous shape and dtype")
+        if mod.in_features != n or mod.out_features != m or not is_blocked(mod.w_blk):
+            raise ValueError("mm8_rows_multi_into: modules must be blocked MM8Linear of one shape")
+        _check_out(x2, m, out, r)
+    _lib.require_gpu(*xs, *outs, name="mm8_rows_multi")
+    if any(t.data_ptr() % 16 for t in (*xs, *(t for md in mods for t in (md.w_blk, md.my, md.ry)))):
+        return False
+    need = mm8_rows_workspace_bytes(k, rows, n, m)
+    ws = _ws.reserve(xs[0].device, need, slot="mm8r", floor=0)
+    if ws is None or int(ws.numel()) < need:
+        return False
+    arr = _lib.ptr_array
+    eps = (ctypes.c_int * k)(*[int(e) for e in epilogues])
+    _lib.call(
+        "rwkv7mi_mm8t_rows_multi", k, arr(xs), arr([md.w_blk for md in mods]), arr([md.mx for md in mods]),
+        arr([md.rx for md in mods]), arr([md.my for md in mods]), arr([md.ry for md in mods]),
+        arr([md.bias for md in mods]), arr(residuals), arr(outs), eps, rows, n, m, _lib.dtype_code(xs[0]),
+        _lib.dtype_code(mods[0].mx), _lib.ptr(ws), need, _lib.stream_of(xs[0]),
+    )
+    return True
+
+
+def mm8_many_rows_into(xs, mods, outs, *, residuals=None, epilogues=None):
+    """More than ``GEMV_ROWS`` rows of up to four blocked products of one shape
+    on the kernel for their row count."""
+    rows, n = (int(s) for s in xs[0].shape)
+    kw = {"residuals": residuals, "epilogues": epilogues}
+    if (_lib.load().rwkv7mi_mm8t_rows_pays(len(mods), rows, n, int(mods[0].out_features), _lib.dtype_code(xs[0]))
+            and mm8_rows_multi_into(xs, mods, outs, **kw)):
+        return outs
+    if rows > GEMM_ROWS:
+        return mm8_gemm_prefill_multi_into(xs, mods, outs, **kw)
+    return mm8_gemm_multi_into(xs, mods, outs, **kw)
 
 
 # x's buffer descriptor in the prefill GEMM spans rows * in_features * 2 bytes,
@@ -734,7 +795,7 @@ def invalidate_model_caches(model) -> None:
             runners.clear()
 
 
-__all__ = ["mm8_gemm_prefill_multi_into", "mm8_block_shape",
+__all__ = ["mm8_gemm_prefill_multi_into", "mm8_rows_multi_into", "mm8_many_rows_into", "mm8_block_shape",
     "quantize_mm8", "dequantize_mm8", "quantize_mm8_outmajor", "quantize_mm8_blocked", "mm8_block", "mm8_unblock", "is_blocked",
     "is_out_major", "mm8_matmul", "mm8_linear", "mm8_matmul_into",
     "mm8_matmul_multi_into", "mm8_gemm_multi_into", "mm8_gemm_workspace_bytes", "mm8_gemv_triton",

@@ -5,7 +5,7 @@ completion counters; the kernel leaves its counters at zero after every call,
 so one zero-initialised buffer per device can be reused by every call issued
 on one stream.  Slot ``"mm8t"`` holds the blocked GEMV's split-K partials
 (written before they are read).  Slot ``"mm8g"`` holds the many-row MM8 GEMM's x', row sums and
-split partials (each call writes them before reading).  Slot ``"lora"`` holds
+split partials, slot ``"mm8r"`` those of the middle-row form (each call writes them before reading).  Slot ``"lora"`` holds
 the LoRA kernels' fp32 partials.  Slot ``"mm8p"`` holds the prefill GEMM's
 fp16 dequantised weights and split partials, slot ``"w4"`` the many-row W4
 product's split partials (each call writes them before reading).  Slots never share memory, so one kernel

@@ -464,6 +464,22 @@ int rwkv7mi_dense_gemm_prefill_ws(int nprob, const void* const* x,
                                   int64_t O, int act_dtype, void* ws,
                                   int64_t ws_bytes, void* stream);
 
+/* rwkv7mi_mm8t_gemm_multi (same arguments and results to rounding) for middle
+ * row counts, fp16 / bf16 activations: 64-row x 256-column tiles, K split only
+ * where they do not fill the chip.  The workspace (256-byte aligned) holds
+ * rwkv7mi_mm8t_rows_workspace_bytes. */
+int64_t rwkv7mi_mm8t_rows_workspace_bytes(int nprob, int64_t rows, int64_t I, int64_t O);
+/* 1 where it is the fastest form for this many rows, else 0. */
+int rwkv7mi_mm8t_rows_pays(int nprob, int64_t rows, int64_t I, int64_t O, int act_dtype);
+int rwkv7mi_mm8t_rows_multi(int nprob, const void* const* x,
+                            const uint8_t* const* w_blk, const void* const* mx,
+                            const void* const* rx, const void* const* my,
+                            const void* const* ry, const void* const* bias,
+                            const void* const* residual, void* const* y,
+                            const int* epilogue, int64_t rows, int64_t I,
+                            int64_t O, int act_dtype, int meta_dtype,
+                            void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Allocation-free form of rwkv7mi_mm8t_gemm_multi (same arguments and results,
  * no workspace argument).  No counterpart in the reference: it is for callers
  * that cannot allocate (code under hipGraph capture, tight serving loops,

@@ -193,3 +193,86 @@ def test_mm8g_workspace_contract():
     with pytest.raises(ValueError, match="1024 inputs"):
         _lib.call("rwkv7mi_mm8t_gemm_multi", *args[:-1], 1, None, 0, _lib.stream_of(x))
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("act,meta", [(torch.float16, torch.float16), (torch.bfloat16, torch.bfloat16),
+                                      (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("IO,rows,epi", [((4096, 264), 65, 0), ((144, 40), 129, 1), ((2064, 520), 300, 2),
+                                         ((1024, 65), 257, 0), ((16384, 272), 200, 2), ((256, 1040), 1030, 1)])
+def test_mm8_rows_matches_oracle(oracle, IO, rows, epi, act, meta):
+    """The middle-row form at the edges of its tiles (rows past 128, column
+    groups past 256, K that ends inside a block, one and several K splits),
+    two problems, every epilogue and an output that is its own residual."""
+    from rwkv7mi.native_quant_mm8 import mm8_rows_multi_into
+
+    I, O = IO
+    rng = np.random.default_rng(I + O + rows)
+    mods = [_packed(rng, I, O, meta, bias=True) for _ in range(2)]
+    xs = [_cuda(rng.standard_normal((rows, I)), act) for _ in range(2)]
+    res = [_cuda(rng.standard_normal((rows, O)), act) for _ in range(2)]
+    outs = [r.clone() if epi == 2 else torch.full((rows, O), float("nan"), device="cuda", dtype=act) for r in res]
+    assert mm8_rows_multi_into(xs, mods, outs, residuals=outs if epi == 2 else None, epilogues=[epi] * 2)
+    torch.cuda.synchronize()
+    for x, mod, r, y in zip(xs, mods, res, outs):
+        ref = _ref(oracle, x, mod)
+        ref = np.maximum(ref, 0.0) ** 2 if epi == 1 else ref + _np(r.float()) if epi == 2 else ref
+        # the rounding of x' (2^-11 of each term) and of the output
+        tol = 2e-3 if act == torch.float16 else 6e-3
+        assert _rel_err(_np(y.float()).astype(np.float64), ref) <= tol
+
+
+@pytest.mark.parametrize("scale", [1e-6, 1.0, 3e4])
+def test_mm8_rows_keeps_row_magnitudes(oracle, scale):
+    """x' is scaled per row: rows far below fp16's normal range and rows that
+    would overflow it as x ry keep the relative error of ordinary rows."""
+    from rwkv7mi.native_quant_mm8 import mm8_rows_multi_into
+
+    I, O, rows = 1024, 256, 140
+    rng = np.random.default_rng(5)
+    mod = _packed(rng, I, O, torch.bfloat16)
+    x = _cuda(rng.standard_normal((rows, I)) * scale * 10.0 ** rng.integers(-3, 4, (rows, 1)), torch.bfloat16)
+    y = torch.empty((rows, O), device="cuda", dtype=torch.bfloat16)
+    assert mm8_rows_multi_into([x], [mod], [y])
+    torch.cuda.synchronize()
+    ref = _ref(oracle, x, mod)
+    got = _np(y.float()).astype(np.float64)
+    err = np.linalg.norm(got - ref, axis=1) / np.linalg.norm(ref, axis=1)
+    assert err.max() <= 4e-3, err.max()  # bf16 output rounding 2^-9 rms and x' 2^-12
+
+
+def test_mm8_rows_route_and_capture(oracle):
+    """mm8_matmul takes the form where it pays; a graph captured with no room
+    for its workspace runs the previous form and replays to the same result."""
+    from rwkv7mi import _lib
+    from rwkv7mi import workspace as _ws
+    from rwkv7mi.native_quant_mm8 import mm8_many_rows_into, mm8_rows_multi_into
+
+    lib = _lib.load()
+    pays = lambda rows, I, O: bool(lib.rwkv7mi_mm8t_rows_pays(1, rows, I, O, _lib.F16))
+    assert pays(100, 4096, 16384) and not pays(64, 4096, 16384) and not pays(100, 2048, 8192)
+    assert pays(300, 2048, 8192) and not pays(8000, 4096, 16384)
+    I, O, rows = 2048, 8192, 300
+    rng = np.random.default_rng(1)
+    mod = _packed(rng, I, O)
+    x = _cuda(rng.standard_normal((rows, I)), torch.float16)
+    y, want = (torch.empty((rows, O), device="cuda", dtype=torch.float16) for _ in range(2))
+    mm8_many_rows_into([x], [mod], [y])
+    assert mm8_rows_multi_into([x], [mod], [want])
+    torch.cuda.synchronize()
+    assert torch.equal(y, want)
+    key = (torch.cuda.current_device(), "mm8r")
+    kept = _ws._buffers.pop(key)
+    try:
+        from rwkv7mi.native_quant_mm8 import mm8_gemm_prefill_multi_into
+
+        mm8_gemm_prefill_multi_into([x], [mod], [want])
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            mm8_many_rows_into([x], [mod], [y])
+        for _ in range(3):
+            y.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, want)
+    finally:
+        _ws._buffers[key] = kept
