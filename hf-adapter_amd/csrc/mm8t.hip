@@ -1326,3 +1326,45 @@ extern "C" int rwkv7mi_mm8t_dequant(const uint8_t* w_blk, const void* mx, const 
   });
 }
 
+// ---- one product on the form for its row count, for callers whose own work per
+// call would outlast the launch
+extern "C" int rwkv7mi_mm8t_linear_plan(int64_t rows, int64_t I, int64_t O, int act_dtype, int64_t* ws_bytes) {
+  *ws_bytes = 0;
+  if (rows <= 0 || I <= 0 || O <= 0) return 0;
+  if (rows <= 16) {
+    *ws_bytes = (int64_t)rwkv7mi_mm8t_matmul_workspace_bytes(1, rows, I, O);
+    return 0;
+  }
+  if (rwkv7mi_mm8t_rows_pays(1, rows, I, O, act_dtype)) {
+    *ws_bytes = rwkv7mi_mm8t_rows_workspace_bytes(1, rows, I, O);
+    return 2;
+  }
+  if (rows <= 256) {
+    *ws_bytes = (int64_t)rwkv7mi_mm8t_gemm_workspace_bytes(1, rows, I, O, 0);
+    return 1;
+  }
+  *ws_bytes = rwkv7mi_mm8t_gemm_prefill_split_ws_bytes(1, rows, I, O);
+  return 3;
+}
+
+extern "C" int rwkv7mi_mm8t_linear(int form, const void* x, const uint8_t* w, const void* mx, const void* rx,
+                                   const void* my, const void* ry, const void* bias, const void* residual, void* y,
+                                   int epilogue, int64_t rows, int64_t I, int64_t O, int act_dtype, int meta_dtype,
+                                   void* ws, int64_t ws_bytes, void* stream) {
+  switch (form) {
+    case 0:
+      return rwkv7mi_mm8t_matmul_multi_ws(1, &x, &w, &mx, &rx, &my, &ry, &bias, &residual, &y, &epilogue, rows, I, O,
+                                          act_dtype, meta_dtype, ws, (size_t)ws_bytes, stream);
+    case 1:
+      return rwkv7mi_mm8t_gemm_multi(1, &x, &w, &mx, &rx, &my, &ry, &bias, &residual, &y, &epilogue, rows, I, O,
+                                     act_dtype, meta_dtype, 0, ws, (size_t)ws_bytes, stream);
+    case 2:
+      return rwkv7mi_mm8t_rows_multi(1, &x, &w, &mx, &rx, &my, &ry, &bias, &residual, &y, &epilogue, rows, I, O,
+                                     act_dtype, meta_dtype, ws, ws_bytes, stream);
+    case 3:
+      return rwkv7mi_mm8t_gemm_prefill_ws(1, &x, &w, &mx, &rx, &my, &ry, &bias, &residual, &y, &epilogue, rows, I, O,
+                                          act_dtype, meta_dtype, ws, ws_bytes, stream);
+    default:
+      return fail(RWKV7MI_EINVAL, "mm8t_linear: form 0..3");
+  }
+}

@@ -80,6 +80,8 @@ SIGNATURES = {
     "rwkv7mi_mm8t_gemm_prefill": (_i32, [_i32] + [_c_p] * 10 + [_i64, _i64, _i64, _i32, _i32, _c_p]),
     "rwkv7mi_mm8t_gemm_prefill_ws": (_i32, [_i32] + [_c_p] * 10 + [_i64, _i64, _i64, _i32, _i32, _c_p, _i64, _c_p]),
     "rwkv7mi_mm8t_rows_workspace_bytes": (_i64, [_i32, _i64, _i64, _i64]),
+    "rwkv7mi_mm8t_linear_plan": (_i32, [_i64, _i64, _i64, _i32, ctypes.POINTER(_i64)]),
+    "rwkv7mi_mm8t_linear": (_i32, [_i32] + [_c_p] * 9 + [_i32, _i64, _i64, _i64, _i32, _i32, _c_p, _i64, _c_p]),
     "rwkv7mi_mm8t_rows_pays": (_i32, [_i32, _i64, _i64, _i64, _i32]),
     "rwkv7mi_mm8t_rows_multi": (_i32, [_i32] + [_c_p] * 10 + [_i64, _i64, _i64, _i32, _i32, _c_p, _i64, _c_p]),
     "rwkv7mi_mm8t_gemm_prefill_ws_bytes": (_i64, [_i32, _i64, _i64]),
@@ -173,9 +175,8 @@ def declared_symbols(header: Path) -> list[str]:
 
 
 def call(name: str, *args):
-    lib = load()
-    fn = getattr(lib, name)
-    rc = fn(*args)
+    lib = _lib if _lib is not None else load()
+    rc = getattr(lib, name)(*args)
     if rc != 0:
         msg = lib.rwkv7mi_last_error().decode(errors="replace")
         if rc == -1:
@@ -185,7 +186,7 @@ def call(name: str, *args):
 
 def ptr_array(tensors) -> ctypes.Array:
     """A C array of device pointers (NULL for None)."""
-    return (ctypes.c_void_p * len(tensors))(*[None if t is None else t.data_ptr() for t in tensors])
+    return (_c_p * len(tensors))(*[None if t is None else t.data_ptr() for t in tensors])
 
 
 def dtype_code(t: torch.Tensor) -> int:
@@ -196,11 +197,16 @@ def dtype_code(t: torch.Tensor) -> int:
 
 
 def ptr(t: torch.Tensor | None):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """The tensor's address for a ``void*`` argument (None: NULL)."""
+    return None if t is None else t.data_ptr()
 
 
 def stream_of(t: torch.Tensor):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    """The current stream of t's device for a ``void*`` argument (the raw query:
+    a ``torch.cuda.Stream`` object for each launch costs more than the launch)."""
+    if not t.is_cuda:
+        raise ValueError(f"rwkv7mi: expected a cuda tensor, got one on {t.device}")
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def require_gpu(*tensors: torch.Tensor | None, name: str) -> None:
@@ -210,7 +216,8 @@ def require_gpu(*tensors: torch.Tensor | None, name: str) -> None:
                 f"{name}: rwkv7mi runs on the GPU only; got a {t.device} tensor "
                 "(there is no CPU fallback)"
             )
-    load()
+    if _lib is None:
+        load()
 
 
 __all__ = [

@@ -11,6 +11,7 @@ tensors: there is no CPU path.
 from __future__ import annotations
 
 import ctypes
+import functools
 import types
 
 import torch
@@ -420,6 +421,50 @@ def mm8_many_rows_into(xs, mods, outs, *, residuals=None, epilogues=None):
     return mm8_gemm_multi_into(xs, mods, outs, **kw)
 
 
+_FORM_SLOT = ("mm8t", "mm8g", "mm8r", "mm8p")
+
+
+@functools.lru_cache(maxsize=4096)
+def _linear_plan(rows: int, n: int, m: int, dt: int, device: int):
+    """(form, workspace bytes, least workspace) of one product: the sizes and
+    the device's CU count alone decide."""
+    need = ctypes.c_int64(0)
+    form = int(_lib.load().rwkv7mi_mm8t_linear_plan(rows, n, m, dt, ctypes.byref(need)))
+    floor = mm8_prefill_workspace_bytes(1, n, m) if form == 3 else int(need.value)
+    return form, int(need.value), floor
+
+
+def _linear_into(x2, w, mx, rx, my, ry, bias, residual, out, epilogue) -> bool:
+    """One blocked product in one library call (``x2 [rows, n]`` and ``out``
+    contiguous and checked by the caller).  False, with nothing run, for the
+    calls that need the general route: mixed prefill dtypes or row chunks, an
+    unaligned operand of the middle-row form, no room under graph capture.
+    The general route's lists, pointer arrays and size queries cost more host
+    time than a small product's kernel runs: the 4096 -> 16384 -> 4096 FFN pair
+    took 49.4 us at 1 row with it and takes 30.2 us (31 us of kernels) on this
+    one, 58.3 -> 46.6 us at 16 rows, 63.4 -> 57.6 us at 200."""
+    rows, n = x2.shape
+    m = out.shape[1]
+    dt = _lib.dtype_code(x2)
+    form, need, floor = _linear_plan(rows, n, m, dt, x2.get_device())
+    if form >= 2:
+        if form == 3 and (dt == _lib.F32 or mx.dtype != x2.dtype or rows * n * 2 > _PREFILL_MAX_BYTES):
+            return False
+        if form == 2 and (x2.data_ptr() | w.data_ptr() | my.data_ptr() | ry.data_ptr()) & 15:
+            return False
+    ws, have = None, 0
+    if need:
+        ws = _ws.reserve(x2.device, need, _FORM_SLOT[form], floor=0 if form == 2 else floor)
+        have = 0 if ws is None else ws.numel()
+        if have < floor:
+            return False
+        ws = ws.data_ptr()
+    _lib.call("rwkv7mi_mm8t_linear", form, x2.data_ptr(), w.data_ptr(), mx.data_ptr(), rx.data_ptr(), my.data_ptr(),
+              ry.data_ptr(), _lib.ptr(bias), _lib.ptr(residual), out.data_ptr(), epilogue, rows, n, m, dt,
+              _lib.dtype_code(mx), ws, min(have, need) if form == 3 else have, _lib.stream_of(x2))
+    return True
+
+
 # x's buffer descriptor in the prefill GEMM spans rows * in_features * 2 bytes,
 # below 2^31: longer inputs are split into row chunks
 _PREFILL_MAX_BYTES = (1 << 31) - 1
@@ -690,18 +735,30 @@ class MM8Linear(torch.nn.Module):
             module.w_blk.copy_(mm8_block(w.to(module.w_blk.device)))
 
     def _run(self, x, out=None, residual=None, epilogue=_lib.EPI_NONE):
-        lead = x.shape[:-1]
-        x2 = x.reshape(-1, self.in_features)
+        n, m = self.in_features, self.out_features
+        flat = x.dim() == 2 and x.shape[1] == n
+        x2 = x if flat else x.reshape(-1, n)
         if not x2.is_contiguous():
             x2 = x2.contiguous()
-        rows = int(x2.shape[0])
-        if out is None:
-            out2 = torch.empty((rows, self.out_features), device=x.device, dtype=x.dtype)
-        else:
-            out2 = out.reshape(rows, self.out_features)
-        mm8_matmul_into(x2, self.w_blk, self.mx, self.rx, self.my.reshape(-1), self.ry.reshape(-1), out2,
-                        bias=self.bias, residual=residual, epilogue=epilogue)
-        return out2.reshape(*lead, self.out_features) if out is None else out
+        rows = x2.shape[0]
+        out2 = torch.empty((rows, m), device=x.device, dtype=x.dtype) if out is None else out.reshape(rows, m)
+        bufs = self._buffers
+        w, mx, rx, my, ry = bufs["w_blk"], bufs["mx"], bufs["rx"], bufs["my"], bufs["ry"]
+        bias = self.bias
+        blocked = (rows > 0 and is_blocked(w) and w.shape[0] == (m + 15) // 16 and w.shape[1] == (n + 127) // 128
+                   and ry.numel() == n and mx.numel() == m)
+        if blocked:
+            res = residual
+            if out is not None or residual is not None:
+                res = _check_out(x2, m, out2, residual)
+            _lib.require_gpu(x2, w, out2, name="mm8_matmul")
+            blocked = _linear_into(x2, w, mx, rx, my, ry, bias, res, out2, epilogue)
+        if not blocked:
+            mm8_matmul_into(x2, w, mx, rx, my.reshape(-1), ry.reshape(-1), out2, bias=bias, residual=residual,
+                            epilogue=epilogue)
+        if out is not None:
+            return out
+        return out2 if flat else out2.reshape(*x.shape[:-1], m)
 
     def forward(self, x):
         return self._run(x)

@@ -47,7 +47,10 @@ def reserve(device: torch.device, nbytes: int, slot: str = "mm8", *, floor: int 
     ``floor``: the least the call can run with.  Under graph capture a buffer
     of at least ``floor`` bytes (with 0 also no buffer: None) is returned as it
     is instead of raising."""
-    key = _key(device, slot)
+    key = (device.index, slot) if type(device) is torch.device and device.index is not None else _key(device, slot)
+    buf = _buffers.get(key)
+    if buf is not None and buf.numel() >= nbytes:
+        return buf
     with _lock:
         buf = _buffers.get(key)
         if buf is None or buf.numel() < nbytes:

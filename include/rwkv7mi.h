@@ -464,6 +464,18 @@ int rwkv7mi_dense_gemm_prefill_ws(int nprob, const void* const* x,
                                   int64_t O, int act_dtype, void* ws,
                                   int64_t ws_bytes, void* stream);
 
+/* One blocked product on the form for its row count.  The plan returns that
+ * form (0 rwkv7mi_mm8t_matmul_multi_ws, 1 rwkv7mi_mm8t_gemm_multi, 2
+ * rwkv7mi_mm8t_rows_multi, 3 rwkv7mi_mm8t_gemm_prefill_ws) and the workspace it
+ * uses; the call runs that entry on one problem, with its checks. */
+int rwkv7mi_mm8t_linear_plan(int64_t rows, int64_t I, int64_t O, int act_dtype, int64_t* ws_bytes);
+int rwkv7mi_mm8t_linear(int form, const void* x, const uint8_t* w_blk,
+                        const void* mx, const void* rx, const void* my,
+                        const void* ry, const void* bias, const void* residual,
+                        void* y, int epilogue, int64_t rows, int64_t I,
+                        int64_t O, int act_dtype, int meta_dtype, void* ws,
+                        int64_t ws_bytes, void* stream);
+
 /* rwkv7mi_mm8t_gemm_multi (same arguments and results to rounding) for middle
  * row counts, fp16 / bf16 activations: 64-row x 256-column tiles, K split only
  * where they do not fill the chip.  The workspace (256-byte aligned) holds

@@ -276,3 +276,36 @@ def test_mm8_rows_route_and_capture(oracle):
             assert torch.equal(y, want)
     finally:
         _ws._buffers[key] = kept
+
+
+@pytest.mark.parametrize("act,meta", [(torch.float16, torch.float16), (torch.bfloat16, torch.float16),
+                                      (torch.float32, torch.float32)])
+@pytest.mark.parametrize("IO", [(144, 72), (2048, 8192)])
+def test_mm8_linear_takes_the_general_routes_kernels(IO, act, meta):
+    """A module's one-call route gives the bits of the general route at the
+    edges of every form, for every shape of x, with and without a residual."""
+    from rwkv7mi.native_quant_mm8 import MM8Linear, mm8_matmul_into
+
+    I, O = IO
+    rng = np.random.default_rng(I)
+    p = _packed(rng, I, O, meta, bias=True)
+    mod = MM8Linear.from_packed(p.w_blk, p.mx, p.rx, p.my.reshape(-1, 1), p.ry.reshape(-1, 1), I, O, p.bias)
+    for rows in (1, 2, 16, 17, 64, 65, 256, 257, 300, 1100):
+        base = _cuda(rng.standard_normal((rows + 1, I)), act)
+        res = _cuda(rng.standard_normal((rows, O)), act)
+        for x in (base[:rows], base[1:], base[:rows].reshape(1, rows, I), base[:rows].t().contiguous().t()):
+            for r in (None, res):
+                want = torch.empty((rows, O), device="cuda", dtype=act)
+                mm8_matmul_into(x.reshape(rows, I).contiguous(), mod.w_blk, mod.mx, mod.rx, mod.my.reshape(-1),
+                                mod.ry.reshape(-1), want, bias=mod.bias, residual=r, epilogue=0 if r is None else 2)
+                got = mod(x) if r is None else mod.rwkv7_forward_add(x, r)
+                into = torch.empty_like(want)
+                if r is None:
+                    mod.rwkv7_forward_into(x, into)
+                    assert torch.equal(into, want)
+                assert got.shape == (*x.shape[:-1], O) and torch.equal(got.reshape(rows, O), want), (rows, x.shape)
+    assert mod(base[0]).shape == (O,)
+    with pytest.raises((ValueError, RuntimeError)):
+        mod(base[:2, : I // 2].contiguous())
+    with pytest.raises(ValueError):
+        mod.rwkv7_forward_into(base[:4], torch.empty((4, O), device="cuda", dtype=torch.float64))
