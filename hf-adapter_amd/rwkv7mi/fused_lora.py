@@ -45,19 +45,21 @@ def lora_multi(xs, downs, ups, biases, outs, acts_down, acts_up):
 
     Two launches for up to four projections: up to 64 rows a split-K down
     kernel and an up kernel that reduces the fp32 partials, above (fp16, bf16)
-    a down and an up kernel over all rows; the partials or the intermediate
-    live in the per-device workspace.  The largest fp16 prefills, fp32 and
-    ranks above 128 run in one launch above 256 rows.
+    a down and an up kernel over all rows.  The partials of up to 64 rows live
+    in the per-device workspace, the scratch of more rows is this call's own (so
+    calls on several streams do not share it).  The largest fp16 prefills, fp32
+    and ranks above 128 run in one launch above 256 rows.
     """
     k = len(xs)
     rows, D = (int(s) for s in xs[0].shape)
     A = int(ups[0].shape[0])
     ranks = [int(d.shape[0]) for d in downs]
     _lib.require_gpu(*xs, *downs, *ups, *outs, name="lora_multi")
-    # more rows than the split-K pair takes also run in its smaller workspace (on
-    # the one-launch kernel), which is what a graph captured without a reserve has
-    ws = _ws.reserve(xs[0].device, lora_workspace_bytes(ranks, rows, D), slot="lora",
-                     floor=lora_workspace_bytes(ranks, min(rows, 64), D))
+    need = lora_workspace_bytes(ranks, rows, D)
+    if rows > 64:
+        ws = torch.empty(need, dtype=torch.uint8, device=xs[0].device)
+    else:
+        ws = _ws.reserve(xs[0].device, need, slot="lora")
     _lib.call("rwkv7mi_lora_multi", k, _lib.ptr_array(xs), _lib.ptr_array(downs), _lib.ptr_array(ups),
               _lib.ptr_array(biases), _lib.ptr_array(outs), (ctypes.c_int64 * k)(*ranks),
               (ctypes.c_int * k)(*[int(a) for a in acts_down]), (ctypes.c_int * k)(*[int(a) for a in acts_up]),

@@ -1073,7 +1073,7 @@ class NativeRWKV7ForCausalLM(_PreTrainedModel, _GenerationMixin):
                 _ws.reserve(self.device, pneed, slot="mm8p")
         cfg = self.config
         ranks = [cfg.decay_low_rank_dim, cfg.a_low_rank_dim, cfg.gate_low_rank_dim, cfg.v_low_rank_dim]
-        _ws.reserve(self.device, lora_workspace_bytes(ranks, rows, cfg.hidden_size), slot="lora")
+        _ws.reserve(self.device, lora_workspace_bytes(ranks, min(rows, 64), cfg.hidden_size), slot="lora")
 
     def named_linears(self):
         """(HF module name, linear) for every projection and the head."""

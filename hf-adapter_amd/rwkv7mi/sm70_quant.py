@@ -11,7 +11,6 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from . import workspace as _ws
 
 
 def quantize_w4_groupwise(weight: torch.Tensor, group_size: int = 128):
@@ -37,15 +36,16 @@ def quantize_w4_groupwise(weight: torch.Tensor, group_size: int = 128):
 
 
 def _w4_call(x2, q, scales, biases, bias, residual, out2, rows, out_features, in_features, group_size, epilogue):
-    """The W4 product (``biases`` None: symmetric) over the ``"w4"`` slot's
-    workspace (many rows; a graph captured without one runs unsplit)."""
+    """The W4 product (``biases`` None: symmetric).  The K splits of many rows
+    keep their partials in a buffer of this call's own: calls on several streams
+    never share one."""
     dt = _lib.dtype_code(x2)
     need = int(_lib.load().rwkv7mi_w4_workspace_bytes(rows, out_features, in_features, group_size,
                                                       int(biases is not None), dt))
-    ws = _ws.reserve(x2.device, need, slot="w4", floor=0) if need else None
+    ws = torch.empty(need, dtype=torch.uint8, device=x2.device) if need else None
     _lib.call("rwkv7mi_w4_matmul_ws", _lib.ptr(x2), _lib.ptr(q), _lib.ptr(scales), _lib.ptr(biases), _lib.ptr(bias),
               _lib.ptr(residual), _lib.ptr(out2), rows, out_features, in_features, group_size, int(epilogue), dt,
-              _lib.dtype_code(scales), _lib.ptr(ws), 0 if ws is None else int(ws.numel()), _lib.stream_of(x2))
+              _lib.dtype_code(scales), _lib.ptr(ws), need, _lib.stream_of(x2))
 
 
 def w4_groupwise_linear_into(x2, q, scales, out2, *, group_size=128, bias=None, residual=None,
