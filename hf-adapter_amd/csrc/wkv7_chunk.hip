@@ -25,7 +25,8 @@
 // the raw pre-activation of the reference's clampw scan (2):
 // w = exp(-0.606531 sigmoid(w_raw)), so log2 w = -0.606531 log2(e) sigmoid(w_raw).
 //
-// Mapping: one workgroup of 8 waves per (batch, head), specialised:
+// Mapping (few heads over many chunks run as two kernels instead, see
+// SPLIT_HEADS): one workgroup of 8 waves per (batch, head), specialised:
 // * waves 0-3 ("chain") hold the fp32 state — wave q owns 16 value rows, as
 //   S^T tiles in MFMA accumulator layout — and per chunk run the products
 //   of U, Y and the state update (30 bf16x3 MFMAs per wave);
@@ -85,6 +86,32 @@ struct ChunkShared {
   float tcol[4][CH][CH];  // per producer: T column-major [s][t]
   int ready[NSLOT];
   int done[4][NSLOT];
+};
+
+// The two-kernel form: up to SPLIT_HEADS (batch, head) pairs and from SPLIT_MIN
+// chunks on.  One workgroup per pair leaves the rest of the chip idle there while
+// its four producer waves set the pace (1.07 us a chunk whatever the head count);
+// made by all CUs the operands cost one chunk's time for 2048 chunks and the
+// chain alone runs at 0.70 us a chunk.  fp16, one launch -> two, us:
+//   tokens      128          256          1000          4096
+//   12 heads    15.2 -> 15.2 23.8 -> 20.5 73.3 -> 55.4  278 -> 199
+//   32 heads    15.4 -> 15.7 24.0 -> 21.8 73.6 -> 59.2  279 -> 227
+//   64 heads    15.8 -> 16.7 24.5 -> 24.2 74.7 -> 67.8  281 -> 271
+//   96 heads                              74.8 -> 76.2  286 -> 341
+// Slots past SPLIT_BYTES are made and used in further launch pairs: with 48 MB
+// the 64 heads took 74.2 us at 1000 tokens and 302 at 4096.
+constexpr int64_t SPLIT_HEADS = 64;
+constexpr int64_t SPLIT_MIN = 16;
+constexpr int64_t SPLIT_BYTES = 192 << 20;
+
+// what a producer wave of the two-kernel form keeps in LDS; the slots are global
+struct SplitShared {
+  struct {
+    bf16x8 wa[2][2][64];
+    bf16x8 rq[2][2][64];
+  } park[4];
+  float nmat[4][CH][CH];
+  float tcol[4][CH][CH];
 };
 
 __device__ __forceinline__ float trunc_bf16(float x) {
@@ -211,14 +238,20 @@ __device__ __forceinline__ float row_val(const RawRow<T>& o, int jt, int e) {
 
 __device__ __forceinline__ float clamp126(float x) { return fminf(fmaxf(x, -126.f), 126.f); }
 
-template <typename TA, typename TW, int WMODE>
-__global__ __launch_bounds__(512, 1) void wkv7_chunk_kernel(
+template <typename TA, typename TW, int WMODE, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 256 : 512, SPLIT ? 2 : 1) void wkv7_chunk_kernel(
     const TA* __restrict__ r, const TW* __restrict__ w, const TA* __restrict__ k,
     const TA* __restrict__ v, const TA* __restrict__ kk, const TA* __restrict__ a,
-    const float* state_in, float* state_out, TA* __restrict__ y, int T, int H) {
+    const float* state_in, float* state_out, TA* __restrict__ y, int T, int H, ChunkSlot* __restrict__ slots,
+    int nbh, int x0, int xn) {
+  using Shared = std::conditional_t<SPLIT, SplitShared, ChunkShared>;
   extern __shared__ __align__(16) char smem_raw[];
-  ChunkShared& L = *reinterpret_cast<ChunkShared*>(smem_raw);
-  const int bh = blockIdx.x;
+  Shared& L = *reinterpret_cast<Shared*>(smem_raw);
+  // (SPLIT: eight workgroups a head group, so a head's slots are made on the XCD,
+  // blockIdx.x % 8, whose L2 its chain reads them from)
+  const int pad = (nbh + 7) & ~7;
+  const int bh = SPLIT ? (int)blockIdx.x % pad : (int)blockIdx.x;
+  if (SPLIT && bh >= nbh) return;
   const int b = bh / H;
   const int h = bh % H;
   const int tid = threadIdx.x;
@@ -229,6 +262,7 @@ __global__ __launch_bounds__(512, 1) void wkv7_chunk_kernel(
   const int nchunks = (T + CH - 1) / CH;
   const int64_t tok = (int64_t)H * HD;  // elements per token
 
+  if constexpr (!SPLIT) {  // (SPLIT makes operands only; its waves share nothing)
   if (tid < NSLOT) L.ready[tid] = -1;
   if (tid < 4 * NSLOT) L.done[tid / NSLOT][tid % NSLOT] = -1;
   __syncthreads();
@@ -323,9 +357,13 @@ __global__ __launch_bounds__(512, 1) void wkv7_chunk_kernel(
     post_status(status);
     return;
   }
+  }  // !SPLIT
 
   // ===================== producer wave p: chunks p, p+4, ...; lane = (token t = l16, kg)
-  const int p = wave - 4;
+  // (SPLIT: the four waves of a workgroup each make one chunk)
+  const int p = SPLIT ? wave : wave - 4;
+  const int xfirst = SPLIT ? x0 + 4 * ((int)blockIdx.x / pad) + p : p;
+  const int xend = SPLIT ? min(x0 + xn, xfirst + 1) : nchunks;
   // The producers bound the chunk rate (the chain waves wait for a ready slot
   // about half of the time), so where a producer and a chain wave can both
   // issue on a SIMD, the producer goes first.
@@ -355,11 +393,11 @@ __global__ __launch_bounds__(512, 1) void wkv7_chunk_kernel(
     load_row<TA>(ra, make_rsrc(a + base, nbA), offA);
     load_row<TW>(rw, make_rsrc(w + base, nbW), offW);
   };
-  if (p < nchunks) issue(p);
+  if (xfirst < xend) issue(xfirst);
 
   bool waited_out = false;
   float gmin = 0.f, gmax = 0.f;  // extremes of the chunk totals gC this lane saw
-  for (int x = p; x < nchunks; x += 4) {
+  for (int x = xfirst; x < xend; x += 4) {
     // A token past T loads w = 0 (log2 -> -inf, or 0 as a log) and must add
     // nothing to the gate sums: its floor is 0 instead of -126.
     const float lwlo = x * CH + t < T ? -126.f : 0.f;
@@ -367,8 +405,16 @@ __global__ __launch_bounds__(512, 1) void wkv7_chunk_kernel(
     // every result below is then stored as soon as it exists (D(ac) and rc are
     // parked in the Wa / Rq areas until Wa and Rq replace them).
     const int s = x % NSLOT;
-    for (int qq = 0; qq < 4; ++qq) waited_out |= !wait_geq(&L.done[qq][s], x - NSLOT);
-    ChunkSlot& Z = L.slot[s];
+    if constexpr (!SPLIT)
+      for (int qq = 0; qq < 4; ++qq) waited_out |= !wait_geq(&L.done[qq][s], x - NSLOT);
+    ChunkSlot& Z = [&]() -> ChunkSlot& {
+      if constexpr (SPLIT) return slots[(int64_t)bh * xn + (x - x0)];
+      else return L.slot[s];
+    }();
+    auto& P = [&]() -> auto& {  // where D(ac) and rc wait
+      if constexpr (SPLIT) return L.park[p];
+      else return L.slot[s];
+    }();
 
     // ---- per K half cc (channel tiles 2cc, 2cc+1): gates, gated rows, their
     // A-matrix products, and the transposed operands (identity MFMAs:
@@ -433,15 +479,15 @@ __global__ __launch_bounds__(512, 1) void wkv7_chunk_kernel(
         split_f4(ac, acH[jj], acL[jj]);
         split_f4(bc, bcH[jj], bcL[jj]);
         // transposed operands: D(ac) (parked in the Wa area), [D(bc) | D(kc)], D(v)
-        reinterpret_cast<bf16x4*>(&Z.wa[0][cc][lane])[jj] = pack_exact(mma16(acH[jj], Ib, ZERO4));
-        reinterpret_cast<bf16x4*>(&Z.wa[1][cc][lane])[jj] = pack_exact(mma16(acL[jj], Ib, ZERO4));
+        reinterpret_cast<bf16x4*>(&P.wa[0][cc][lane])[jj] = pack_exact(mma16(acH[jj], Ib, ZERO4));
+        reinterpret_cast<bf16x4*>(&P.wa[1][cc][lane])[jj] = pack_exact(mma16(acL[jj], Ib, ZERO4));
         Z.bk[0][jt][lane] = cat(pack_exact(mma16(bcH[jj], Ib, ZERO4)), pack_exact(mma16(kcH[jj], Ib, ZERO4)));
         Z.bk[1][jt][lane] = cat(pack_exact(mma16(bcL[jj], Ib, ZERO4)), pack_exact(mma16(kcL[jj], Ib, ZERO4)));
         bf16x4 hi, lo;
         split_f4(xv, hi, lo);
         Z.vt[0][jt][lane] = pack_exact(mma16(hi, Ib, ZERO4));
         Z.vt[1][jt][lane] = pack_exact(mma16(lo, Ib, ZERO4));
-        *reinterpret_cast<f32x4*>(&Z.rq[jj][cc][lane]) = rc;  // rc, until Rq
+        *reinterpret_cast<f32x4*>(&P.rq[jj][cc][lane]) = rc;  // rc, until Rq
       }
       const bf16x8 rH = cat(rcH[0], rcH[1]), rL = cat(rcL[0], rcL[1]);
       const bf16x8 kH = cat(kcH[0], kcH[1]), kL = cat(kcL[0], kcL[1]);
@@ -472,7 +518,7 @@ __global__ __launch_bounds__(512, 1) void wkv7_chunk_kernel(
       reinterpret_cast<float*>(&Z.pc[jt][kg])[e] = __builtin_amdgcn_exp2f(clamp126(myGC - myCF));
       reinterpret_cast<float*>(&Z.cen[jt][kg])[e] = __builtin_amdgcn_ldexpf(1.f, ci);
     }
-    if (x + 4 < nchunks) issue(x + 4);  // the raw rows are consumed; the next ones land meanwhile
+    if (x + 4 < xend) issue(x + 4);  // the raw rows are consumed; the next ones land meanwhile
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int s4 = 4 * kg + e;
@@ -553,9 +599,9 @@ __global__ __launch_bounds__(512, 1) void wkv7_chunk_kernel(
     // ---- Wa = T ac and Rq = rc + Pm ac (lane (t, sigma) layout) replace D(ac) and rc
 #pragma unroll
     for (int cc = 0; cc < 2; ++cc) {
-      const bf16x8 dH = Z.wa[0][cc][lane], dL = Z.wa[1][cc][lane];
-      const f32x4 rc0 = *reinterpret_cast<const f32x4*>(&Z.rq[0][cc][lane]);
-      const f32x4 rc1 = *reinterpret_cast<const f32x4*>(&Z.rq[1][cc][lane]);
+      const bf16x8 dH = P.wa[0][cc][lane], dL = P.wa[1][cc][lane];
+      const f32x4 rc0 = *reinterpret_cast<const f32x4*>(&P.rq[0][cc][lane]);
+      const f32x4 rc1 = *reinterpret_cast<const f32x4*>(&P.rq[1][cc][lane]);
       bf16x4 waH[2], waL[2], rqH[2], rqL[2];
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj) {
@@ -580,11 +626,211 @@ __global__ __launch_bounds__(512, 1) void wkv7_chunk_kernel(
       Z.aq[0][lane] = qH;
       Z.aq[1][lane] = qL;
     }
-    set_flag(&L.ready[s], x);
+    if constexpr (!SPLIT) set_flag(&L.ready[s], x);
   }
   // |gC| <= 252 keeps every centred exponent (at most |gC| / 2 + 1/2) within +-126
   const bool clamped = __builtin_amdgcn_ballot_w64(gmin < -252.f || gmax > 252.f) != 0;
   post_status((waited_out ? WKV7_STATUS_TIMEOUT : 0) | (clamped ? WKV7_STATUS_CLAMPED : 0));
+}
+
+// ---- the chain of the two-kernel form: one workgroup per (batch, head) over the
+// chunks x0 .. x0 + xn - 1 whose slots the producers left in memory.  A step is a
+// serial chain of split, U products, split, update products on one wave, so all
+// else is taken off the four chain waves (value tile q each): waves 4 .. 7 bring
+// the slots into a ring of CRING LDS stages by LDS DMA (a quarter of a slot
+// each) and make Y of tile q one chunk later, from the S' operand that the chain
+// wave leaves in LDS.  One barrier a chunk is the only hand-over.  Bound by the
+// latency of that serial chain: 0.70 us a chunk, against 0.83 with the DMA and Y
+// on the chain waves and 0.37 for the slots' way through L2 and LDS alone.
+constexpr int CRING = 5;
+constexpr int CSTAGE = 24 * 1024;
+static_assert(sizeof(ChunkSlot) <= CSTAGE && sizeof(ChunkSlot) % 16 == 0, "a stage holds one slot");
+struct ChainShared {
+  char ring[CRING][CSTAGE];
+  bf16x8 sp[2][4][2][2][64];  // [chunk parity][tile][hi/lo][k half cc][lane]: S' as the B operand of U and Y
+};
+
+// y[jt][e] = x[jt][e] times the factor of channel slot 4 jt + e, which lane 4 jt + e of the 16-lane row holds
+template <int JT>
+__device__ __forceinline__ f32x4 row_scale(const f32x4& x, float f) {
+  const int v = __float_as_int(f);
+  return (f32x4){x[0] * __int_as_float(__builtin_amdgcn_update_dpp(0, v, 0x150 + 4 * JT, 0xF, 0xF, true)),
+                 x[1] * __int_as_float(__builtin_amdgcn_update_dpp(0, v, 0x151 + 4 * JT, 0xF, 0xF, true)),
+                 x[2] * __int_as_float(__builtin_amdgcn_update_dpp(0, v, 0x152 + 4 * JT, 0xF, 0xF, true)),
+                 x[3] * __int_as_float(__builtin_amdgcn_update_dpp(0, v, 0x153 + 4 * JT, 0xF, 0xF, true))};
+}
+__device__ __forceinline__ void row_scale4(f32x4 (&y)[4], const f32x4 (&x)[4], float f) {
+  y[0] = row_scale<0>(x[0], f);
+  y[1] = row_scale<1>(x[1], f);
+  y[2] = row_scale<2>(x[2], f);
+  y[3] = row_scale<3>(x[3], f);
+}
+
+template <typename TA>
+__global__ __launch_bounds__(512, 1) void wkv7_chain_kernel(const ChunkSlot* __restrict__ slots, const float* state_in,
+                                                            float* state_out, TA* __restrict__ y, int T, int H, int x0,
+                                                            int xn_) {
+  extern __shared__ __align__(16) char smem_raw[];
+  ChainShared& L = *reinterpret_cast<ChainShared*>(smem_raw);
+  typedef __attribute__((address_space(3))) void* lds_ptr;
+  const int xn = __builtin_amdgcn_readfirstlane(xn_);
+  const int bh = blockIdx.x, b = bh / H, h = bh % H;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int q = wave & 3, l16 = lane & 15, kg = lane >> 4;
+  const int ich = 32 * (q >> 1) + 8 * (l16 >> 2) + 4 * (q & 1) + (l16 & 3);
+  auto slot = [&](int st) -> const ChunkSlot& { return *reinterpret_cast<const ChunkSlot*>(&L.ring[st][0]); };
+
+  if (wave >= 4) {
+    // ===== DMA and Y of tile q.  Step i: chunk i + 1 has landed (for the chain
+    // waves to read in this step); the stage of chunk i - 2, whose Y was made in
+    // step i - 1, takes chunk i + 3; Y of chunk i - 1.
+    const ChunkSlot* base = slots + (int64_t)bh * xn;
+    auto issue = [&](int c, int st) {  // past the slot's end, or the last slot: read nothing
+      const int c0 = __builtin_amdgcn_readfirstlane(c < xn ? c : 0);
+      const int bytes = __builtin_amdgcn_readfirstlane(c < xn ? (int)sizeof(ChunkSlot) : 0);
+      const __amdgpu_buffer_rsrc_t rs = make_rsrc(base + c0, (uint32_t)bytes);
+#pragma unroll
+      for (int u = 0; u < 6; ++u)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr)(&L.ring[st][1024 * (6 * q + u)]), 16,
+                                                 1024 * (6 * q + u) + 16 * lane, 0, 0, 0);
+    };
+    const int64_t tok = (int64_t)H * HD;
+    uint32_t yoff[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) yoff[e] = (uint32_t)(((4 * kg + e) * tok + ich) * (int64_t)sizeof(TA));
+    TA* yc = y + (((int64_t)b * T + (int64_t)x0 * CH) * H + h) * HD;
+    int left = T - x0 * CH;  // tokens from chunk i - 1 on
+#pragma unroll
+    for (int c = 0; c < 3; ++c) issue(c, c);
+    __builtin_amdgcn_s_waitcnt(0x0F7C);  // vmcnt(12): chunk 0 landed
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0, st = 0; i <= xn; ++i) {  // st: the stage of chunk i
+      // outstanding after chunk i + 1's six loads: chunk i + 2's, and from step
+      // 3 on the four stores of each of the two steps before
+      if (i < 3) __builtin_amdgcn_s_waitcnt(0x0F76);  // vmcnt(6)
+      else __builtin_amdgcn_s_waitcnt(0x0F7E);        // vmcnt(14)
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      issue(i + 3, st + 3 >= CRING ? st + 3 - CRING : st + 3);
+      if (i > 0) {
+        const ChunkSlot& Z = slot(st == 0 ? CRING - 1 : st - 1);
+        const auto& SP = L.sp[(i - 1) & 1][q];
+        f32x4 Yv = ZERO4;
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc)
+          Yv = mma3_32(Z.rq[0][cc][lane], Z.rq[1][cc][lane], SP[0][cc][lane], SP[1][cc][lane], Yv);
+        const bf16x4 vH = Z.vt[0][q][lane], vL = Z.vt[1][q][lane], aqH = Z.aq[0][lane], aqL = Z.aq[1][lane];
+        Yv = mfma16x16x32(cat(aqH, aqH), cat(vH, vL), Yv);
+        Yv = mfma16x16x32(cat(aqL, (bf16x4){}), cat(vH, (bf16x4){}), Yv);
+        const __amdgpu_buffer_rsrc_t ys = make_rsrc(yc, (uint32_t)(min(CH, left) * tok * (int64_t)sizeof(TA)));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) store_y<TA>(ys, yoff[e], Yv[e]);
+        yc += CH * tok;
+        left -= CH;
+      }
+      st = st + 1 == CRING ? 0 : st + 1;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): no load into LDS is pending when the wave ends
+    return;
+  }
+
+  // ===== chain wave of tile q (the products of the one-launch kernel, in its order)
+  __builtin_amdgcn_s_setprio(1);
+  f32x4 S[4];
+  {
+    const float* src = state_in + ((int64_t)bh * HD + ich) * HD + 8 * kg;
+#pragma unroll
+    for (int jt = 0; jt < 4; ++jt) {
+      const float4 t4 = *reinterpret_cast<const float4*>(src + 32 * (jt >> 1) + 4 * (jt & 1));
+      S[jt] = (f32x4){t4.x, t4.y, t4.z, t4.w};
+    }
+  }
+  // a chunk's operands, read in three parts as the chunk before is done with each
+  bf16x8 wa[2][2], bk[2][4];
+  bf16x4 v[2], am[2];
+  float pc, cen;  // of channel slot l16 of row kg
+  auto load0 = [&](const ChunkSlot& Z) {
+    cen = reinterpret_cast<const float*>(&Z.cen[l16 >> 2][kg])[l16 & 3];
+#pragma unroll
+    for (int cc = 0; cc < 2; ++cc) {
+      wa[0][cc] = Z.wa[0][cc][lane];
+      wa[1][cc] = Z.wa[1][cc][lane];
+    }
+  };
+  auto load1 = [&](const ChunkSlot& Z) {
+#pragma unroll
+    for (int hl = 0; hl < 2; ++hl) {
+      v[hl] = Z.vt[hl][q][lane];
+      am[hl] = Z.am[hl][lane];
+#pragma unroll
+      for (int jt = 0; jt < 4; ++jt) bk[hl][jt] = Z.bk[hl][jt][lane];
+    }
+  };
+  auto load2 = [&](const ChunkSlot& Z) { pc = reinterpret_cast<const float*>(&Z.pc[l16 >> 2][kg])[l16 & 3]; };
+  __builtin_amdgcn_s_barrier();  // chunk 0 landed
+  __builtin_amdgcn_sched_barrier(0);
+  // (in the loop's order, so that a step waits for part 0 alone at its start)
+  load0(slot(0));
+  __builtin_amdgcn_sched_barrier(0);
+  load1(slot(0));
+  __builtin_amdgcn_sched_barrier(0);
+  load2(slot(0));
+  __builtin_amdgcn_sched_barrier(0);
+  for (int c = 0, st = 0; c < xn; ++c) {
+    st = st + 1 == CRING ? 0 : st + 1;
+    const ChunkSlot& Zn = slot(st);  // chunk c + 1
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 Sp[4];
+    bf16x4 SH[4], SL[4];
+    row_scale4(Sp, S, cen);
+#pragma unroll
+    for (int jt = 0; jt < 4; ++jt) split_f4(Sp[jt], SH[jt], SL[jt]);
+    f32x4 U = ZERO4;
+    auto& SP = L.sp[c & 1][q];
+#pragma unroll
+    for (int cc = 0; cc < 2; ++cc) {
+      const bf16x8 sh = cat(SH[2 * cc], SH[2 * cc + 1]), sl = cat(SL[2 * cc], SL[2 * cc + 1]);
+      U = mma3_32(wa[0][cc], wa[1][cc], sh, sl, U);
+      SP[0][cc][lane] = sh;
+      SP[1][cc][lane] = sl;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    load0(Zn);
+    __builtin_amdgcn_sched_barrier(0);
+    const bf16x8 vHL = cat(v[0], v[1]), vH0 = cat(v[0], (bf16x4){});
+    U = mfma16x16x32(cat(am[0], am[0]), vHL, U);
+    U = mfma16x16x32(cat(am[1], (bf16x4){}), vH0, U);
+    bf16x4 UH, UL;
+    split_f4(U, UH, UL);
+    const bf16x8 uvH = cat(UH, v[0]), uvL = cat(UL, v[1]);
+#pragma unroll
+    for (int jt = 0; jt < 4; ++jt) Sp[jt] = mma3_32(bk[0][jt], bk[1][jt], uvH, uvL, Sp[jt]);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): S' is in LDS before this wave's next barrier
+    load1(Zn);
+    __builtin_amdgcn_sched_barrier(0);
+    row_scale4(S, Sp, pc);
+    __builtin_amdgcn_sched_barrier(0);
+    load2(Zn);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  __builtin_amdgcn_s_barrier();  // the last chunk's S' for its Y
+  float* dst = state_out + ((int64_t)bh * HD + ich) * HD + 8 * kg;
+#pragma unroll
+  for (int jt = 0; jt < 4; ++jt)
+    *reinterpret_cast<float4*>(dst + 32 * (jt >> 1) + 4 * (jt & 1)) = make_float4(S[jt][0], S[jt][1], S[jt][2], S[jt][3]);
+}
+
+// chunks of one producer / chain launch pair: all of them up to SPLIT_BYTES of slots
+static int split_chunks(int64_t BH, int64_t T) {
+  const int64_t n = (T + CH - 1) / CH;
+  if (BH <= 0 || n < SPLIT_MIN || BH > SPLIT_HEADS) return 0;
+  const int64_t cap = std::max<int64_t>(1, SPLIT_BYTES / (BH * (int64_t)sizeof(ChunkSlot)));
+  const int64_t segs = (n + cap - 1) / cap;
+  return (int)((n + segs - 1) / segs);
 }
 
 }  // namespace rwkv7mi
@@ -594,23 +840,49 @@ using namespace rwkv7mi;
 template <typename TA, typename TW, int WMODE>
 static int chunk_go(int64_t B, int64_t T, int64_t H, void* stream, const void* r, const void* w, const void* k,
                     const void* v, const void* kk, const void* a, const float* state_in, float* state_out,
-                    void* y) {
+                    void* y, void* ws, int64_t ws_bytes) {
+  const int xn = split_chunks(B * H, T);
+  if (xn > 0 && ws && ws_bytes >= B * H * xn * (int64_t)sizeof(ChunkSlot) && !(reinterpret_cast<uintptr_t>(ws) & 15)) {
+    static std::atomic<uint64_t> chain_raised{0};
+    if (int rc = raise_dynamic_lds(reinterpret_cast<const void*>(&wkv7_chain_kernel<TA>), (int)sizeof(ChainShared), chain_raised,
+                                   "wkv7_chain_kernel"))
+      return rc;
+    const int nchunks = (int)((T + CH - 1) / CH), nbh = (int)(B * H), pad = (nbh + 7) & ~7;
+    for (int x0 = 0; x0 < nchunks; x0 += xn) {
+      const int n = std::min(xn, nchunks - x0);
+      hipLaunchKernelGGL((wkv7_chunk_kernel<TA, TW, WMODE, true>), dim3((unsigned)((n + 3) / 4 * pad)), dim3(256),
+                         sizeof(SplitShared), as_stream(stream), (const TA*)r, (const TW*)w, (const TA*)k, (const TA*)v,
+                         (const TA*)kk, (const TA*)a, state_in, state_out, (TA*)y, (int)T, (int)H, (ChunkSlot*)ws, nbh,
+                         x0, n);
+      if (int rc = check_launch("wkv7_chunk_kernel")) return rc;
+      hipLaunchKernelGGL((wkv7_chain_kernel<TA>), dim3((unsigned)nbh), dim3(512), sizeof(ChainShared), as_stream(stream),
+                         (const ChunkSlot*)ws, x0 ? (const float*)state_out : state_in, state_out, (TA*)y, (int)T,
+                         (int)H, x0, n);
+      if (int rc = check_launch("wkv7_chain_kernel")) return rc;
+    }
+    return RWKV7MI_OK;
+  }
   static std::atomic<uint64_t> lds_raised{0};  // devices whose dynamic LDS limit is raised for this instance
   const size_t lds = sizeof(ChunkShared);
-  if (int rc = raise_dynamic_lds(reinterpret_cast<const void*>(&wkv7_chunk_kernel<TA, TW, WMODE>), (int)lds,
+  if (int rc = raise_dynamic_lds(reinterpret_cast<const void*>(&wkv7_chunk_kernel<TA, TW, WMODE, false>), (int)lds,
                                  lds_raised, "wkv7_chunk_kernel"))
     return rc;
-  hipLaunchKernelGGL((wkv7_chunk_kernel<TA, TW, WMODE>), dim3((unsigned)(B * H)), dim3(512), lds, as_stream(stream),
+  hipLaunchKernelGGL((wkv7_chunk_kernel<TA, TW, WMODE, false>), dim3((unsigned)(B * H)), dim3(512), lds, as_stream(stream),
                      (const TA*)r, (const TW*)w, (const TA*)k, (const TA*)v, (const TA*)kk, (const TA*)a, state_in,
-                     state_out, (TA*)y, (int)T, (int)H);
+                     state_out, (TA*)y, (int)T, (int)H, nullptr, 0, 0, 0);
   return check_launch("wkv7_chunk_kernel");
 }
 
-extern "C" int rwkv7mi_wkv7_chunk_prefill(const void* r, const void* w, const void* k, const void* v,
+extern "C" int64_t rwkv7mi_wkv7_chunk_workspace_bytes(int64_t B, int64_t T, int64_t H) {
+  if (B <= 0 || T <= 0 || H <= 0 || B > INT32_MAX || H > INT32_MAX || T > INT32_MAX) return 0;
+  return B * H * split_chunks(B * H, T) * (int64_t)sizeof(ChunkSlot);
+}
+
+extern "C" int rwkv7mi_wkv7_chunk_prefill_ws(const void* r, const void* w, const void* k, const void* v,
                                           const void* kk, const void* a, const float* state_in,
                                           float* state_out, void* y, int64_t B, int64_t T, int64_t H,
                                           int64_t N, int64_t chunk, int w_is_log, int act_dtype,
-                                          int w_dtype, void* stream) {
+                                          int w_dtype, void* ws, int64_t ws_bytes, void* stream) {
   if (N != HD) return fail(RWKV7MI_EINVAL, "wkv7 chunk: head size must be 64");
   if (w_is_log < 0 || w_is_log > 2) return fail(RWKV7MI_EINVAL, "wkv7 chunk: w mode must be 0, 1 or 2");
   if (chunk != 16 && chunk != 32 && chunk != 64)
@@ -633,11 +905,20 @@ extern "C" int rwkv7mi_wkv7_chunk_prefill(const void* r, const void* w, const vo
     if (al & 15) return fail(RWKV7MI_EINVAL, "wkv7 chunk: inputs must be 16-byte aligned");
     return dispatch_dtype(w_dtype, [&](auto tw) {
       using TW = decltype(tw);
-      if (w_is_log == 1) return chunk_go<TA, TW, 1>(B, T, H, stream, r, w, k, v, kk, a, state_in, state_out, y);
-      if (w_is_log == 2) return chunk_go<TA, TW, 2>(B, T, H, stream, r, w, k, v, kk, a, state_in, state_out, y);
-      return chunk_go<TA, TW, 0>(B, T, H, stream, r, w, k, v, kk, a, state_in, state_out, y);
+      if (w_is_log == 1) return chunk_go<TA, TW, 1>(B, T, H, stream, r, w, k, v, kk, a, state_in, state_out, y, ws, ws_bytes);
+      if (w_is_log == 2) return chunk_go<TA, TW, 2>(B, T, H, stream, r, w, k, v, kk, a, state_in, state_out, y, ws, ws_bytes);
+      return chunk_go<TA, TW, 0>(B, T, H, stream, r, w, k, v, kk, a, state_in, state_out, y, ws, ws_bytes);
     });
   });
+}
+
+extern "C" int rwkv7mi_wkv7_chunk_prefill(const void* r, const void* w, const void* k, const void* v,
+                                          const void* kk, const void* a, const float* state_in,
+                                          float* state_out, void* y, int64_t B, int64_t T, int64_t H,
+                                          int64_t N, int64_t chunk, int w_is_log, int act_dtype,
+                                          int w_dtype, void* stream) {
+  return rwkv7mi_wkv7_chunk_prefill_ws(r, w, k, v, kk, a, state_in, state_out, y, B, T, H, N, chunk, w_is_log,
+                                       act_dtype, w_dtype, nullptr, 0, stream);
 }
 
 extern "C" int rwkv7mi_wkv7_chunk_status(int clear, int* status) {

@@ -45,6 +45,11 @@ SIGNATURES = {
         _i32,
         [_c_p] * 9 + [_i64, _i64, _i64, _i64, _i64, _i32, _i32, _i32, _c_p],
     ),
+    "rwkv7mi_wkv7_chunk_prefill_ws": (
+        _i32,
+        [_c_p] * 9 + [_i64, _i64, _i64, _i64, _i64, _i32, _i32, _i32, _c_p, _i64, _c_p],
+    ),
+    "rwkv7mi_wkv7_chunk_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "rwkv7mi_wkv7_chunk_status": (_i32, [_i32, ctypes.POINTER(_i32)]),
     "rwkv7mi_wkv7_fp16_decode_output_prepare_raw": (
         _i32,

@@ -43,11 +43,14 @@ def _run_chunk(r4, w4, k4, v4, kk4, a4, state, *, w_is_log: int, chunk: int,
     st = state.contiguous()
     final = _state_dst(st, state_out)
     y = out if out is not None else torch.empty((B, T, H, N), device=r4.device, dtype=r4.dtype)
+    # the two-launch form's operands; the call's own, so concurrent streams share nothing
+    need = int(_lib.load().rwkv7mi_wkv7_chunk_workspace_bytes(B, T, H)) if N == 64 else 0
+    ws = torch.empty(need, dtype=torch.uint8, device=r4.device) if need else None
     _lib.call(
-        "rwkv7mi_wkv7_chunk_prefill",
+        "rwkv7mi_wkv7_chunk_prefill_ws",
         _lib.ptr(r4), _lib.ptr(w4), _lib.ptr(k4), _lib.ptr(v4), _lib.ptr(kk4), _lib.ptr(a4),
         _lib.ptr(st), _lib.ptr(final), _lib.ptr(y), B, T, H, N, int(chunk), int(w_is_log),
-        _lib.dtype_code(r4), _lib.dtype_code(w4), _lib.stream_of(r4),
+        _lib.dtype_code(r4), _lib.dtype_code(w4), _lib.ptr(ws), need, _lib.stream_of(r4),
     )
     return y, final
 

@@ -147,6 +147,19 @@ int rwkv7mi_wkv7_chunk_prefill(const void* r, const void* w, const void* k,
                                int64_t N, int64_t chunk, int w_is_log,
                                int act_dtype, int w_dtype, void* stream);
 
+/* The same over a 16-byte aligned workspace of rwkv7mi_wkv7_chunk_workspace_bytes
+ * (0: none is used): few heads then run as a launch that makes the chunks'
+ * operands on the whole chip and one that moves the states over them.  Without
+ * (or with a smaller) workspace: rwkv7mi_wkv7_chunk_prefill, the same results. */
+int64_t rwkv7mi_wkv7_chunk_workspace_bytes(int64_t B, int64_t T, int64_t H);
+int rwkv7mi_wkv7_chunk_prefill_ws(const void* r, const void* w, const void* k,
+                                  const void* v, const void* kk, const void* a,
+                                  const float* state_in, float* state_out,
+                                  void* y, int64_t B, int64_t T, int64_t H,
+                                  int64_t N, int64_t chunk, int w_is_log,
+                                  int act_dtype, int w_dtype, void* ws,
+                                  int64_t ws_bytes, void* stream);
+
 /* Sticky status bits of the chunk kernel on the current device since the last
  * clear: 1 = a bounded wait between the kernel's waves gave up (that call's
  * output is void), 2 = a chunk's log2-decay span exceeded 252 and the gate

@@ -164,3 +164,43 @@ def test_chunk_full_size_properties(H):
     assert torch.isfinite(y1).all() and torch.isfinite(s1).all()
     assert (y1.float() - y2.float()).abs().max().item() <= 1e-2
     assert ((s1 - s2).abs().max() / s2.abs().max()).item() <= 2e-4
+
+
+@pytest.mark.parametrize("B,T,H,mode,dtype", [
+    (1, 241, 1, 0, torch.float16),   # the least chunk count, the last chunk of one token; one head of a group of eight
+    (1, 336, 12, 1, torch.bfloat16),  # 21 chunks: a last producer workgroup of one chunk
+    (3, 305, 5, 2, torch.float32),   # an even number of chunks over 15 heads
+    (1, 2200, 64, 1, torch.float16),  # two launch pairs
+    (1, 2113, 8, 0, torch.bfloat16),  # many times around the ring
+])
+def test_chunk_two_kernel_form_has_the_fused_bits(B, T, H, mode, dtype):
+    """Few heads run as producers over the whole chip and a chain per head: the
+    same operands and products as the one-launch kernel, so the same bits."""
+    from rwkv7mi import _lib
+    from rwkv7mi.self_chunk_rwkv7 import _run_chunk, wkv7_chunk_status
+
+    args, st, _ = _inputs(np.random.default_rng(T), B, T, H, dtype=dtype, state_scale=0.1)
+    if mode:
+        args[1] = torch.log(args[1]) if mode == 1 else torch.randn_like(args[1])
+    lib = _lib.load()
+    assert lib.rwkv7mi_wkv7_chunk_workspace_bytes(B, T, H) > 0
+    assert lib.rwkv7mi_wkv7_chunk_workspace_bytes(B, 240, H) == 0 == lib.rwkv7mi_wkv7_chunk_workspace_bytes(64, T, 64)
+    wkv7_chunk_status(clear=True)
+    want, ws_ = torch.empty_like(args[0]), st.clone()
+    _lib.call("rwkv7mi_wkv7_chunk_prefill", *(_lib.ptr(t) for t in (*args, st, ws_, want)), B, T, H, 64, 16, mode,
+              _lib.dtype_code(want), _lib.F32, _lib.stream_of(want))
+    y, s = _run_chunk(*args, st, w_is_log=mode, chunk=16)
+    inplace = st.clone()
+    _run_chunk(*args, inplace, w_is_log=mode, chunk=16, state_out=inplace)
+    torch.cuda.synchronize()
+    assert torch.equal(y, want) and torch.equal(s, ws_) and torch.equal(inplace, ws_)
+    assert wkv7_chunk_status(clear=True) == 0
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        y, s = _run_chunk(*args, st, w_is_log=mode, chunk=16)
+    for _ in range(3):
+        y.zero_()
+        s.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want) and torch.equal(s, ws_)
