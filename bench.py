@@ -135,6 +135,8 @@ def time_graph(calls, reps=20):
     returns the mean ms per call."""
     import torch
 
+    from rwkv7mi.model import graph_capture
+
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
@@ -142,7 +144,7 @@ def time_graph(calls, reps=20):
             c()
     torch.cuda.current_stream().wait_stream(side)
     graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
+    with graph_capture(graph):
         for c in calls:
             c()
     graph.replay()

@@ -16,8 +16,11 @@ library GEMMs of dense (unquantised) projections (rocBLAS through torch).
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
+import gc
 import os
+import threading
 import weakref
 import zlib
 from dataclasses import dataclass
@@ -1714,6 +1717,36 @@ class _LazyWeights(dict):
 
 
 # ------------------------------------------------------------------ graph runner
+_captures = 0
+_captures_lock = threading.Lock()
+_gc_was_on = False
+
+
+@contextlib.contextmanager
+def graph_capture(graph):
+    """``torch.cuda.graph(graph)`` with the cyclic collector off.
+
+    A dropped model and its runners are a reference cycle, so their graphs are
+    destroyed whenever the collector happens to run.  Destroying one waits for
+    the device, which is an error while a stream is capturing, and the error
+    leaves a C++ destructor: the process aborts.  What became garbage is
+    collected as usual after the capture."""
+    global _captures, _gc_was_on
+    with _captures_lock:
+        if _captures == 0:
+            _gc_was_on = gc.isenabled()
+            gc.disable()
+        _captures += 1
+    try:
+        with torch.cuda.graph(graph):
+            yield
+    finally:
+        with _captures_lock:
+            _captures -= 1
+            if _captures == 0 and _gc_was_on:
+                gc.enable()
+
+
 class NativeGraphRunner:
     """hipGraph-captured decode step for a fixed batch (rwkv7_hf/native_graph_runtime.py:212-711).
 
@@ -1745,7 +1778,7 @@ class NativeGraphRunner:
                 self._step()
         torch.cuda.current_stream(dev).wait_stream(side)
         self.graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self.graph):
+        with graph_capture(self.graph):
             self._step()
         self._copy_into(snapshot)
         self.replays = 0
@@ -1868,7 +1901,7 @@ class NativePrefillGraphRunner:
         torch.cuda.current_stream(dev).wait_stream(side)
         self._zero_state()
         self.graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self.graph):
+        with graph_capture(self.graph):
             self.logits = model.prefill_(self.ids, self.cache, logits_to_keep=self.logits_to_keep)
         self.replays = 0
 

@@ -263,11 +263,12 @@ def test_mm8_rows_route_and_capture(oracle):
     key = (torch.cuda.current_device(), "mm8r")
     kept = _ws._buffers.pop(key)
     try:
+        from rwkv7mi.model import graph_capture
         from rwkv7mi.native_quant_mm8 import mm8_gemm_prefill_multi_into
 
         mm8_gemm_prefill_multi_into([x], [mod], [want])
         g = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(g):
+        with graph_capture(g):
             mm8_many_rows_into([x], [mod], [y])
         for _ in range(3):
             y.zero_()
