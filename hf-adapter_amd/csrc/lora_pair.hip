@@ -8,11 +8,11 @@
 // mid (the reference's own tensor, in the activation dtype) goes through the
 // workspace: rows x 288 values against rows x 4 x 4096 of x and y.
 //
-// Measured (D = A = 4096, ranks 64/64/128/32, kernel time, before -> after):
-//   fp16  700 rows  233 -> 42 us (the one-launch kernel put 12 workgroups on
-//         the chip), 2000 rows 235 -> 73, 4000 rows 238 -> 137; 250 rows at
-//         2048: 68 -> 22 (four 64-row split-K pairs)
-//   bf16  700 rows  475 -> 42 us, 16000 rows 1250 -> 414 (bf16 MFMAs on the
+// Measured (D = A = 4096, ranks 64/64/128/32, both launches, before -> after):
+//   fp16  700 rows  233 -> 35 us (the one-launch kernel put 12 workgroups on
+//         the chip), 2000 rows 235 -> 63, 4000 rows 238 -> 115; 250 rows at
+//         2048: 68 -> 16 (four 64-row split-K pairs)
+//   bf16  700 rows  475 -> 35 us, 16000 rows 1250 -> 371 (bf16 MFMAs on the
 //         values themselves instead of three fp16 ones on a split)
 // From LORA_SEQ_WGS workgroups of lora_seq_kernel on the chip is full and it
 // moves fewer bytes: 16000 rows at 2048 183 against 216, 32768 at 4096 738
@@ -30,7 +30,7 @@ namespace {
 template <typename TA> struct LpVec { typedef f16x8 V; typedef _Float16 E; };
 template <> struct LpVec<__hip_bfloat16> { typedef bf16x8 V; typedef __bf16 E; };
 
-constexpr int LP_NW = 8;       // mid: waves per workgroup, each a share of K
+constexpr int LP_NW = 4;       // mid: waves per workgroup, each a share of K
 constexpr int LP_RT = 4;       // mid: rank tiles of 16 per workgroup (64 rank columns)
 constexpr int LP_RS = 68;      // mid: LDS row (floats): 64 rank columns, 16-byte aligned, bank-skewed
 constexpr int LP_MAXUNITS = 8; // 4 problems x ceil(128 / 64)
@@ -51,26 +51,42 @@ struct LpBatch {
 
 }  // namespace
 
-// A workgroup takes 16 MT rows x 64 rank columns of one problem over all of K.
-// Bound by what one CU pulls through its L1 (about 33 GB/s here, whatever the
-// load order or the number in flight): 64 rank columns are 512 KB at D = 4096,
-// so the 128-column G problem is two units, and the rows are cut finely enough
-// (MT) to give every CU a workgroup.  Its eight
-// waves split K: wave w takes the 64-input steps w, w + 8, ..; a lane reads
-// inputs 16 kg .. +15 of a step (two 16-byte loads: whole 128-byte lines per
-// row over the four kg), the same k order for both operands.  The next step's
-// loads are issued before this step's MFMAs.  The waves' sums meet in LDS, one
-// 16-row tile at a time, added in wave order.
+// A workgroup takes 16 MT rows x 64 rank columns of one problem over all of K;
+// the 128-column G problem is two units, and the rows are cut finely enough (MT)
+// to give every CU a workgroup.  Bound by what one CU pulls: in the MFMA operand
+// order neighbouring lanes read different rows, 16 bytes of a line at a time,
+// and a CU's L1 then gave about 33 GB/s (the two launches at 4096: 65 rows 28 us
+// against 16 now, 250 rows 33 and 21, 700 rows 44 and 35, 8000 215 and 184; 65
+// rows at 768 14 and 10).  So each of the four waves brings its own
+// 64-input steps (w, w + 4, ..) in by LDS DMA, 128 contiguous bytes per eight
+// lanes, into a ring of LP_R stages of its own: no barrier in the loop, only the
+// wave's own counters.  The 16-byte chunk c of a row lies at position c ^ (r % 8)
+// ^ (r / 8 % 2), which leaves the operand reads free of bank conflicts on gfx950.
+// The waves' sums meet in LDS, one 16-row tile at a time, added in wave order.
+template <int MT>
+struct LpMid {
+  static constexpr int R = MT == 4 ? 2 : 3;       // stages of a wave
+  static constexpr int NL = 2 * MT + 2 * LP_RT;   // DMA instructions (KB) of a step: 8 rows each
+  static constexpr int LDS = LP_NW * R * NL * 1024;
+  // vmcnt: the steps after the oldest one may be in flight
+  static constexpr int LEFT = (R - 1) * NL;
+  static constexpr int WAIT = (LEFT & 15) | 0x0F70 | ((LEFT >> 4) << 14);
+  static_assert(LDS <= 160 * 1024 && LDS >= LP_NW * 16 * LP_RS * 4 && LEFT < 64, "ring of a workgroup");
+};
+
 template <typename TA, int MT>
-__global__ __launch_bounds__(64 * LP_NW) void lora_mid_kernel(const LpBatch B) {
+__global__ __launch_bounds__(64 * LP_NW, 1) void lora_mid_kernel(const LpBatch B) {
   using V = typename LpVec<TA>::V;
-  __shared__ __align__(16) float red[LP_NW][16][LP_RS];
+  typedef __attribute__((address_space(3))) void* lds_ptr;
+  using M = LpMid<MT>;
+  extern __shared__ __align__(16) char smem[];
   const LpProb& P = B.p[B.unit_p[blockIdx.y]];
   const int D = B.D, r = P.r;
   const int c0 = 64 * B.unit_t[blockIdx.y];
   const int row0 = blockIdx.x * 16 * MT;
   const int nrow = min(16 * MT, B.rows - row0);
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, kg = lane >> 4;
   // descriptors end at the tile's last row / the problem's last rank: rows and
   // ranks past them read zeros
@@ -85,65 +101,76 @@ __global__ __launch_bounds__(64 * LP_NW) void lora_mid_kernel(const LpBatch B) {
 #pragma unroll
     for (int t = 0; t < LP_RT; ++t) acc[m][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-  auto load = [&](int s, V (&xa)[MT][2], V (&wb)[LP_RT][2]) {
+  char* ring = smem + wave * M::R * M::NL * 1024;
+  // instruction u: rows 8 u + lane / 8, the chunk of position lane % 8
+  const int ch = (lane & 7) ^ (lane >> 3);
+  auto issue = [&](int s, int st) {
+    char* d = ring + st * M::NL * 1024;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int kk = 64 * s + 16 * kg + 8 * h;
-      const bool ok = kk < D;  // D % 8 == 0
-#pragma unroll
-      for (int m = 0; m < MT; ++m)
-        xa[m][h] = __builtin_bit_cast(V, buf_ld16(xr, ok ? (uint32_t)(((16 * m + n) * D + kk) * 2) : BUF_OOB));
-#pragma unroll
-      for (int t = 0; t < LP_RT; ++t)
-        wb[t][h] = __builtin_bit_cast(V, buf_ld16(wr, ok ? (uint32_t)(((16 * t + n) * D + kk) * 2) : BUF_OOB));
+    for (int u = 0; u < M::NL; ++u) {
+      const int uu = u < 2 * MT ? u : u - 2 * MT;
+      const int kk = 64 * s + 8 * (ch ^ (uu & 1));
+      const int off = kk < D ? ((8 * uu + (lane >> 3)) * D + kk) * 2 : (int)BUF_OOB;  // D % 8 == 0
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(u < 2 * MT ? xr : wr, (lds_ptr)(d + 1024 * u), 16, off, 0, 0, 0);
     }
   };
-  // Wd as the A operand, x as B: a lane holds one row and four consecutive ranks
-  auto mma = [&](const V (&xa)[MT][2], const V (&wb)[LP_RT][2]) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int t = 0; t < LP_RT; ++t) acc[m][t] = mfma16x16x32(wb[t][h], xa[m][h], acc[m][t]);
+  const int key = (n & 7) ^ (n >> 3);
+  auto read = [&](int st, int tile, int h) {  // 16-row tile, inputs 16 kg + 8 h of the step
+    return *reinterpret_cast<const V*>(ring + st * M::NL * 1024 + (16 * tile + n) * 128 + 16 * ((2 * kg + h) ^ key));
   };
-  // a ring of R steps in flight; the barriers keep the compiler from sinking
-  // the loads to their uses
-  constexpr int R = MT == 1 ? 4 : MT == 2 ? 3 : 2;
-  V xa[R][MT][2], wb[R][LP_RT][2];
   const int nst = ((D + 63) / 64 + LP_NW - 1) / LP_NW;  // steps per wave (past the end: zeros)
 #pragma unroll
-  for (int j = 0; j < R; ++j) load(wave + LP_NW * j, xa[j], wb[j]);
-  __builtin_amdgcn_sched_barrier(0);
-  for (int i = 0; i < nst; i += R) {
+  for (int j = 0; j < M::R; ++j) issue(wave + LP_NW * j, j);
+  for (int i = 0; i < nst; i += M::R) {
 #pragma unroll
-    for (int j = 0; j < R; ++j) {
-      mma(xa[j], wb[j]);
+    for (int j = 0; j < M::R; ++j) {
       __builtin_amdgcn_sched_barrier(0);
-      load(wave + LP_NW * (i + j + R), xa[j], wb[j]);
+      __builtin_amdgcn_s_waitcnt(M::WAIT);  // the oldest step has landed
       __builtin_amdgcn_sched_barrier(0);
+      V xa[MT][2], wb[LP_RT][2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) xa[m][h] = read(j, m, h);
+#pragma unroll
+        for (int t = 0; t < LP_RT; ++t) wb[t][h] = read(j, MT + t, h);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the stage is read and may be overwritten
+      __builtin_amdgcn_sched_barrier(0);
+      issue(wave + LP_NW * (i + j + M::R), j);
+      __builtin_amdgcn_sched_barrier(0);
+      // Wd as the A operand, x as B: a lane holds one row and four consecutive ranks
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int t = 0; t < LP_RT; ++t) acc[m][t] = mfma16x16x32(wb[t][h], xa[m][h], acc[m][t]);
     }
   }
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the trailing loads have landed, the ring is free
+  __syncthreads();
 
+  float(*red)[16][LP_RS] = reinterpret_cast<float(*)[16][LP_RS]>(smem);
   TA* mid = static_cast<TA*>(P.mid);
-  const int er = tid >> 5, ec = 2 * (tid & 31);  // 16 rows x 32 pairs of rank columns
+  const int er = tid >> 4, ec = 4 * (tid & 15);  // 16 rows x 16 runs of four rank columns
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
     if (m) __syncthreads();
 #pragma unroll
     for (int t = 0; t < LP_RT; ++t) *reinterpret_cast<f32x4*>(&red[wave][n][16 * t + 4 * kg]) = acc[m][t];
     __syncthreads();
-    float a = red[0][er][ec], b = red[0][er][ec + 1];
+    f32x4 v = *reinterpret_cast<const f32x4*>(&red[0][er][ec]);
 #pragma unroll
-    for (int w = 1; w < LP_NW; ++w) {
-      a += red[w][er][ec];
-      b += red[w][er][ec + 1];
-    }
-    if (16 * m + er < nrow && c0 + ec < r) {
-      TA* d = mid + (int64_t)(row0 + 16 * m + er) * r + c0 + ec;
-      const uint32_t lo = __builtin_bit_cast(uint16_t, from_f32<TA>(lora_act_fast(a, P.act_d)));
-      const uint32_t hi = __builtin_bit_cast(uint16_t, from_f32<TA>(lora_act_fast(b, P.act_d)));
-      *reinterpret_cast<uint32_t*>(d) = lo | (hi << 16);
+    for (int w = 1; w < LP_NW; ++w) v += *reinterpret_cast<const f32x4*>(&red[w][er][ec]);
+    if (16 * m + er < nrow && c0 + ec < r) {  // r % 8 == 0
+      uint16_t o[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = __builtin_bit_cast(uint16_t, from_f32<TA>(lora_act_fast(v[e], P.act_d)));
+      *reinterpret_cast<uint2*>(mid + (int64_t)(row0 + 16 * m + er) * r + c0 + ec) =
+          make_uint2((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16));
     }
   }
 }
@@ -265,10 +292,12 @@ bool lora_pair_supported(const LoraBatch& b, int64_t rows, int act_dtype, const 
 template <typename TA>
 static int lora_pair_go(LpBatch& b, int nprob, int units, hipStream_t s) {
   const int64_t t16 = ((int64_t)b.rows + 15) / 16;
-  auto mid = [&](auto kern, int mt) {
-    hipLaunchKernelGGL(kern, dim3((unsigned)((t16 + mt - 1) / mt), (unsigned)units), dim3(64 * LP_NW), 0, s, b);
+  auto mid = [&](auto kern, int mt, int lds, std::atomic<uint64_t>& raised) {
+    if (int rc = raise_dynamic_lds(reinterpret_cast<const void*>(kern), lds, raised, "lora_mid_kernel")) return rc;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((t16 + mt - 1) / mt), (unsigned)units), dim3(64 * LP_NW), (size_t)lds, s, b);
     return check_launch("lora_mid_kernel");
   };
+  static std::atomic<uint64_t> raised[3];  // devices whose dynamic LDS limit is raised for each instance
   // rows per workgroup (16 mt): the least time at a fixed rate per CU, i.e.
   // rounds of 256 workgroups x the 64 rank and 16 mt input rows each one reads
   int mt = 1;
@@ -277,8 +306,9 @@ static int lora_pair_go(LpBatch& b, int nprob, int units, hipStream_t s) {
     const int64_t cost = ((t16 + c - 1) / c * units + 255) / 256 * (64 + 16 * c);
     if (cost < best) best = cost, mt = c;
   }
-  const int rc = mt == 4 ? mid(lora_mid_kernel<TA, 4>, 4)
-                         : mt == 2 ? mid(lora_mid_kernel<TA, 2>, 2) : mid(lora_mid_kernel<TA, 1>, 1);
+  const int rc = mt == 4   ? mid(&lora_mid_kernel<TA, 4>, 4, LpMid<4>::LDS, raised[2])
+                 : mt == 2 ? mid(&lora_mid_kernel<TA, 2>, 2, LpMid<2>::LDS, raised[1])
+                           : mid(&lora_mid_kernel<TA, 1>, 1, LpMid<1>::LDS, raised[0]);
   if (rc) return rc;
   b.ncb = (b.A + 255) / 256;
   // rows per workgroup, 16..256: about 512 workgroups (each re-reads its 256

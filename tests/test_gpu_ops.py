@@ -315,7 +315,8 @@ def test_dense_prefill_routes(dt, rows, K, N, epi):
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rows,D,A,ranks", [(65, 512, 264, (64, 72, 128, 8)), (257, 72, 100, (32, 96, 40, 16)),
-                                            (400, 1088, 520, (64, 64, 128, 32)), (2100, 264, 256, (24, 128, 56, 32))])
+                                            (400, 1088, 520, (64, 64, 128, 32)), (2100, 264, 256, (24, 128, 56, 32)),
+                                            (1000, 1096, 264, (64, 64, 128, 32)), (1700, 1160, 256, (64, 24, 128, 32))])
 def test_lora_row_pair_edges(oracle, dt, rows, D, A, ranks):
     """The down / up pair over all rows: row counts that end inside a 16-, 32-
     and 64-row tile, K that ends inside a 64-input step, ranks that end inside
