@@ -15,10 +15,12 @@
 //   bf16  700 rows  475 -> 35 us, 16000 rows 1250 -> 371 (bf16 MFMAs on the
 //         values themselves instead of three fp16 ones on a split)
 // From LORA_SEQ_WGS workgroups of lora_seq_kernel on the chip is full and it
-// moves fewer bytes: 16000 rows at 2048 183 against 216, 32768 at 4096 738
-// against 824; 8000 rows at 4096 (128 workgroups) 247 against 215.
-// At 64 rows and fewer the split-K pair of lora.hip is the faster one (33 rows
-// at 768: 14 against 15 us; 17 at 4096: 14 against 27).
+// moves fewer bytes (seq against this pair, us): 16000 rows (250 workgroups) at
+// 4096 333 and 374, at 2048 166 and 194; 10240 rows (160) 276 and 245, 138 and
+// 127; 8000 rows (128) at 4096 247 and 184.
+// Against the split-K pair of lora.hip, us: 33 rows at 4096 18.7 -> 15.4, 64 rows
+// 22.2 -> 15.9, at 768 12.6 -> 9.3 and 16.4 -> 9.5; 16 rows at 4096 take 13.5 there,
+// and up to 32 rows keep it.
 #include <algorithm>
 
 #include "lora_common.h"

@@ -43,9 +43,9 @@ def lora_workspace_bytes(ranks, rows: int, D: int) -> int:
 def lora_multi(xs, downs, ups, biases, outs, acts_down, acts_up):
     """Grouped LoRA: ``outs[i] = act_up(act_down(xs[i] @ downs[i].T) @ ups[i].T + biases[i])``.
 
-    Two launches for up to four projections: up to 64 rows a split-K down
-    kernel and an up kernel that reduces the fp32 partials, above (fp16, bf16)
-    a down and an up kernel over all rows.  The partials of up to 64 rows live
+    Two launches for up to four projections: up to 32 rows (fp32: 64) a split-K
+    down kernel and an up kernel that reduces the fp32 partials, above (fp16, bf16)
+    a down and an up kernel over all rows.  The scratch of up to 64 rows lives
     in the per-device workspace, the scratch of more rows is this call's own (so
     calls on several streams do not share it).  The largest fp16 prefills, fp32
     and ranks above 128 run in one launch above 256 rows.

@@ -679,8 +679,8 @@ int rwkv7mi_argmax_rows_ws(const void* x, int64_t rows, int64_t n, int64_t ld,
 
 /* ------------------------------------------------------------------ LoRA */
 
-/* Bytes of workspace rwkv7mi_lora_multi uses: fp32 split-K partials up to 64
- * rows, the intermediate in the activation type above (rows x the ranks' sum;
+/* Bytes of workspace rwkv7mi_lora_multi uses: fp32 split-K partials up to 32
+ * rows (fp32: 64), the intermediate in the activation type above (rows x the ranks' sum;
  * more than 256 rows also run without one, on a slower kernel). */
 size_t rwkv7mi_lora_workspace_bytes(int64_t nprob, const int64_t* ranks,
                                     int64_t rows, int64_t D);
