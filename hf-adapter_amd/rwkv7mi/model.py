@@ -256,7 +256,8 @@ class DenseLinear:
         the products do not share a shape and dtype."""
         x = xs[0]
         rows = int(x.shape[0])
-        if (len(lins) > 4 or len({(l.in_features, l.out_features, l.weight.dtype) for l in lins}) != 1
+        if (len(lins) > 4 or not len(lins) == len(xs) == len(outs)
+                or len({(l.in_features, l.out_features, l.weight.dtype) for l in lins}) != 1
                 or any(q.dtype != x.dtype or tuple(q.shape) != tuple(x.shape) for q in xs)
                 or lins[0].weight.dtype != x.dtype):
             return False

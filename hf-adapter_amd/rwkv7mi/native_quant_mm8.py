@@ -380,6 +380,8 @@ def mm8_rows_multi_into(xs, mods, outs, *, residuals=None, epilogues=None) -> bo
     being captured and the ``"mm8r"`` slot is smaller than the call needs, or an
     operand is not 16-byte aligned."""
     k = len(mods)
+    if not 1 <= k <= 4 or len(xs) != k or len(outs) != k or (residuals is not None and len(residuals) != k):
+        raise ValueError("mm8_rows_multi_into: 1..4 problems, one x, output and residual each")
     rows, n = (int(s) for s in xs[0].shape)
     m = int(mods[0].out_features)
     residuals = list(residuals) if residuals is not None else [None] * k
