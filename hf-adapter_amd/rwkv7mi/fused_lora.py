@@ -20,7 +20,8 @@ ACT_NONE, ACT_TANH, ACT_SIGMOID, ACT_RELU2 = 0, 1, 2, 3
 
 def dense_multi(problems, rows: int, residuals=None):
     """problems: list of (x2 [rows,K], W [N,K], bias or None, y [rows,N], act);
-    ``residuals`` (one ``[rows, N]`` tensor or None each) are added after the activation."""
+    ``residuals`` (None, or one per problem: None or a contiguous tensor of y's
+    device, shape and dtype, y itself among them) are added after the activation."""
     xs = [p[0] for p in problems]
     Ws = [p[1] for p in problems]
     bs = [p[2] for p in problems]
@@ -30,9 +31,16 @@ def dense_multi(problems, rows: int, residuals=None):
     Ks = (ctypes.c_int64 * k)(*[int(p[1].shape[1]) for p in problems])
     acts = (ctypes.c_int * k)(*[int(p[4]) for p in problems])
     _lib.require_gpu(*xs, *Ws, *ys, name="dense_multi")
+    residuals = [None] * k if residuals is None else list(residuals)
+    if len(residuals) != k:
+        raise ValueError("dense_multi: one residual or None per problem")
+    for r, y in zip(residuals, ys):
+        if r is not None and not (r.device == y.device and r.dtype == y.dtype and r.shape == y.shape
+                                  and r.is_contiguous() and y.is_contiguous()):
+            raise ValueError("dense_multi: a residual is contiguous with its output's device, shape and dtype")
     _lib.call("rwkv7mi_dense_multi_residual", _lib.ptr_array(xs), _lib.ptr_array(Ws), _lib.ptr_array(bs),
-              _lib.ptr_array(list(residuals) if residuals is not None else [None] * k), _lib.ptr_array(ys), Ns, Ks, acts,
-              len(problems), int(rows), _lib.dtype_code(xs[0]), _lib.stream_of(xs[0]))
+              _lib.ptr_array(residuals), _lib.ptr_array(ys), Ns, Ks, acts, len(problems), int(rows),
+              _lib.dtype_code(xs[0]), _lib.stream_of(xs[0]))
 
 
 def lora_workspace_bytes(ranks, rows: int, D: int) -> int:

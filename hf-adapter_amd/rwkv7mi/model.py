@@ -194,6 +194,12 @@ def random_weights(cfg: NativeRWKV7Config, *, seed: int = 0, device="cpu", dtype
 
 
 # ------------------------------------------------------------------ linears
+def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether two contiguous tensors share memory."""
+    pa, pb = a.data_ptr(), b.data_ptr()
+    return pa < pb + b.numel() * b.element_size() and pb < pa + a.numel() * a.element_size()
+
+
 class DenseLinear:
     """Unquantised Linear ``y = x W^T`` (projections below the MM8 size
     threshold, and every projection of an unquantised model such as the fp32
@@ -222,12 +228,15 @@ class DenseLinear:
             out.copy_(y)
             return out
         if residual is not None:
-            if residual.dtype != out.dtype or residual.numel() != out.numel():  # torch's promotion / broadcasting
-                tmp = torch.empty_like(out)
+            same = (residual.dtype == out.dtype and residual.shape == out.shape and residual.device == out.device
+                    and out.is_contiguous())
+            residual = residual.contiguous() if same else residual
+            if not same or _overlap(x2, out) or (residual.data_ptr() != out.data_ptr() and _overlap(residual, out)):
+                # torch's promotion, broadcasting, strides and checks; an output over x's memory
+                tmp = torch.empty((rows, self.out_features), dtype=out.dtype, device=out.device)
                 dense_multi([(x2, self.weight, self.bias, tmp, act)], rows)
                 torch.add(residual, tmp, out=out)
                 return out
-            residual = residual.reshape(out.shape).contiguous()
         dense_multi([(x2, self.weight, self.bias, out, act)], rows, [residual])
         return out
 

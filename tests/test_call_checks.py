@@ -34,3 +34,61 @@ def test_dense_group_of_uneven_lists_runs_one_by_one(rows):
     xs = [torch.zeros(rows, 64, dtype=torch.float16)] * 2
     outs = [torch.zeros(rows, 32, dtype=torch.float16)] * 3
     assert DenseLinear.apply_group(lins, xs, outs) is False
+
+
+@pytest.fixture
+def dense_calls(monkeypatch):
+    """The dense products' library calls, recorded instead of run."""
+    from rwkv7mi import _lib, model
+
+    calls = []
+    monkeypatch.setattr(_lib, "require_gpu", lambda *t, name: None)
+    monkeypatch.setattr(_lib, "stream_of", lambda t: 0)
+    monkeypatch.setattr(_lib, "call", lambda name, *args: calls.append(args))
+    return calls
+
+
+def test_dense_multi_refuses_residuals_the_kernel_would_misread(dense_calls):
+    from rwkv7mi.fused_lora import dense_multi
+
+    x, w, y = torch.zeros(4, 64), torch.zeros(32, 64), torch.zeros(4, 32)
+    run = lambda res, out=y, k=1: dense_multi([(x, w, None, out, 0)] * k, 4, res)
+    for bad in (torch.zeros(4, 32, dtype=torch.float16), torch.zeros(1, 32), torch.zeros(32, 4).t(),
+                torch.zeros(4, 32, device="meta")):
+        with pytest.raises(ValueError, match="residual"):
+            run([bad])
+    with pytest.raises(ValueError, match="residual"):
+        run([y], torch.zeros(4, 64)[:, :32])
+    with pytest.raises(ValueError, match="residual"):
+        run([y], k=2)
+    assert not dense_calls
+    run([y])
+    run([None])
+    run(None)
+    assert len(dense_calls) == 3
+
+
+def test_dense_linear_residual_forms_go_through_torch(dense_calls, monkeypatch):
+    """A residual or an output that the kernel's epilogue cannot take is added
+    by torch, which handles strides and refuses another device or a partial
+    overlap; an output over x's memory is not written during the product."""
+    from rwkv7mi.model import DenseLinear
+
+    torch_add, added = torch.add, []
+    monkeypatch.setattr(torch, "add", lambda *a, **k: (added.append(a), torch_add(*a, **k))[1])
+    lin = DenseLinear(torch.zeros(32, 32))
+    x = torch.zeros(4, 32)
+    buf = torch.zeros(5, 32)
+    for out, res in ((torch.zeros(4, 64)[:, :32], torch.ones(4, 32)), (x, torch.ones(4, 32)), (torch.zeros(4, 32),
+                     torch.ones(1, 32))):
+        n = len(added)
+        lin.apply(x, out, residual=res)
+        assert len(added) == n + 1
+    for out, res in ((torch.zeros(4, 32), torch.ones(4, 32, device="meta")), (buf[:4], buf[1:])):
+        with pytest.raises(RuntimeError):
+            lin.apply(torch.zeros(4, 32), out, residual=res)
+    n = len(added)
+    y = torch.zeros(4, 32)
+    lin.apply(x, y, residual=y)
+    lin.apply(x, y, residual=torch.ones(32, 4).t())
+    assert len(added) == n  # in the kernel
