@@ -16,10 +16,11 @@ library GEMMs of dense (unquantised) projections (rocBLAS through torch).
 """
 from __future__ import annotations
 
+import collections
 import contextlib
 import ctypes
-import gc
 import os
+import sys
 import threading
 import weakref
 import zlib
@@ -1727,25 +1728,45 @@ class _LazyWeights(dict):
 
 
 # ------------------------------------------------------------------ graph runner
+# Graphs of runners that are gone, kept until no stream captures
+_dead_graphs: collections.deque = collections.deque()
 _captures = 0
-_captures_lock = threading.Lock()
-_gc_was_on = False
+_captures_lock = threading.RLock()  # (reentrant: the collector may run a runner's __del__ inside it)
+
+
+def _drop_graphs() -> None:
+    """Destroy the dead runners' graphs unless a capture is under way (on this
+    thread's stream, or a :func:`graph_capture` of any thread)."""
+    with _captures_lock:
+        while _dead_graphs and not _captures and not torch.cuda.is_current_stream_capturing():
+            _dead_graphs.popleft()
+
+
+class _OwnsGraph:
+    """A runner whose graph outlives it until it can be destroyed.
+
+    Destroying a graph waits for the device, which is an error while a stream is
+    capturing, and the error leaves a C++ destructor: the process aborts.  A model
+    and its runners are a reference cycle, so the collector may come upon a
+    dropped one at any time, in the middle of a capture too; its graph then
+    waits for the capture's end."""
+
+    graph = None
+
+    def __del__(self):
+        graph, self.graph = self.graph, None
+        if graph is not None and not sys.is_finalizing():
+            _dead_graphs.append(graph)
+            del graph
+            _drop_graphs()
 
 
 @contextlib.contextmanager
 def graph_capture(graph):
-    """``torch.cuda.graph(graph)`` with the cyclic collector off.
-
-    A dropped model and its runners are a reference cycle, so their graphs are
-    destroyed whenever the collector happens to run.  Destroying one waits for
-    the device, which is an error while a stream is capturing, and the error
-    leaves a C++ destructor: the process aborts.  What became garbage is
-    collected as usual after the capture."""
-    global _captures, _gc_was_on
+    """``torch.cuda.graph(graph)``, during which no dead runner's graph is
+    destroyed on any thread."""
+    global _captures
     with _captures_lock:
-        if _captures == 0:
-            _gc_was_on = gc.isenabled()
-            gc.disable()
         _captures += 1
     try:
         with torch.cuda.graph(graph):
@@ -1753,11 +1774,10 @@ def graph_capture(graph):
     finally:
         with _captures_lock:
             _captures -= 1
-            if _captures == 0 and _gc_was_on:
-                gc.enable()
+        _drop_graphs()
 
 
-class NativeGraphRunner:
+class NativeGraphRunner(_OwnsGraph):
     """hipGraph-captured decode step for a fixed batch (rwkv7_hf/native_graph_runtime.py:212-711).
 
     The runner owns static cache tensors; ``replay`` copies a foreign cache in
@@ -1878,7 +1898,7 @@ class NativeGraphRunner:
         return self.next_tokens
 
 
-class NativePrefillGraphRunner:
+class NativePrefillGraphRunner(_OwnsGraph):
     """hipGraph-captured prefill for one shape ``(B, T, logits_to_keep)``
     (rwkv7_hf/model_prefill_graph.py:38-381): the whole layer stack of
     :meth:`NativeRWKV7ForCausalLM.prefill_` — embedding, mixes, MM8 GEMMs,
