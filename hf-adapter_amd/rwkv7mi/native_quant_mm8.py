@@ -745,7 +745,10 @@ class MM8Linear(torch.nn.Module):
         rows = x2.shape[0]
         out2 = torch.empty((rows, m), device=x.device, dtype=x.dtype) if out is None else out.reshape(rows, m)
         bufs = self._buffers
-        w, mx, rx, my, ry = bufs["w_blk"], bufs["mx"], bufs["rx"], bufs["my"], bufs["ry"]
+        try:  # (a module attribute that is looked up by name costs more than the rest of this function)
+            w, mx, rx, my, ry = bufs["w_blk"], bufs["mx"], bufs["rx"], bufs["my"], bufs["ry"]
+        except KeyError:  # some of them reassigned as parameters
+            w, mx, rx, my, ry = self.w_blk, self.mx, self.rx, self.my, self.ry
         bias = self.bias
         blocked = (rows > 0 and is_blocked(w) and w.shape[0] == (m + 15) // 16 and w.shape[1] == (n + 127) // 128
                    and ry.numel() == n and mx.numel() == m)

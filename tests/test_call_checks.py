@@ -92,3 +92,19 @@ def test_dense_linear_residual_forms_go_through_torch(dense_calls, monkeypatch):
     lin.apply(x, y, residual=y)
     lin.apply(x, y, residual=torch.ones(32, 4).t())
     assert len(added) == n  # in the kernel
+
+
+@pytest.mark.parametrize("name", ["w_blk", "mx", "ry"])
+def test_mm8_linear_reads_its_tensors_where_they_are(monkeypatch, name):
+    """A module whose packed tensors were reassigned as parameters runs."""
+    from rwkv7mi import _lib, native_quant_mm8 as Q
+
+    seen = []
+    monkeypatch.setattr(_lib, "require_gpu", lambda *t, name: None)
+    monkeypatch.setattr(Q, "_linear_into", lambda *a: seen.append(a) or True)
+    b = _blocked(128, 32)
+    mod = Q.MM8Linear.from_packed(b.w_blk, b.mx, b.rx, b.my, b.ry, 128, 32)
+    setattr(mod, name, torch.nn.Parameter(getattr(mod, name), requires_grad=False))
+    mod(torch.zeros(4, 128, dtype=torch.float16))
+    for got, want in zip(seen[0][1:6], ("w_blk", "mx", "rx", "my", "ry")):
+        assert got is getattr(mod, want)
