@@ -789,26 +789,30 @@ class MM8Linear(torch.nn.Module):
         res = residual.reshape(*hidden.shape[:-1], down.out_features).contiguous()
         return down._run(hidden, residual=res, epilogue=_lib.EPI_RESIDUAL)
 
-    def _workspace_slot(self, rows: int):
-        rows = int(rows)
+    def _workspace_slots(self, rows: int):
+        """(slot, bytes) of every form that a ``rows``-row call may run on, the usual one first."""
+        rows, n, m = int(rows), self.in_features, self.out_features
         if GEMV_ROWS < rows <= GEMM_ROWS:
-            return "mm8g", mm8_gemm_workspace_bytes(1, rows, self.in_features, self.out_features)
+            # (other activation types than the metadata's and unaligned operands stay on the tile GEMM)
+            mid = mm8_rows_reserve_bytes(1, rows, n, m, self.mx.dtype)
+            return ([("mm8r", mid)] if mid else []) + [("mm8g", mm8_gemm_workspace_bytes(1, rows, n, m))]
         if 0 < rows <= GEMV_ROWS:
-            return "mm8t", mm8t_workspace_bytes(1, rows, self.in_features, self.out_features)
-        return None, 0
+            return [("mm8t", mm8t_workspace_bytes(1, rows, n, m))]
+        return [(None, 0)]
 
     def rwkv7_workspace_bytes(self, rows: int) -> int:
         """Scratch bytes a ``rows``-row call needs: the fused GEMV's split-K
         partials (``"mm8t"`` slot, only when the rows' x' exceeds one LDS chunk)
-        up to GEMV_ROWS rows, the tile GEMM's x', row sums and split partials
-        (``"mm8g"`` slot) from GEMV_ROWS + 1 to GEMM_ROWS rows."""
-        return self._workspace_slot(rows)[1]
+        up to GEMV_ROWS rows; from GEMV_ROWS + 1 to GEMM_ROWS rows x', row sums
+        and split partials of the tile GEMM (``"mm8g"`` slot) or, where it is
+        the faster one, of the middle-row kernel (``"mm8r"`` slot)."""
+        return self._workspace_slots(rows)[0][1]
 
     def rwkv7_reserve_workspace(self, rows: int) -> None:
-        """Grow the slot a ``rows``-row call uses (call before graph capture)."""
-        slot, need = self._workspace_slot(rows)
-        if need:
-            _ws.reserve(self.w_blk.device, need, slot=slot)
+        """Grow the slots a ``rows``-row call may use (call before graph capture)."""
+        for slot, need in self._workspace_slots(rows):
+            if need:
+                _ws.reserve(self.w_blk.device, need, slot=slot)
 
     def extra_repr(self):
         return f"in={self.in_features}, out={self.out_features}, mm8(fused={self.fused}, hip=gfx950)"

@@ -108,3 +108,24 @@ def test_mm8_linear_reads_its_tensors_where_they_are(monkeypatch, name):
     mod(torch.zeros(4, 128, dtype=torch.float16))
     for got, want in zip(seen[0][1:6], ("w_blk", "mx", "rx", "my", "ry")):
         assert got is getattr(mod, want)
+
+
+def test_mm8_reserve_hook_grows_the_slots_a_call_uses(monkeypatch):
+    """4096 -> 8192 (2^25 weights): above 64 rows the middle-row kernel and its
+    own slot, the tile GEMM's beside it for calls that stay on that one."""
+    from rwkv7mi import native_quant_mm8 as Q
+
+    grown = {}
+    monkeypatch.setattr(Q._ws, "reserve", lambda device, need, slot, **k: grown.__setitem__(slot, need))
+    n, m = 4096, 8192
+    b = _blocked(n, m)
+    mod = Q.MM8Linear.from_packed(b.w_blk, b.mx, b.rx, b.my, b.ry, n, m)
+    for rows in (17, 64, 65, 256):
+        grown.clear()
+        mod.rwkv7_reserve_workspace(rows)
+        form, need = Q._linear_plan(rows, n, m, Q._lib.F16, 0)[:2]
+        assert (form == 2) == (rows > 64)
+        assert grown[Q._FORM_SLOT[form]] == need == mod.rwkv7_workspace_bytes(rows)
+        assert grown["mm8g"] == Q.mm8_gemm_workspace_bytes(1, rows, n, m)
+    mod.mx = mod.mx.float()  # fp32 metadata: fp32 activations, the tile GEMM
+    assert mod.rwkv7_workspace_bytes(100) == Q.mm8_gemm_workspace_bytes(1, 100, n, m)
