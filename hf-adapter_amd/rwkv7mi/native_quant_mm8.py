@@ -374,6 +374,15 @@ def mm8_rows_reserve_bytes(nprob: int, rows: int, n: int, m: int, dtype: torch.d
     return mm8_rows_workspace_bytes(nprob, rows, n, m)
 
 
+def _other_slot(nprob: int, rows: int, n: int, m: int):
+    """(slot, bytes) of the form that a middle-row call falls back to.  Eager
+    calls grow it too, so that one of them readies a capture at other row counts
+    (which may run that form), as it did when it was the only one."""
+    if rows > GEMM_ROWS:
+        return "mm8p", mm8_prefill_workspace_bytes(nprob, n, m)
+    return "mm8g", mm8_gemm_workspace_bytes(nprob, rows, n, m)
+
+
 def mm8_rows_multi_into(xs, mods, outs, *, residuals=None, epilogues=None) -> bool:
     """:func:`mm8_gemm_multi_into` for middle row counts (fp16 / bf16): the
     128-row x 256-column tile kernel.  False, with nothing run, when a graph is
@@ -396,6 +405,8 @@ def mm8_rows_multi_into(xs, mods, outs, *, residuals=None, epilogues=None) -> bo
     if any(t.data_ptr() % 16 for t in (*xs, *(t for md in mods for t in (md.w_blk, md.my, md.ry)))):
         return False
     need = mm8_rows_workspace_bytes(k, rows, n, m)
+    slot, other = _other_slot(k, rows, n, m)
+    _ws.reserve(xs[0].device, other, slot=slot, floor=0)
     ws = _ws.reserve(xs[0].device, need, slot="mm8r", floor=0)
     if ws is None or int(ws.numel()) < need:
         return False
@@ -428,12 +439,13 @@ _FORM_SLOT = ("mm8t", "mm8g", "mm8r", "mm8p")
 
 @functools.lru_cache(maxsize=4096)
 def _linear_plan(rows: int, n: int, m: int, dt: int, device: int):
-    """(form, workspace bytes, least workspace) of one product: the sizes and
-    the device's CU count alone decide."""
+    """(form, workspace bytes, least workspace, :func:`_other_slot` of the
+    middle-row form) of one product: the sizes and the device's CU count alone
+    decide."""
     need = ctypes.c_int64(0)
     form = int(_lib.load().rwkv7mi_mm8t_linear_plan(rows, n, m, dt, ctypes.byref(need)))
     floor = mm8_prefill_workspace_bytes(1, n, m) if form == 3 else int(need.value)
-    return form, int(need.value), floor
+    return form, int(need.value), floor, _other_slot(1, rows, n, m) if form == 2 else None
 
 
 def _linear_into(x2, w, mx, rx, my, ry, bias, residual, out, epilogue) -> bool:
@@ -448,13 +460,15 @@ def _linear_into(x2, w, mx, rx, my, ry, bias, residual, out, epilogue) -> bool:
     rows, n = x2.shape
     m = out.shape[1]
     dt = _lib.dtype_code(x2)
-    form, need, floor = _linear_plan(rows, n, m, dt, x2.get_device())
+    form, need, floor, other = _linear_plan(rows, n, m, dt, x2.get_device())
     if form >= 2:
         if form == 3 and (dt == _lib.F32 or mx.dtype != x2.dtype or rows * n * 2 > _PREFILL_MAX_BYTES):
             return False
         if form == 2 and (x2.data_ptr() | w.data_ptr() | my.data_ptr() | ry.data_ptr()) & 15:
             return False
     ws, have = None, 0
+    if other is not None:
+        _ws.reserve(x2.device, other[1], other[0], floor=0)
     if need:
         ws = _ws.reserve(x2.device, need, _FORM_SLOT[form], floor=0 if form == 2 else floor)
         have = 0 if ws is None else ws.numel()

@@ -129,3 +129,32 @@ def test_mm8_reserve_hook_grows_the_slots_a_call_uses(monkeypatch):
         assert grown["mm8g"] == Q.mm8_gemm_workspace_bytes(1, rows, n, m)
     mod.mx = mod.mx.float()  # fp32 metadata: fp32 activations, the tile GEMM
     assert mod.rwkv7_workspace_bytes(100) == Q.mm8_gemm_workspace_bytes(1, 100, n, m)
+
+
+@pytest.mark.parametrize("rows,slot", [(200, "mm8g"), (300, "mm8p")])
+@pytest.mark.parametrize("route", ["one", "many"])
+def test_mm8_middle_rows_ready_a_capture_at_other_row_counts(monkeypatch, rows, slot, route):
+    """An eager call grows the slot of the form beside it: a graph captured
+    later at 64 or 1500 rows runs that form and cannot grow it itself."""
+    from rwkv7mi import _lib, native_quant_mm8 as Q
+
+    grown = {}
+
+    def reserve(device, need, slot="mm8", **k):
+        grown[slot] = need
+        return torch.empty(need, dtype=torch.uint8, device="meta")
+
+    monkeypatch.setattr(Q._ws, "reserve", reserve)
+    monkeypatch.setattr(_lib, "require_gpu", lambda *t, name: None)
+    monkeypatch.setattr(_lib, "stream_of", lambda t: 0)
+    monkeypatch.setattr(_lib, "call", lambda *a: None)
+    n, m = 4096, 8192
+    b = _blocked(n, m)
+    x, y = torch.zeros(rows, n, dtype=torch.float16), torch.zeros(rows, m, dtype=torch.float16)
+    if route == "one":
+        assert Q._linear_into(x, b.w_blk, b.mx, b.rx, b.my, b.ry, None, None, y, 0)
+    else:
+        Q.mm8_many_rows_into([x], [b], [y])
+    assert "mm8r" in grown
+    want = Q.mm8_gemm_workspace_bytes(1, rows, n, m) if slot == "mm8g" else Q.mm8_prefill_workspace_bytes(1, n, m)
+    assert grown[slot] == want
