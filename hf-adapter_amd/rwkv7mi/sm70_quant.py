@@ -8,6 +8,8 @@ only.
 """
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from . import _lib
@@ -35,13 +37,19 @@ def quantize_w4_groupwise(weight: torch.Tensor, group_size: int = 128):
     return packed, scales, in_features
 
 
+@functools.lru_cache(maxsize=4096)
+def _w4_scratch(rows: int, out_features: int, in_features: int, group_size: int, affine: int, dt: int, device: int):
+    """Scratch bytes of one product (the sizes and the device's CU count alone
+    decide): a library call of 1 us that a small product's host time would show."""
+    return int(_lib.load().rwkv7mi_w4_workspace_bytes(rows, out_features, in_features, group_size, affine, dt))
+
+
 def _w4_call(x2, q, scales, biases, bias, residual, out2, rows, out_features, in_features, group_size, epilogue):
     """The W4 product (``biases`` None: symmetric).  The K splits of many rows
     keep their partials in a buffer of this call's own: calls on several streams
     never share one."""
     dt = _lib.dtype_code(x2)
-    need = int(_lib.load().rwkv7mi_w4_workspace_bytes(rows, out_features, in_features, group_size,
-                                                      int(biases is not None), dt))
+    need = _w4_scratch(rows, out_features, in_features, group_size, int(biases is not None), dt, x2.get_device())
     ws = torch.empty(need, dtype=torch.uint8, device=x2.device) if need else None
     _lib.call("rwkv7mi_w4_matmul_ws", _lib.ptr(x2), _lib.ptr(q), _lib.ptr(scales), _lib.ptr(biases), _lib.ptr(bias),
               _lib.ptr(residual), _lib.ptr(out2), rows, out_features, in_features, group_size, int(epilogue), dt,

@@ -158,3 +158,30 @@ def test_mm8_middle_rows_ready_a_capture_at_other_row_counts(monkeypatch, rows, 
     assert "mm8r" in grown
     want = Q.mm8_gemm_workspace_bytes(1, rows, n, m) if slot == "mm8g" else Q.mm8_prefill_workspace_bytes(1, n, m)
     assert grown[slot] == want
+
+
+def test_w4_asks_for_its_scratch_once_a_shape(monkeypatch):
+    """One library call a product: the size query is kept by the sizes."""
+    from rwkv7mi import _lib, sm70_quant as W
+
+    asked, calls = [], []
+
+    class Lib:
+        @staticmethod
+        def rwkv7mi_w4_workspace_bytes(*a):
+            asked.append(a)
+            return 0
+
+    monkeypatch.setattr(_lib, "require_gpu", lambda *t, name: None)
+    monkeypatch.setattr(_lib, "stream_of", lambda t: 0)
+    monkeypatch.setattr(_lib, "load", lambda: Lib)
+    monkeypatch.setattr(_lib, "call", lambda *a: calls.append(a))
+    x, q, s = torch.zeros(3, 256), torch.zeros(48, 128, dtype=torch.uint8), torch.zeros(48, 2)
+    W._w4_scratch.cache_clear()
+    try:
+        for _ in range(5):
+            W.w4_groupwise_linear(x, q, s, 48, 256)
+        W.w4_affine_groupwise_linear(x, q, s, s, 48, 256)
+    finally:
+        W._w4_scratch.cache_clear()  # (filled by the stand-in library)
+    assert len(calls) == 6 and [a[4] for a in asked] == [0, 1]
