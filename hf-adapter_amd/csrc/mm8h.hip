@@ -45,6 +45,7 @@
 //    The tile order is XCD-aware: a workgroup's linear id L runs on XCD L % 8,
 //    so tiles are numbered to give each XCD contiguous groups of 4 row tiles x
 //    8 column tiles (their x rows and weight columns stay in that XCD's L2).
+#include <algorithm>
 #include <string>
 
 #include "dense_common.h"
@@ -497,22 +498,63 @@ extern "C" int64_t rwkv7mi_mm8t_gemm_prefill_ws_bytes(int nprob, int64_t I, int6
 }
 
 namespace rwkv7mi {
-// K splits of a launch of `tiles` 256 x 256 tiles (over all problems) with SB
-// steps: fewer than one tile per CU leaves CUs idle, so K is cut into equal
-// ranges while tiles x splits <= 256.  The estimate, in us: 1.1 per step with
-// the chip nearly idle, 1.66 with every CU streaming (measured: 16384 -> 4096
-// at 1000 rows, 64 tiles, 289 us for 256 steps; 4096 -> 16384, 256 tiles, 107
-// us for 64), and the fp32 partials (part_bytes a split) written and read back
-// at about 4 TB/s plus a launch.
-static int mh_splits(int64_t tiles, int64_t I, int64_t part_bytes, double* us = nullptr) {
+// The launch's tile grid: gm x gn XCD groups, padded to whole groups.
+struct MhGrid {
+  int64_t mt, nt, gm, gn, T, per;
+};
+static MhGrid mh_grid(int64_t rows, int64_t O) {
+  MhGrid g;
+  g.mt = (rows + MH_M - 1) / MH_M;
+  g.nt = (O + MH_N - 1) / MH_N;
+  g.gm = std::min<int64_t>(g.mt, 4);
+  g.gn = std::min<int64_t>(g.nt, 8);
+  g.T = (g.mt + g.gm - 1) / g.gm * g.gm * ((g.nt + g.gn - 1) / g.gn) * g.gn;
+  g.per = (g.T + 7) / 8;
+  return g;
+}
+// real tiles of one problem on each XCD (mm8h_gemm_kernel's order)
+static void mh_xcd_tiles(const MhGrid& g, int (&n)[8]) {
+  for (int x = 0; x < 8; ++x) n[x] = 0;
+  int x = 0;
+  int64_t left = g.per;
+  for (int64_t m0 = 0; m0 < g.mt; m0 += g.gm)
+    for (int64_t n0 = 0; n0 < g.nt; n0 += g.gn)
+      for (int64_t m = m0; m < m0 + g.gm; ++m)
+        for (int64_t c = n0; c < n0 + g.gn; ++c, --left) {
+          if (left == 0) ++x, left = g.per;
+          n[x] += m < g.mt && c < g.nt;
+        }
+}
+// K splits of a launch: fewer than one tile per CU leaves CUs idle, so K is cut
+// into equal ranges while tiles x splits <= 256.  The estimate, in us: rounds of
+// 32 workgroups on the fullest XCD (a grid that does not fill its groups loads
+// the XCDs unevenly) x the steps, 1.1 each with the chip nearly idle, 1.66 with
+// every CU streaming (measured: 16384 -> 4096 at 1000 rows, 64 tiles, 289 us for
+// 256 steps; 4096 -> 16384, 256 tiles, 107 us for 64), and the fp32 partials
+// written and read back at about 4 TB/s plus a launch.  Without the XCDs'
+// loads 10240 -> 2560 at 2500 rows (100 tiles, 24 on one XCD) ran in two splits,
+// 262 us against 203 unsplit, and 8192 -> 2048 at 1025 rows (40 tiles, 8 on each
+// of five XCDs) in five, 114 us, where four are one round, 84.6.
+static int mh_splits(int64_t nprob, int64_t rows, int64_t I, int64_t O, double* us = nullptr) {
   const int64_t SB = (I + 63) / 64;
+  const MhGrid g = mh_grid(rows, O);
+  const int64_t tiles = nprob * g.mt * g.nt;
+  const double pb = (double)nprob * rows * ((O + 31) / 32 * 32) * 4;
+  if (tiles > 256) {
+    if (us) *us = (tiles + 255) / 256 * (SB + 6) * 1.66;
+    return 1;
+  }
+  int n[8];
+  mh_xcd_tiles(g, n);
+  const int64_t most = nprob * *std::max_element(n, n + 8);
   int best = 1;
   double cost = 1e30;
   for (int S = 1; S <= 16 && (S == 1 || tiles * S <= 256); ++S) {
     const int64_t sps = (SB + S - 1) / S;
     if (S > 1 && (I % 64 || sps < 4 || (SB + sps - 1) / sps != S)) continue;  // no empty split
-    const double t = (tiles * S + 255) / 256 * (sps + 6) * (1.1 + 0.56 * std::min<double>(1.0, tiles * S / 256.0)) +
-                     (S > 1 ? 5.0 + 2.0 * part_bytes * S / 4e6 : 0.0);
+    const int64_t rounds = (most * S + 31) / 32;
+    const double busy = (double)tiles * S / (256.0 * rounds);
+    const double t = rounds * (sps + 6) * (1.1 + 0.56 * busy) + (S > 1 ? 5.0 + 2.0 * pb * S / 4e6 : 0.0);
     if (t < cost) cost = t, best = S;
   }
   if (us) *us = cost;
@@ -532,25 +574,24 @@ static int mh_gemm_launch(MhBatch& b, int nprob, int64_t rows, int64_t I, int64_
   b.I = (int)I;
   b.O = (int)O;
   b.SB = (int)((I + 63) / 64);
-  b.mt = (int)((rows + MH_M - 1) / MH_M);
-  b.nt = (int)((O + MH_N - 1) / MH_N);
-  b.gm = std::min(b.mt, 4);
-  b.gn = std::min(b.nt, 8);
-  const int64_t T = (int64_t)((b.mt + b.gm - 1) / b.gm) * b.gm * ((b.nt + b.gn - 1) / b.gn) * b.gn;
-  if (T > (int64_t)INT32_MAX / 2) return fail(RWKV7MI_EINVAL, w + ": too many tiles");
-  const int64_t per = (T + 7) / 8;
+  const MhGrid grid = mh_grid(rows, O);
+  if (grid.T > (int64_t)INT32_MAX / 2) return fail(RWKV7MI_EINVAL, w + ": too many tiles");
+  b.mt = (int)grid.mt;
+  b.nt = (int)grid.nt;
+  b.gm = (int)grid.gm;
+  b.gn = (int)grid.gn;
   // partials follow the weights in the workspace (a caller that gave only the
   // weights' bytes gets no splits)
   b.ldp = (O + 31) / 32 * 32;
   const int64_t wb = mh_weight_bytes(nprob, I, O), pb = mh_part_bytes(nprob, rows, O);
-  b.S = mh_splits(mh_tiles(nprob, rows, O), I, pb);
+  b.S = mh_splits(nprob, rows, I, O);
   if (ws_bytes < wb + (b.S > 1 ? b.S * pb : 0)) b.S = 1;
   b.sps = (b.SB + b.S - 1) / b.S;
   b.part = reinterpret_cast<float*>(static_cast<char*>(ws) + wb);
   auto launch = [&](auto kern, std::atomic<uint64_t>& raised) {
     if (int rc = raise_dynamic_lds(reinterpret_cast<const void*>(kern), MH_LDS, raised, "mm8h_gemm_kernel"))
       return rc;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(per * 8), (unsigned)nprob, (unsigned)b.S), dim3(MH_THREADS), MH_LDS,
+    hipLaunchKernelGGL(kern, dim3((unsigned)(grid.per * 8), (unsigned)nprob, (unsigned)b.S), dim3(MH_THREADS), MH_LDS,
                        as_stream(stream), b);
     if (int rc = check_launch("mm8h_gemm_kernel")) return rc;
     if (b.S == 1) return (int)RWKV7MI_OK;
@@ -566,7 +607,7 @@ static int mh_gemm_launch(MhBatch& b, int nprob, int64_t rows, int64_t I, int64_
 
 double mm8h_estimate_us(int64_t nprob, int64_t rows, int64_t I, int64_t O) {
   double us = 0;
-  mh_splits(mh_tiles(nprob, rows, O), I, mh_part_bytes(nprob, rows, O), &us);
+  mh_splits(nprob, rows, I, O, &us);
   return us + 4.0 + 3.0 * nprob * I * O / 4.8e6;  // + the dequantisation
 }
 
@@ -575,7 +616,7 @@ double mm8h_estimate_us(int64_t nprob, int64_t rows, int64_t I, int64_t O) {
 extern "C" int64_t rwkv7mi_mm8t_gemm_prefill_split_ws_bytes(int nprob, int64_t rows, int64_t I, int64_t O) {
   if (nprob < 1 || rows <= 0 || I <= 0 || O <= 0) return 0;
   const int64_t pb = mh_part_bytes(nprob, rows, O);
-  const int S = mh_splits(mh_tiles(nprob, rows, O), I, pb);
+  const int S = mh_splits(nprob, rows, I, O);
   return mh_weight_bytes(nprob, I, O) + (S > 1 ? S * pb : 0);
 }
 

@@ -1,0 +1,52 @@
+"""Dispatch rules that the library answers on the host: each is held to a model
+of its launch and to the points at which both sides were measured."""
+from __future__ import annotations
+
+import pytest
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from rwkv7mi import _lib
+
+    return _lib.load()
+
+
+def _cd(a, b):
+    return -(-a // b)
+
+
+def _prefill_splits(lib, k, rows, I, O):
+    part = lib.rwkv7mi_mm8t_gemm_prefill_split_ws_bytes(k, rows, I, O) - lib.rwkv7mi_mm8t_gemm_prefill_ws_bytes(k, I, O)
+    return max(1, part // (k * rows * _cd(O, 32) * 32 * 4))
+
+
+def _fullest_xcd(rows, O):
+    """256 x 256 tiles on the fullest of the eight XCDs: groups of 4 x 8 tiles,
+    padded to whole groups, each XCD a contiguous eighth of their order."""
+    mt, nt = _cd(rows, 256), _cd(O, 256)
+    gm, gn = min(mt, 4), min(nt, 8)
+    order = [(m, c) for m0 in range(0, mt, gm) for c0 in range(0, nt, gn)
+             for m in range(m0, m0 + gm) for c in range(c0, c0 + gn)]
+    per = _cd(len(order), 8)
+    return max(sum(m < mt and c < nt for m, c in order[x * per:(x + 1) * per]) for x in range(8))
+
+
+@pytest.mark.parametrize("k", [1, 2, 3])
+@pytest.mark.parametrize("I,O", [(8192, 2048), (2048, 2048), (10240, 2560), (2560, 2560), (16384, 4096), (4096, 4096),
+                                 (4096, 1000), (3072, 768), (2560, 10240)])
+def test_prefill_splits_shorten_the_fullest_xcd(lib, k, I, O):
+    """A K split is taken where the steps that the fullest XCD's CUs run one
+    after the other fall by a sixth or more; 32 CUs an XCD."""
+    steps = I // 64
+    for rows in (257, 300, 513, 768, 1025, 1100, 1281, 1500, 1537, 2304, 2500, 3000, 3072, 4000, 6000):
+        S = _prefill_splits(lib, k, rows, I, O)
+        if S > 1:
+            most = k * _fullest_xcd(rows, O)
+            assert _cd(most * S, 32) * _cd(steps, S) <= 5 / 6 * _cd(most, 32) * steps, (rows, S)
+
+
+def test_prefill_splits_at_measured_points(lib):
+    assert _prefill_splits(lib, 1, 2500, 10240, 2560) == 1  # 262 us in two, 199 in one
+    assert _prefill_splits(lib, 1, 1025, 8192, 2048) == 4   # 114 us in five (two rounds), 84.6 in four
+    assert _prefill_splits(lib, 1, 1100, 4096, 4096) == 2   # 104.6 us in three, 83.8 in two
