@@ -597,7 +597,11 @@ __global__ __launch_bounds__(512, 1) void mm8r_kernel(const Mm8gBatch B) {
 }
 
 // K splits of the middle-row kernel: rounds of 256 workgroups (one a CU) against
-// the partials' traffic
+// the partials' traffic.  Unsplit the workgroup ends with its own epilogue, whose
+// loads wait for the stores between them, and the pre-pass is not hidden: 30 us
+// beside 1.5 a block (measured, us: 2048 -> 8192, 16 blocks, 128 workgroups 54,
+// 256 62; 4096 -> 16384, 32 blocks, 192 workgroups 76, 256 84-89; three 2048 ->
+// 2048 at 1000 rows 64), split 2.2 a block with the pre-pass and the reduce in it.
 static int mm8r_splits(int nprob, int64_t rows, int64_t I, int64_t O, double* us = nullptr) {
   const int64_t KB = (I + 127) / 128;  // two steps each
   const int64_t tiles = nprob * ((rows + MM8R_ROWS - 1) / MM8R_ROWS) * ((O + MM8R_COLS - 1) / MM8R_COLS);
@@ -607,7 +611,8 @@ static int mm8r_splits(int nprob, int64_t rows, int64_t I, int64_t O, double* us
   for (int S = 1; S <= 32 && (S == 1 || tiles * S <= 256); ++S) {
     const int64_t bps = (KB + S - 1) / S;
     if (S > 1 && (bps < 2 || (KB + bps - 1) / bps != S)) continue;  // no empty split
-    const double t = ((tiles * S + 255) / 256) * (4.0 + 2.2 * bps) + (S > 1 ? 4.0 + 2.0 * pb * S / 4e6 : 0.0);
+    const double t = S == 1 ? (tiles + 255) / 256 * (30.0 + 1.5 * bps) + 4.0 * nprob * rows * I / 4e6
+                            : 8.0 + 2.2 * bps + 2.0 * pb * S / 4e6;
     if (t < cost) cost = t, best = S;
   }
   if (us) *us = cost;
@@ -823,8 +828,9 @@ extern "C" int rwkv7mi_mm8t_gemm_multi_lora(int nprob, const void* const* x, con
 // rows 61 -> 61, so only where one product has 2^25 weights.  Against the
 // dequantise + GEMM form (300 / 600 / 1000 / 1500 / 2500 rows): 232 -> 149, 287
 // -> 247, 353 -> 312, 536 -> 526, 770 -> 875 at 7.2B widths, 107 -> 87, 128 ->
-// 100, 142 -> 116, 167 -> 186, 292 -> 309 at 2048; there by the two estimates
-// (that form's runs about a tenth high) up to 1024 rows.
+// 100, 142 -> 116, 167 -> 186, 292 -> 309 at 2048;
+// there by the two estimates up to 1024 rows (three 2048 -> 2048 at 1000 rows 59
+// on that form, 64 here).
 extern "C" int rwkv7mi_mm8t_rows_pays(int nprob, int64_t rows, int64_t I, int64_t O, int act_dtype) {
   if (nprob < 1 || nprob > MM8T_MAXPROB || rows <= 64 || I <= 0 || O <= 0 || act_dtype == RWKV7MI_F32) return 0;
   if (I % 16 || I > (1 << 22) || O > (1 << 24) || rows * std::max(I, O) > INT32_MAX) return 0;
@@ -832,7 +838,7 @@ extern "C" int rwkv7mi_mm8t_rows_pays(int nprob, int64_t rows, int64_t I, int64_
   if (rows > 1024) return 0;
   double us = 0;
   mm8r_splits(nprob, rows, I, O, &us);
-  return us + 5.0 < 0.9 * mm8h_estimate_us(nprob, rows, I, O);
+  return us < 0.95 * mm8h_estimate_us(nprob, rows, I, O);
 }
 // workspace: x' | row sums | row scales | partials, each part 256-byte aligned
 struct Mm8rWs {

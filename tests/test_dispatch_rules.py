@@ -50,3 +50,19 @@ def test_prefill_splits_at_measured_points(lib):
     assert _prefill_splits(lib, 1, 2500, 10240, 2560) == 1  # 262 us in two, 199 in one
     assert _prefill_splits(lib, 1, 1025, 8192, 2048) == 4   # 114 us in five (two rounds), 84.6 in four
     assert _prefill_splits(lib, 1, 1100, 4096, 4096) == 2   # 104.6 us in three, 83.8 in two
+
+
+@pytest.mark.parametrize("k,rows,I,O,pays", [
+    (3, 1000, 2048, 2048, 0),    # 64 us, 58 on the dequantised weight
+    (3, 512, 2048, 2048, 1), (1, 1000, 2048, 8192, 1), (1, 768, 16384, 4096, 1), (3, 600, 4096, 4096, 1),
+    (1, 600, 4096, 16384, 0),    # two rounds of its tiles
+])
+def test_middle_row_kernel_against_the_prefill_gemm(lib, k, rows, I, O, pays):
+    """Above 256 rows by the two estimates; an unsplit launch is priced with its own epilogue and pre-pass."""
+    assert lib.rwkv7mi_mm8t_rows_pays(k, rows, I, O, 1) == pays
+
+
+def test_middle_row_kernel_splits_before_it_runs_an_epilogue(lib):
+    """2048 -> 8192 at 512 rows: 53.7 us unsplit, 41.8 in two K ranges."""
+    x = 512 * 2048 * 2 + 512 * 16
+    assert lib.rwkv7mi_mm8t_rows_workspace_bytes(1, 512, 2048, 8192) >= x + 2 * 512 * 8192 * 4
