@@ -825,16 +825,18 @@ extern "C" int rwkv7mi_mm8t_gemm_multi_lora(int nprob, const void* const* x, con
 // Whether these rows run faster on it.  Measured (key + value of an FFN, kernel
 // time, us): against mm8g_kernel at 7.2B widths (4096 / 16384) 64 rows 64 -> 66,
 // 100 rows 88 -> 76, 200 rows 147 -> 101; at 2048 / 8192 100 rows 45 -> 50, 200
-// rows 61 -> 61, so only where one product has 2^25 weights.  Against the
-// dequantise + GEMM form (300 / 600 / 1000 / 1500 / 2500 rows): 232 -> 149, 287
-// -> 247, 353 -> 312, 536 -> 526, 770 -> 875 at 7.2B widths, 107 -> 87, 128 ->
-// 100, 142 -> 116, 167 -> 186, 292 -> 309 at 2048;
+// rows 61 -> 61, so only where one product has 2^25 weights, and up to 128 rows
+// (two full tiles of mm8g_kernel) 5 x 2^23 (one product, 128 rows: 8192 -> 4096
+// 28.5 -> 31.0, 4096 -> 8192 29.6 -> 32.2, 10240 -> 4096 43.9 -> 34.9; 129 rows 38.8
+// -> 33.0, 40.3 -> 33.1).  Against the dequantise + GEMM form (300 / 600 / 1000 /
+// 1500 / 2500 rows): 232 -> 149, 287 -> 247, 353 -> 312, 536 -> 526, 770 -> 875 at
+// 7.2B widths, 107 -> 87, 128 -> 100, 142 -> 116, 167 -> 186, 292 -> 309 at 2048;
 // there by the two estimates up to 1024 rows (three 2048 -> 2048 at 1000 rows 59
 // on that form, 64 here).
 extern "C" int rwkv7mi_mm8t_rows_pays(int nprob, int64_t rows, int64_t I, int64_t O, int act_dtype) {
   if (nprob < 1 || nprob > MM8T_MAXPROB || rows <= 64 || I <= 0 || O <= 0 || act_dtype == RWKV7MI_F32) return 0;
   if (I % 16 || I > (1 << 22) || O > (1 << 24) || rows * std::max(I, O) > INT32_MAX) return 0;
-  if (rows <= 256) return I * O >= ((int64_t)1 << 25);
+  if (rows <= 256) return I * O >= (rows <= 128 ? (int64_t)5 << 23 : (int64_t)1 << 25);
   if (rows > 1024) return 0;
   double us = 0;
   mm8r_splits(nprob, rows, I, O, &us);

@@ -111,13 +111,13 @@ def test_mm8_linear_reads_its_tensors_where_they_are(monkeypatch, name):
 
 
 def test_mm8_reserve_hook_grows_the_slots_a_call_uses(monkeypatch):
-    """4096 -> 8192 (2^25 weights): above 64 rows the middle-row kernel and its
+    """4096 -> 16384 (2^26 weights): above 64 rows the middle-row kernel and its
     own slot, the tile GEMM's beside it for calls that stay on that one."""
     from rwkv7mi import native_quant_mm8 as Q
 
     grown = {}
     monkeypatch.setattr(Q._ws, "reserve", lambda device, need, slot, **k: grown.__setitem__(slot, need))
-    n, m = 4096, 8192
+    n, m = 4096, 16384
     b = _blocked(n, m)
     mod = Q.MM8Linear.from_packed(b.w_blk, b.mx, b.rx, b.my, b.ry, n, m)
     for rows in (17, 64, 65, 256):
@@ -148,7 +148,7 @@ def test_mm8_middle_rows_ready_a_capture_at_other_row_counts(monkeypatch, rows, 
     monkeypatch.setattr(_lib, "require_gpu", lambda *t, name: None)
     monkeypatch.setattr(_lib, "stream_of", lambda t: 0)
     monkeypatch.setattr(_lib, "call", lambda *a: None)
-    n, m = 4096, 8192
+    n, m = 4096, 16384
     b = _blocked(n, m)
     x, y = torch.zeros(rows, n, dtype=torch.float16), torch.zeros(rows, m, dtype=torch.float16)
     if route == "one":

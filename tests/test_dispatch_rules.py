@@ -66,3 +66,13 @@ def test_middle_row_kernel_splits_before_it_runs_an_epilogue(lib):
     """2048 -> 8192 at 512 rows: 53.7 us unsplit, 41.8 in two K ranges."""
     x = 512 * 2048 * 2 + 512 * 16
     assert lib.rwkv7mi_mm8t_rows_workspace_bytes(1, 512, 2048, 8192) >= x + 2 * 512 * 8192 * 4
+
+
+@pytest.mark.parametrize("rows,I,O,pays", [
+    (128, 8192, 4096, 0), (128, 4096, 8192, 0),     # 31.0 and 32.2 us; 28.5 and 29.6 on the 64-row tiles
+    (129, 8192, 4096, 1), (256, 4096, 8192, 1),     # 33.0 and 38.4 us; 38.8 and 45.5
+    (65, 10240, 4096, 1), (128, 16384, 4096, 1),    # 29.1 and 42.0 us; 40.2 and 44.0
+    (64, 16384, 4096, 0), (200, 2560, 10240, 0),
+])
+def test_middle_row_kernel_against_the_64_row_tiles(lib, rows, I, O, pays):
+    assert lib.rwkv7mi_mm8t_rows_pays(1, rows, I, O, 1) == pays
