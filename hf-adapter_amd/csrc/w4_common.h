@@ -28,7 +28,7 @@ __device__ __forceinline__ f16x8 w4_nibbles_to_f16(uint32_t d) {
 // shapes, the workspace of its K splits (0: none), and its launches (a
 // workspace below that runs unsplit).
 bool w4m_supported(int64_t rows, int64_t O, int64_t I, int64_t group, int act_dtype);
-int64_t w4m_workspace_bytes(int64_t rows, int64_t O, int64_t I, int64_t group);
+int64_t w4m_workspace_bytes(int64_t rows, int64_t O, int64_t I, int act_dtype, bool aff);
 int w4m_run(const void* x, const uint8_t* packed, const void* scales, const void* gbias, const void* bias,
             const void* residual, void* y, int64_t rows, int64_t O, int64_t I, int64_t group, int epilogue,
             int act_dtype, int scale_dtype, void* ws, int64_t ws_bytes, void* stream);

@@ -719,7 +719,7 @@ extern "C" int rwkv7mi_w4a_matmul(const void* x, const uint8_t* packed, const vo
 extern "C" int64_t rwkv7mi_w4_workspace_bytes(int64_t rows, int64_t O, int64_t I, int64_t group, int affine,
                                               int act_dtype) {
   if (rows <= 0 || O <= 0 || I <= 0 || (group != 128 && group != 256) || I % group) return 0;
-  return w4_many(rows, O, I, group, act_dtype, affine != 0) ? w4m_workspace_bytes(rows, O, I, group) : 0;
+  return w4_many(rows, O, I, group, act_dtype, affine != 0) ? w4m_workspace_bytes(rows, O, I, act_dtype, affine != 0) : 0;
 }
 
 extern "C" int rwkv7mi_w4_matmul_ws(const void* x, const uint8_t* packed, const void* scales, const void* biases,

@@ -261,17 +261,31 @@ __global__ __launch_bounds__(256) void w4m_reduce_kernel(const W4mArgs A) {
 // row tiles of a workgroup: 32 or 64 rows
 static int w4m_mt(int64_t rows) { return rows <= 32 ? 2 : 4; }
 
-static int w4m_splits(int64_t rows, int64_t O, int64_t I, int64_t group) {
-  const int64_t tiles = (rows + 16 * w4m_mt(rows) - 1) / (16 * w4m_mt(rows)) * ((O + 255) / 256);
+// K splits: a tile alone runs a serial chain of its blocks, with up to 256
+// workgroups 1.4 us each (64 rows; 1.2 for 32), with two on a CU 1.9 to 2.2 (1.4), the
+// affine form with its row sums and converted bf16 inputs more (measured unsplit,
+// 64 rows: fp16 768 -> 768 13.8 us, 1024 -> 1024 16.5, affine 19.0, bf16 17.6, both
+// 24.4; 96 rows 2048 -> 8192, 64 workgroups, 28.1; 4096 -> 16384 at 200 rows, 256,
+// 55.8, at 300, 320, 68.0).  A split adds the reduce, 0.4 us a partial, and the
+// partials' traffic, and an eager call then takes the host 15 us for the scratch
+// and the second launch.  Priced at 0.9 a block, 1024 -> 1024 ran unsplit at 64
+// rows and more (now 10.5-12 us) and 2048 -> 8192 at 96 (now 20.1).
+static int w4m_splits(int64_t rows, int64_t O, int64_t I, int act_dtype, bool aff) {
+  const int mt = w4m_mt(rows);
+  const int64_t tiles = (rows + 16 * mt - 1) / (16 * mt) * ((O + 255) / 256);
   const int64_t nblk = I / 128;
   const double pb = 4.0 * rows * ((O + 7) / 8 * 8);
+  const bool bf = act_dtype == RWKV7MI_BF16;
+  const double block = mt == 2 ? 1.2 : 1.4 * (aff && bf ? 1.75 : aff ? 1.15 : bf ? 1.06 : 1.0);
   int best = 1;
   double cost = 1e30;
   for (int S = 1; S <= 32 && (S == 1 || tiles * S <= 512); ++S) {
-    const int64_t bps = (nblk + S - 1) / S;
+    const int64_t bps = (nblk + S - 1) / S, wgs = tiles * S;
     if (S > 1 && (bps < 2 || (nblk + bps - 1) / bps != S)) continue;
-    const double t = (bps + 3) * (0.6 + 0.6 * std::max<double>(1.0, tiles * S / 256.0) * 0.5) * ((tiles * S + 511) / 512) +
-                     (S > 1 ? 5.0 + 2.0 * pb * S / 4e6 : 0.0);
+    const double two = (mt == 2 ? 0.25 : 1.0) * (0.5 + 0.3 * (std::min<int64_t>(wgs, 512) - 256) / 256.0);
+    const double per = block + (wgs > 256 ? two : 0.0);
+    const double k = (bps + 4) * per * ((wgs + 511) / 512);
+    const double t = S > 1 ? std::max(15.0, k + 3.0 + 0.4 * S + pb * S / 4e6) : k;
     if (t < cost) cost = t, best = S;
   }
   return best;
@@ -285,8 +299,8 @@ bool w4m_supported(int64_t rows, int64_t O, int64_t I, int64_t group, int act_dt
   return rows > 0 && rows <= INT32_MAX / 2 && O <= INT32_MAX / 2 && tiles <= INT32_MAX / 2;
 }
 
-int64_t w4m_workspace_bytes(int64_t rows, int64_t O, int64_t I, int64_t group) {
-  const int S = w4m_splits(rows, O, I, group);
+int64_t w4m_workspace_bytes(int64_t rows, int64_t O, int64_t I, int act_dtype, bool aff) {
+  const int S = w4m_splits(rows, O, I, act_dtype, aff);
   return S > 1 ? S * rows * ((O + 7) / 8 * 8) * 4 : 0;
 }
 
@@ -315,8 +329,9 @@ int w4m_run(const void* x, const uint8_t* packed, const void* scales, const void
   a.gsh = group == 256 ? 1 : 0;
   a.nt = (int)((O + 255) / 256);
   a.ldp = (int)((O + 7) / 8 * 8);
-  a.S = w4m_splits(rows, O, I, group);
-  if (!ws || (reinterpret_cast<uintptr_t>(ws) & 15) || ws_bytes < w4m_workspace_bytes(rows, O, I, group)) a.S = 1;
+  const bool aff = gbias != nullptr;
+  a.S = w4m_splits(rows, O, I, act_dtype, aff);
+  if (!ws || (reinterpret_cast<uintptr_t>(ws) & 15) || ws_bytes < w4m_workspace_bytes(rows, O, I, act_dtype, aff)) a.S = 1;
   a.bps = (int)((I / 128 + a.S - 1) / a.S);
   a.epilogue = epilogue;
   a.vec = O % 8 == 0 && !(reinterpret_cast<uintptr_t>(y) & 15) &&
@@ -325,7 +340,7 @@ int w4m_run(const void* x, const uint8_t* packed, const void* scales, const void
   const auto go = [&](auto ta, auto ts) {
     using TA = decltype(ta);
     using TS = decltype(ts);
-    return gbias ? w4m_go<true, TA, TS>(a, mt, as_stream(stream)) : w4m_go<false, TA, TS>(a, mt, as_stream(stream));
+    return aff ? w4m_go<true, TA, TS>(a, mt, as_stream(stream)) : w4m_go<false, TA, TS>(a, mt, as_stream(stream));
   };
   return dispatch_dtype(scale_dtype, [&](auto ts) {
     return act_dtype == RWKV7MI_BF16 ? go(__hip_bfloat16{}, ts) : go(__half{}, ts);
