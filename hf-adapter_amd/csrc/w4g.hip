@@ -597,15 +597,34 @@ static int w4t_go(int nw, int csw, dim3 grid, size_t lds, void* stream, const W4
   return w4t_launch<TA, TS, 8, 8, AFF>(grid, lds, stream, a);
 }
 
-// The many-row product (w4m.hip) from 17 rows on, and below that where the
-// rows' x does not fit the GEMV's LDS at once (it would re-stage x for every
-// column group).  Measured, GEMV -> many-row kernel: 17 rows 4096 x 4096 15 ->
-// 14 us (w4g_kernel there); staged once: 16 rows 4096 x 65536 54 -> 57, 9 rows
-// 4096 x 4096 8 -> 14; in chunks: bf16 16 rows 4096 x 65536 affine 246 -> 67,
-// 9 rows 16384 x 4096 48 -> 25, fp16 12 rows 29 -> 22.
+// 17 rows and more that stay on w4g_kernel: a launch per 64 rows and no scratch,
+// about 2 us + 3.3 us per 1024 inputs up to 32 rows and 5.2 above (bf16, whose x
+// it splits, and the affine form a third more each), while its workgroups, one
+// for 16 outputs, are all on the chip.  The many-row kernel needs 8 to 16 us there
+// and, where it splits K, a scratch tensor and a second launch, together 16 us
+// of host time a call.  Measured, w4g_kernel and many-row, GPU us: 17 rows fp16
+// 768 -> 768 5.3 and 7.8, 2048 -> 2048 8.5 and 9.7, 4096 -> 4096 15.6 and 14.4
+// (eager calls back to back 14.3 and 16.4), 4096 -> 8192 21.6 and 15.4; bf16
+// 3072 -> 4096 15.0 and 12.7, 4096 -> 4096 18.9 and 14.6; affine bf16 2560 -> 2560
+// 13.8 and 12; 48 rows fp16 1024 -> 1024 7.6 and 10.0, 2048 -> 4096 13.4 and 14.3,
+// 2048 -> 8192 18.0 and 16.3, 3072 -> 2048 18.9 and 14.4; 96 rows fp16 768 -> 768
+// 13.6 and 10.2 (eager 13.6 and 16), 1536 -> 2048 18.0 and 12.9; 128 rows 512 ->
+// 2048 11.1 and 11.1, affine 11.7 and 12.4, 768 -> 768 16.6 and 10.4.
+static bool w4_few(int64_t rows, int64_t O, int64_t I, bool f16, bool aff) {
+  const double k = I * (1.0 + 0.3 * !f16 + 0.3 * aff);
+  if (rows <= 32) return k <= 4100 && O * I <= ((int64_t)1 << 24);
+  if (rows <= 64) return k <= (rows <= 48 ? 2700 : 2100) && O * I <= ((int64_t)1 << (rows <= 48 && k <= 1700 ? 24 : 23));
+  return (rows <= 96 || (rows <= 128 && I <= 512)) && k <= 1340 && O * I <= ((int64_t)1 << 22);
+}
+
+// The many-row product (w4m.hip) above 16 rows but for those, and below that where
+// the rows' x does not fit the GEMV's LDS at once (it would re-stage x for every
+// column group).  Measured, GEMV -> many-row kernel: staged once: 16 rows
+// 4096 x 65536 54 -> 57, 9 rows 4096 x 4096 8 -> 14; in chunks: bf16 16 rows
+// 4096 x 65536 affine 246 -> 67, 9 rows 16384 x 4096 48 -> 25, fp16 12 rows 29 -> 22.
 static bool w4_many(int64_t rows, int64_t O, int64_t I, int64_t group, int act_dtype, bool aff) {
   if (!w4m_supported(rows, O, I, group, act_dtype)) return false;
-  if (rows > 16) return true;
+  if (rows > 16) return !w4_few(rows, O, I, act_dtype == RWKV7MI_F16, aff);
   // (7 rows bf16 16384 x 4096 in chunks: 27 us, 16 rows bf16 4096 x 4096: 15,
   // about the many-row kernel and its reduce there)
   if (rows <= 8 || O * I < ((int64_t)1 << 25)) return false;
@@ -661,10 +680,8 @@ static int w4_matmul(const char* who, const void* x, const uint8_t* packed, cons
   if (many)
     return w4m_run(x, packed, scales, gbias, bias, residual, y, rows, O, I, group, epilogue, act_dtype, scale_dtype,
                    ws, ws_bytes, stream);
-  // fp32 (and 16-bit inputs too wide for the kernels above, 16 rows a launch)
-  const int64_t step = act_dtype == RWKV7MI_F32 ? 64 : 16;
-  for (int64_t r0 = 0; r0 < rows; r0 += step) {
-    const int64_t nr = rows - r0 > step ? step : rows - r0;
+  for (int64_t r0 = 0; r0 < rows; r0 += 64) {
+    const int64_t nr = rows - r0 > 64 ? 64 : rows - r0;
     const int mt = nr <= 16 ? 1 : nr <= 32 ? 2 : 4;
     const char* xr = reinterpret_cast<const char*>(x) + r0 * I * esz;
     char* yr = reinterpret_cast<char*>(y) + r0 * O * esz;
@@ -678,18 +695,14 @@ static int w4_matmul(const char* who, const void* x, const uint8_t* packed, cons
   hipLaunchKernelGGL((w4g_kernel<MT_, TA, TS, AFF_>), grid, dim3(256), 0, as_stream(stream), (const TA*)xr, \
                      packed, (const TS*)scales, (const TS*)gbias, (const TS*)bias, (const TA*)rr, (TA*)yr,   \
                      (int)nr, (int)O, (int)I, (int)group, epilogue)
-        if constexpr (std::is_same<TA, float>::value) {
-          if (mt == 2) {
-            if (gbias) W4_LAUNCH(2, true);
-            else W4_LAUNCH(2, false);
-          } else if (mt == 4) {
-            if (gbias) W4_LAUNCH(4, true);
-            else W4_LAUNCH(4, false);
-          }
-        }
-        if (mt == 1) {
-          if (gbias) W4_LAUNCH(1, true);
-          else W4_LAUNCH(1, false);
+        if (gbias) {
+          if (mt == 1) W4_LAUNCH(1, true);
+          else if (mt == 2) W4_LAUNCH(2, true);
+          else W4_LAUNCH(4, true);
+        } else {
+          if (mt == 1) W4_LAUNCH(1, false);
+          else if (mt == 2) W4_LAUNCH(2, false);
+          else W4_LAUNCH(4, false);
         }
 #undef W4_LAUNCH
         return check_launch("w4g_kernel");

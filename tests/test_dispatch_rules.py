@@ -86,3 +86,12 @@ def test_middle_row_kernel_against_the_64_row_tiles(lib, rows, I, O, pays):
 ])
 def test_w4_splits(lib, rows, I, O, aff, dt, split):
     assert (lib.rwkv7mi_w4_workspace_bytes(rows, O, I, 128, aff, dt) > 0) is split
+
+
+@pytest.mark.parametrize("rows,I,O,aff,dt,few", [
+    (17, 4096, 4096, 0, 1, True), (32, 2048, 8192, 0, 1, True), (17, 2560, 2560, 1, 2, True), (64, 2048, 2048, 0, 1, True),
+    (17, 4096, 4096, 0, 2, False), (17, 4096, 16384, 0, 1, False), (33, 4096, 4096, 0, 1, False), (65, 2048, 2048, 0, 1, False),
+])
+def test_w4_few_rows_of_small_weights_take_no_scratch(lib, rows, I, O, aff, dt, few):
+    """They run on the 64-row launches of the GEMV's kernel; the others here split K."""
+    assert (lib.rwkv7mi_w4_workspace_bytes(rows, O, I, 128, aff, dt) == 0) is few

@@ -233,6 +233,8 @@ def test_w4_stream_gemv_edges(oracle, case):
     (520, 4096, 128, 100, torch.bfloat16, True, 0),
     (264, 16384, 128, 32, torch.float16, True, 0),
     (4100, 1152, 128, 131, torch.float16, False, 2),  # 9 blocks: uneven K ranges
+    (44012, 384, 128, 17, torch.float16, False, 0),   # three K blocks on the many-row kernel
+    (70004, 256, 256, 33, torch.bfloat16, False, 1),  # two blocks of one group
 ])
 def test_w4_many_rows(oracle, case):
     """More than 16 rows: row, column and K edges of the 32- and 64-row tiles,

@@ -1,0 +1,29 @@
+"""The kernels that calls run on at the lines of the dispatch rules that the
+library decides without a trace on the host."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from graph_routes import kernels
+
+pytestmark = pytest.mark.gpu
+F16, BF16 = torch.float16, torch.bfloat16
+
+
+def _r(*shape, dt=F16, scale=1.0):
+    return torch.randn(*shape, device="cuda", dtype=dt) * scale
+
+
+@pytest.mark.parametrize("rows,K,N,kernel", [(17, 768, 768, "w4g_kernel"), (64, 1024, 4096, "w4g_kernel"),
+                                             (48, 1024, 16384, "w4g_kernel"), (96, 1024, 1024, "w4g_kernel"),
+                                             (97, 1024, 16384, "w4m_kernel"), (17, 512, 65536, "w4m_kernel")])
+def test_w4_few_rows(rows, K, N, kernel):
+    from rwkv7mi.sm70_quant import w4_groupwise_linear
+
+    q = torch.randint(0, 256, (N, K // 2), device="cuda", dtype=torch.uint8)
+    s = torch.rand(N, K // 128, device="cuda").to(F16) * 0.02
+    x = _r(rows, K)
+    out = torch.empty(rows, N, device="cuda", dtype=F16)
+    launches = (rows + 63) // 64 if kernel == "w4g_kernel" else 1
+    assert kernels(lambda: w4_groupwise_linear(x, q, s, N, K, out=out)) == [kernel] * launches
