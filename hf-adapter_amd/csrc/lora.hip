@@ -333,6 +333,25 @@ extern "C" size_t rwkv7mi_lora_workspace_bytes(int64_t nprob, const int64_t* ran
   return (size_t)std::max(ks * nr * sr * (int64_t)sizeof(float), rows > LORA_PAIR_MIN ? rows * sr * 2 : (int64_t)0);
 }
 
+// fp16: whether the one-launch kernel of lora_seq.hip, one 1024-lane workgroup a
+// CU, beats the down / up pair.  Its round of up to 256 workgroups takes the same
+// time however many there are, about 10 us + 0.055 us x D, until the bytes count;
+// the pair's time grows with the rows, and narrow problems reach the round's
+// sooner.  Measured, seq and pair, us (workgroups): four problems 768 wide 53 and
+// 41 (80), 53 and 52 (112), 52 and 58 (144), 53 and 70 (196); 1024 wide 67 and 64
+// (144), 67 and 69 (160); 1536 wide 96 and 87 (144), 96 and 103 (160); 2048 wide
+// 131 and 124 (160), 150 and 150 (196), 160 and 160 (204); 4096 wide 303 and 303
+// (196); three problems 1024 wide 61 and 65 (147), 2560 wide 168 and 166 (165).
+// A second round that leaves most CUs idle goes to the pair where a round is
+// long: 2048 wide 265 and 211 (268), 264 and 255 (316), 321 and 327 (392); 4096
+// wide 545 and 410 (268), three problems 455 and 495 (330); but 768 wide 89 and 97
+// (268).
+static bool lora_seq_faster(int64_t nprob, int64_t rows, int64_t D) {
+  const int64_t wgs = (rows + 255) / 256 * nprob;
+  const int64_t line = D <= 1024 ? 18 + D / 8 : D <= 1536 ? 146 : std::min<int64_t>(200, 146 + (D - 1536) / 9);
+  return wgs >= line && !(D >= 1536 && wgs > 256 && wgs < 320);
+}
+
 static int lora_run(bool up, int64_t nprob, const void* const* xs, const void* const* w_down,
                     const void* const* w_up, const void* const* b_up, void* const* ys, const int64_t* ranks,
                     const int* act_down, const int* act_up, int64_t rows, int64_t D, int64_t A, int act_dtype,
@@ -391,9 +410,8 @@ static int lora_run(bool up, int64_t nprob, const void* const* xs, const void* c
   if (up && rows > LORA_PREFILL_ROWS &&
       (rows * std::max(D, A) * (int64_t)esz > INT32_MAX || A * LORA_MAXR * (int64_t)esz > INT32_MAX))
     return fail(RWKV7MI_EINVAL, "lora_multi: too large");
-  const bool full = act_dtype == RWKV7MI_F16 && (rows + 255) / 256 * nprob >= LORA_SEQ_WGS &&
-                    lora_seq_supported(batch, rows);
-  if (up && rows > LORA_PAIR_MIN && !full && lora_pair_supported(batch, rows, act_dtype, workspace, workspace_bytes))
+  const bool seq = act_dtype == RWKV7MI_F16 && lora_seq_faster(nprob, rows, D) && lora_seq_supported(batch, rows);
+  if (up && rows > LORA_PAIR_MIN && !seq && lora_pair_supported(batch, rows, act_dtype, workspace, workspace_bytes))
     return lora_pair_run(batch, rows, act_dtype, workspace, stream);
   if (up && rows > LORA_PREFILL_ROWS) {
     // many rows: the fused per-row-tile kernel, one launch, no partials

@@ -9,8 +9,7 @@ namespace rwkv7mi {
 enum { LORA_ACT_NONE = 0, LORA_ACT_TANH = 1, LORA_ACT_SIGMOID = 2 };
 constexpr int LORA_MAXR = 256;   // largest rank
 constexpr int LORA_PAIR_MIN = 32;         // above: the two-launch pair of lora_pair.hip (fp16 / bf16)
-constexpr int LORA_SEQ_WGS = 200;         // fp16: from this many of its workgroups on, lora_seq.hip instead
-constexpr int LORA_PREFILL_ROWS = 256;  // above: the fused many-row kernel (no workspace)
+constexpr int LORA_PREFILL_ROWS = 256;  // above: a call can run without a workspace (the one-launch kernels)
 
 struct LoraProb {
   const void* x;

@@ -14,10 +14,7 @@
 //         2048: 68 -> 16 (four 64-row split-K pairs)
 //   bf16  700 rows  475 -> 35 us, 16000 rows 1250 -> 371 (bf16 MFMAs on the
 //         values themselves instead of three fp16 ones on a split)
-// From LORA_SEQ_WGS workgroups of lora_seq_kernel on the chip is full and it
-// moves fewer bytes (seq against this pair, us): 16000 rows (250 workgroups) at
-// 4096 333 and 374, at 2048 166 and 194; 10240 rows (160) 276 and 245, 138 and
-// 127; 8000 rows (128) at 4096 247 and 184.
+// Against lora_seq_kernel: lora_seq_faster in lora.hip.
 // Against the split-K pair of lora.hip, us: 33 rows at 4096 18.7 -> 15.4, 64 rows
 // 22.2 -> 15.9, at 768 12.6 -> 9.3 and 16.4 -> 9.5; 16 rows at 4096 take 13.5 there,
 // and up to 32 rows keep it.
@@ -61,7 +58,7 @@ struct LpBatch {
 // against 16 now, 250 rows 33 and 21, 700 rows 44 and 35, 8000 215 and 184; 65
 // rows at 768 14 and 10).  So each of the four waves brings its own
 // 64-input steps (w, w + 4, ..) in by LDS DMA, 128 contiguous bytes per eight
-// lanes, into a ring of LP_R stages of its own: no barrier in the loop, only the
+// lanes, into a ring of R stages of its own: no barrier in the loop, only the
 // wave's own counters.  The 16-byte chunk c of a row lies at position c ^ (r % 8)
 // ^ (r / 8 % 2), which leaves the operand reads free of bank conflicts on gfx950.
 // The waves' sums meet in LDS, one 16-row tile at a time, added in wave order.

@@ -27,3 +27,17 @@ def test_w4_few_rows(rows, K, N, kernel):
     out = torch.empty(rows, N, device="cuda", dtype=F16)
     launches = (rows + 63) // 64 if kernel == "w4g_kernel" else 1
     assert kernels(lambda: w4_groupwise_linear(x, q, s, N, K, out=out)) == [kernel] * launches
+
+
+@pytest.mark.parametrize("rows,D,seq", [
+    (7000, 768, False), (9000, 768, True), (12500, 768, True), (8000, 1024, False), (12000, 1024, True),
+    (10240, 2048, False), (13000, 2048, True), (17000, 2048, False), (17000, 768, True), (32768, 1536, True),
+])
+def test_lora_one_launch_or_pair(rows, D, seq):
+    from rwkv7mi.fused_lora import fused_wavg_lora
+
+    ranks = (64, 64, 128, 32)
+    x = _r(rows, D)
+    dn, up = [_r(r, D, scale=0.02) for r in ranks], [_r(D, r, scale=0.02) for r in ranks]
+    got = kernels(lambda: fused_wavg_lora(x, x, x, x, *dn, *up, None, None, None, None))
+    assert got == (["lora_seq_kernel"] if seq else ["lora_mid_kernel", "lora_out_kernel"])
