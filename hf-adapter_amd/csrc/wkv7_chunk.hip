@@ -88,20 +88,25 @@ struct ChunkShared {
   int done[4][NSLOT];
 };
 
-// The two-kernel form: up to SPLIT_HEADS (batch, head) pairs and from SPLIT_MIN
+// The two-kernel form: up to SPLIT_ALWAYS (batch, head) pairs and from SPLIT_MIN
 // chunks on.  One workgroup per pair leaves the rest of the chip idle there while
 // its four producer waves set the pace (1.07 us a chunk whatever the head count);
 // made by all CUs the operands cost one chunk's time for 2048 chunks and the
 // chain alone runs at 0.70 us a chunk.  fp16, one launch -> two, us:
 //   tokens      128          256          1000          4096
-//   12 heads    15.2 -> 15.2 23.8 -> 20.5 73.3 -> 55.4  278 -> 199
-//   32 heads    15.4 -> 15.7 24.0 -> 21.8 73.6 -> 59.2  279 -> 227
-//   64 heads    15.8 -> 16.7 24.5 -> 24.2 74.7 -> 67.8  281 -> 271
+//   12 heads    15.2 -> 15.2 25.4 -> 22.3 75.2 -> 57.1  280 -> 202
+//   32 heads    15.4 -> 15.7 25.5 -> 23.1 76.4 -> 61.4  282 -> 230
+//   48 heads                 25.8 -> 25.1 76.7 -> 67.1  281 -> 262
+//   64 heads    15.8 -> 16.7 26.0 -> 26.0 76.8 -> 70.6  284 -> 282
 //   96 heads                              74.8 -> 76.2  286 -> 341
+// Between SPLIT_ALWAYS and SPLIT_HEADS pairs only the middle gains (64 heads, us:
+// 288 tokens 28.5 -> 29.9, 320 30.2 -> 31.8, 400 36.2 -> 34.9, 2000 142.6 ->
+// 138.4, 3000 210 -> 214; fp32 1500 109.2 -> 108.9, 2000 146 -> 152, 8192 575 ->
+// 620): SPLIT_FROM to SPLIT_TO chunks, fp32 SPLIT_TO32.
 // Slots past SPLIT_BYTES are made and used in further launch pairs: with 48 MB
 // the 64 heads took 74.2 us at 1000 tokens and 302 at 4096.
-constexpr int64_t SPLIT_HEADS = 64;
-constexpr int64_t SPLIT_MIN = 16;
+constexpr int64_t SPLIT_HEADS = 64, SPLIT_ALWAYS = 48;
+constexpr int64_t SPLIT_MIN = 16, SPLIT_FROM = 25, SPLIT_TO = 160, SPLIT_TO32 = 96;
 constexpr int64_t SPLIT_BYTES = 192 << 20;
 
 // what a producer wave of the two-kernel form keeps in LDS; the slots are global
@@ -825,9 +830,10 @@ __global__ __launch_bounds__(512, 1) void wkv7_chain_kernel(const ChunkSlot* __r
 }
 
 // chunks of one producer / chain launch pair: all of them up to SPLIT_BYTES of slots
-static int split_chunks(int64_t BH, int64_t T) {
+static int split_chunks(int64_t BH, int64_t T, bool f32) {
   const int64_t n = (T + CH - 1) / CH;
   if (BH <= 0 || n < SPLIT_MIN || BH > SPLIT_HEADS) return 0;
+  if (BH > SPLIT_ALWAYS && (n < SPLIT_FROM || n > (f32 ? SPLIT_TO32 : SPLIT_TO))) return 0;
   const int64_t cap = std::max<int64_t>(1, SPLIT_BYTES / (BH * (int64_t)sizeof(ChunkSlot)));
   const int64_t segs = (n + cap - 1) / cap;
   return (int)((n + segs - 1) / segs);
@@ -841,7 +847,7 @@ template <typename TA, typename TW, int WMODE>
 static int chunk_go(int64_t B, int64_t T, int64_t H, void* stream, const void* r, const void* w, const void* k,
                     const void* v, const void* kk, const void* a, const float* state_in, float* state_out,
                     void* y, void* ws, int64_t ws_bytes) {
-  const int xn = split_chunks(B * H, T);
+  const int xn = split_chunks(B * H, T, std::is_same<TA, float>::value);
   if (xn > 0 && ws && ws_bytes >= B * H * xn * (int64_t)sizeof(ChunkSlot) && !(reinterpret_cast<uintptr_t>(ws) & 15)) {
     static std::atomic<uint64_t> chain_raised{0};
     if (int rc = raise_dynamic_lds(reinterpret_cast<const void*>(&wkv7_chain_kernel<TA>), (int)sizeof(ChainShared), chain_raised,
@@ -875,7 +881,7 @@ static int chunk_go(int64_t B, int64_t T, int64_t H, void* stream, const void* r
 
 extern "C" int64_t rwkv7mi_wkv7_chunk_workspace_bytes(int64_t B, int64_t T, int64_t H) {
   if (B <= 0 || T <= 0 || H <= 0 || B > INT32_MAX || H > INT32_MAX || T > INT32_MAX) return 0;
-  return B * H * split_chunks(B * H, T) * (int64_t)sizeof(ChunkSlot);
+  return B * H * split_chunks(B * H, T, false) * (int64_t)sizeof(ChunkSlot);  // (fp32 uses it up to SPLIT_TO32)
 }
 
 extern "C" int rwkv7mi_wkv7_chunk_prefill_ws(const void* r, const void* w, const void* k, const void* v,
