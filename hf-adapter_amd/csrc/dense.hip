@@ -240,11 +240,14 @@ extern "C" int rwkv7mi_dense_multi_residual(const void* const* xs, const void* c
   // Two to four 16-bit rows with many short outputs: the GEMV's per-feature
   // reduction outweighs its loads there, and the tile kernel is faster (GEMV ->
   // tile, us: 4 rows 768 -> 65536 80 -> 26, 768 -> 3072 5.2 -> 3.2, 2048 -> 8192
-  // 10.8 -> 9.3; 2 rows 768 -> 65536 39 -> 26, but 2048 -> 65536 51 -> 61; the
-  // other way 4 rows 2048 -> 2048 3.8 -> 5.0, 3072 -> 768 3.9 -> 5.8).
+  // 10.8 -> 9.3, three 2048 -> 2048 10.8 -> 8.4; 2 rows 768 -> 65536 39 -> 26, but
+  // 2048 -> 65536 51 -> 61; the other way 4 rows 2048 -> 2048 3.8 -> 5.0, 3072 ->
+  // 768 3.9 -> 5.8).  Two fp16 rows below 3072 outputs stay: 768 -> 2048 3.63 ->
+  // 3.78, two 768 -> 768 3.42 -> 3.64 (bf16, whose GEMV converts, 3.73 -> 3.42).
   int64_t nsum = 0, kmax = 0;
   for (int i = 0; i < nprob; ++i) nsum += Ns[i], kmax = std::max(kmax, Ks[i]);
-  const bool wide = nsum >= 2 * kmax && (rows >= 3 || (rows == 2 && kmax <= 1024)) &&
+  const bool f16 = act_dtype == RWKV7MI_F16;
+  const bool wide = nsum >= 2 * kmax && (rows >= 3 || (rows == 2 && kmax <= 1024 && (!f16 || nsum >= 3072))) &&
                     dense_tile_supported(batch, rows, act_dtype);
   if (rows <= 4 && !wide) {  // the GEMV form: tiles of four features, one wave each
     DenseBatch gb = batch;
@@ -267,7 +270,8 @@ extern "C" int rwkv7mi_dense_multi_residual(const void* const* xs, const void* c
       return check_launch("dense_gemv_kernel");
     });
   }
-  if (dense_tile_supported(batch, rows, act_dtype)) return dense_tile_run(batch, rows, act_dtype, 1, nullptr, 0, stream);
+  if (dense_tile_supported(batch, rows, act_dtype))
+    return dense_tile_run(batch, rows, act_dtype, 1, nullptr, 0, stream);
   // fp32 (and 16-bit inputs too wide for the tile kernel, 16 rows a launch)
   const int64_t step = act_dtype == RWKV7MI_F32 ? 64 : 16;
   for (int64_t r0 = 0; r0 < rows; r0 += step) {

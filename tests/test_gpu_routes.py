@@ -41,3 +41,22 @@ def test_lora_one_launch_or_pair(rows, D, seq):
     dn, up = [_r(r, D, scale=0.02) for r in ranks], [_r(D, r, scale=0.02) for r in ranks]
     got = kernels(lambda: fused_wavg_lora(x, x, x, x, *dn, *up, None, None, None, None))
     assert got == (["lora_seq_kernel"] if seq else ["lora_mid_kernel", "lora_out_kernel"])
+
+
+def _dense(rows, K, Ns, dt):
+    from rwkv7mi.fused_lora import dense_multi
+
+    x = _r(rows, K, dt=dt)
+    probs = [(x, _r(n, K, dt=dt, scale=0.05), None, torch.empty(rows, n, device="cuda", dtype=dt), 0) for n in Ns]
+    got = kernels(lambda: dense_multi(probs, rows))
+    step = 2.0 ** -11 if dt == F16 else 2.0 ** -8  # one rounding of the output, fp32 sums
+    for _, W, _, y, _ in probs:
+        ref = x.double() @ W.double().t()
+        assert bool(((y.double() - ref).abs() <= step * ref.abs() + 2e-5 * ref.abs().max()).all())
+    return got
+
+
+@pytest.mark.parametrize("Ns,dt,kernel", [((2048,), F16, "dense_gemv_kernel"), ((768, 768), F16, "dense_gemv_kernel"),
+                                          ((3072,), F16, "dense_tile_kernel"), ((768, 768), BF16, "dense_tile_kernel")])
+def test_dense_two_rows(Ns, dt, kernel):
+    assert _dense(2, 768, Ns, dt) == [kernel]
