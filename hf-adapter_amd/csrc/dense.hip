@@ -249,6 +249,12 @@ extern "C" int rwkv7mi_dense_multi_residual(const void* const* xs, const void* c
   const bool f16 = act_dtype == RWKV7MI_F16;
   const bool wide = nsum >= 2 * kmax && (rows >= 3 || (rows == 2 && kmax <= 1024 && (!f16 || nsum >= 3072))) &&
                     dense_tile_supported(batch, rows, act_dtype);
+  // Up to 12 fp16 rows (16 up to 512 inputs) of many short outputs: one round of
+  // 16-column tiles whose waves split K beats the tile kernel's 64 columns a
+  // workgroup (us: 5 rows 512 -> 65536 15.5 against 23.0, 768 -> 65536 22.9 and
+  // 26.5, 1024 -> 32768 15.0 and 18.4; 12 rows 27.1 and 26.7, 17.9 and 18.7; 16
+  // rows 512 -> 32768 11.2 and 12.4, 768 -> 65536 29.7 and 26.9).
+  const bool short_k = f16 && kmax <= 1024 && nsum >= 16384 && rows > 4 && rows <= (kmax <= 512 ? 16 : 12);
   if (rows <= 4 && !wide) {  // the GEMV form: tiles of four features, one wave each
     DenseBatch gb = batch;
     int gt = 0;
@@ -270,7 +276,7 @@ extern "C" int rwkv7mi_dense_multi_residual(const void* const* xs, const void* c
       return check_launch("dense_gemv_kernel");
     });
   }
-  if (dense_tile_supported(batch, rows, act_dtype))
+  if (!short_k && dense_tile_supported(batch, rows, act_dtype))
     return dense_tile_run(batch, rows, act_dtype, 1, nullptr, 0, stream);
   // fp32 (and 16-bit inputs too wide for the tile kernel, 16 rows a launch)
   const int64_t step = act_dtype == RWKV7MI_F32 ? 64 : 16;

@@ -60,3 +60,13 @@ def _dense(rows, K, Ns, dt):
                                           ((3072,), F16, "dense_tile_kernel"), ((768, 768), BF16, "dense_tile_kernel")])
 def test_dense_two_rows(Ns, dt, kernel):
     assert _dense(2, 768, Ns, dt) == [kernel]
+
+
+@pytest.mark.parametrize("rows,K,Ns,dt,kernel", [
+    (5, 768, (32768,), F16, "dense_kernel"), (12, 1024, (16380,) + (8,), F16, "dense_kernel"),
+    (16, 512, (65536,), F16, "dense_kernel"), (13, 768, (32768,), F16, "dense_tile_kernel"),
+    (5, 768, (32768,), BF16, "dense_tile_kernel"), (5, 1536, (32768,), F16, "dense_tile_kernel"),
+    (4, 768, (32768,), F16, "dense_tile_kernel"),
+])
+def test_dense_few_rows_of_many_short_outputs(rows, K, Ns, dt, kernel):
+    assert _dense(rows, K, Ns, dt) == [kernel]
