@@ -208,7 +208,6 @@ def test_sequence_shift_mix_runs_equal_one_token_calls(D, dt, norm):
     assert torch.equal(last, p6) and torch.equal(last_f, p1)
 
 
-# rows above 256 take the fused many-row kernel (prefills)
 @pytest.mark.parametrize("rows,D,ranks", [(1, 4096, (64, 64, 128, 32)), (8, 2048, (64, 64, 128, 32)),
                                           (40, 768, (64, 64, 128, 32)), (64, 4096, (64, 64, 128, 32)),
                                           (100, 2048, (64, 64, 128, 32)), (300, 256, (64, 64, 128, 32)),
@@ -216,9 +215,7 @@ def test_sequence_shift_mix_runs_equal_one_token_calls(D, dt, norm):
                                           (513, 768, (96, 32, 64, 128)), (700, 320, (64, 48, 128, 32))])
 def test_wavg_lora(oracle, rows, D, ranks):
     """fp16 W/A/G/V LoRA against the fp64 oracle: decode sizes (split-K down,
-    up kernel), and above 256 rows the many-row kernels (ranks that are
-    multiples of 32 with D a multiple of 64: the LDS-shared form; the last case
-    the per-row-tile form)."""
+    up kernel) and, above 32 rows, the down / up pair over all rows."""
     from rwkv7mi.fused_lora import fused_wavg_lora
 
     rng = np.random.default_rng(rows + D)
@@ -290,8 +287,8 @@ def test_dense_tile_edges(dt, rows, K, Ns):
 @pytest.mark.parametrize("rows,K,N,epi", [(257, 768, 768, 2), (300, 3072, 104, 1), (520, 784, 3072, 0),
                                           (700, 4096, 264, 2), (1500, 2048, 2048, 0)])
 def test_dense_prefill_routes(dt, rows, K, N, epi):
-    """Above 256 rows: the tile kernel, its K splits (whose partials take the
-    place of W's copy) and the 256 x 256 form, one and three products a call."""
+    """Above 256 rows: the tile kernel and the 256 x 256 form, one and three
+    products a call."""
     from rwkv7mi.model import DenseLinear
 
     rng = np.random.default_rng(rows + K + N)
@@ -311,6 +308,83 @@ def test_dense_prefill_routes(dt, rows, K, N, epi):
         assert np.all(np.abs(_f(o) - r) <= tol(r))
     ref = np.maximum(refs[0], 0) ** 2 if epi == 1 else refs[0] + (_f(res) if epi == 2 else 0)
     assert np.all(np.abs(_f(y) - ref) <= tol(ref))
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,K,N,k,epi", [(300, 8192, 2048, 1, 2), (300, 8192, 2044, 1, 1), (257, 4096, 1000, 1, 0),
+                                            (600, 6400, 520, 1, 2), (300, 16384, 768, 3, 0), (600, 8192, 262, 3, 0)])
+def test_dense_prefill_k_splits(dt, rows, K, N, k, epi):
+    """The tile kernel in three to eight K ranges (uneven ones too), whose fp32
+    partials take the place of W's copy and are added by the prefill GEMM's
+    reduce: bias, relu^2, a residual that is the output, widths that end inside
+    its 8-column runs, one and three products."""
+    from graph_routes import kernels
+    from rwkv7mi.model import DenseLinear
+
+    rng = np.random.default_rng(rows + K + N)
+    lins = [DenseLinear(_t(rng.standard_normal((N, K)) * 0.05, dt), _t(rng.standard_normal(N) * 0.1, dt))
+            for _ in range(k)]
+    xs = [_t(rng.standard_normal((rows, K)), dt) for _ in range(k)]
+    outs = [torch.full((rows, N), float("nan"), device="cuda", dtype=dt) for _ in range(k)]
+    res = _t(rng.standard_normal((rows, N)), dt)
+
+    def call():
+        if k > 1:
+            assert DenseLinear.apply_group(lins, xs, outs)
+            return
+        outs[0].copy_(res)
+        lins[0].apply(xs[0], outs[0], act=3 if epi == 1 else 0, residual=outs[0] if epi == 2 else None)
+
+    assert kernels(call) == ["dense_tile_kernel", "mm8h_reduce_kernel"]
+    for o in outs:
+        o.fill_(float("nan"))
+    call()
+    torch.cuda.synchronize()
+    step = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8  # one rounding of the output, fp32 sums
+    for o, x, l in zip(outs, xs, lins):
+        ref = _f(x) @ _f(l.weight).T + _f(l.bias)
+        ref = np.maximum(ref, 0) ** 2 if epi == 1 else ref + (_f(res) if epi == 2 else 0)
+        assert np.all(np.abs(_f(o) - ref) <= step * np.abs(ref) + 2e-5 * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("rows,D,ranks,ws", [(300, 256, (64, 64, 128, 32), False), (257, 512, (64, 64, 128, 32), False),
+                                             (1000, 4096, (64, 64, 128, 32), False), (513, 768, (96, 32, 64, 128), False),
+                                             (3072, 256, (64, 64, 128, 32), True), (3073, 256, (64, 64, 128, 32), True)])
+def test_lora_one_launch_form(oracle, rows, D, ranks, ws):
+    """The one-launch kernel of the largest fp16 prefills (also any call above
+    256 rows without a workspace) against the fp64 oracle, and both sides of the
+    line between it and the pair at 256 wide."""
+    import ctypes
+
+    from graph_routes import kernels
+    from rwkv7mi import _lib
+    from rwkv7mi.fused_lora import fused_wavg_lora
+
+    rng = np.random.default_rng(rows + D)
+    xs = [_t(rng.standard_normal((rows, D))) for _ in range(4)]
+    downs = [_t(rng.standard_normal((r, D)) * 0.02) for r in ranks]
+    ups = [_t(rng.standard_normal((D, r)) * 0.1) for r in ranks]
+    biases = [_t(rng.standard_normal(D) * 0.01), _t(rng.standard_normal(D) * 0.01), None,
+              _t(rng.standard_normal(D) * 0.01)]
+    if ws:
+        outs = fused_wavg_lora(*xs, *downs, *ups, *biases)
+        route = kernels(lambda: fused_wavg_lora(*xs, *downs, *ups, *biases))
+    else:
+        outs = [torch.full((rows, D), float("nan"), device="cuda", dtype=torch.float16) for _ in range(4)]
+        arr, k32 = _lib.ptr_array, lambda v: (ctypes.c_int * 4)(*v)
+
+        def call():
+            _lib.call("rwkv7mi_lora_multi", 4, arr(xs), arr(downs), arr(ups), arr(biases), arr(outs),
+                      (ctypes.c_int64 * 4)(*ranks), k32((1, 0, 2, 0)), k32((0, 0, 0, 2)), rows, D, D, _lib.F16, None, 0,
+                      _lib.stream_of(xs[0]))
+
+        route = kernels(call)
+    torch.cuda.synchronize()
+    assert route == (["lora_mid_kernel", "lora_out_kernel"] if rows == 3072 else ["lora_seq_kernel"])
+    ref = oracle.wavg_lora(*map(_f, xs), *map(_f, downs), *map(_f, ups),
+                           *[None if b is None else _f(b) for b in biases])
+    for g, r in zip(outs, ref):
+        _ok(g, r)
 
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
