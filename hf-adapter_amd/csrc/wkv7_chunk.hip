@@ -99,14 +99,17 @@ struct ChunkShared {
 //   48 heads                 25.8 -> 25.1 76.7 -> 67.1  281 -> 262
 //   64 heads    15.8 -> 16.7 26.0 -> 26.0 76.8 -> 70.6  284 -> 282
 //   96 heads                              74.8 -> 76.2  286 -> 341
-// Between SPLIT_ALWAYS and SPLIT_HEADS pairs only the middle gains (64 heads, us:
-// 288 tokens 28.5 -> 29.9, 320 30.2 -> 31.8, 400 36.2 -> 34.9, 2000 142.6 ->
-// 138.4, 3000 210 -> 214; fp32 1500 109.2 -> 108.9, 2000 146 -> 152, 8192 575 ->
-// 620): SPLIT_FROM to SPLIT_TO chunks, fp32 SPLIT_TO32.
+// Between SPLIT_ALWAYS and SPLIT_HEADS pairs only the middle gains, from
+// SPLIT_FROM chunks to a type's SPLIT_TO (64 heads, us: fp16 288 tokens 28.5 ->
+// 29.9, 320 30.2 -> 31.8, 400 36.2 -> 34.9, 2000 142.6 -> 138.4, 4000 273 -> 270,
+// 8192 564 -> 573-581; bf16 320 30.6 -> 31.8, 4000 284 -> 270, 8192 575 -> 565-569;
+// fp32 1500 109.2 -> 108.9, 2000 146 -> 152, 8192 575 -> 620).
 // Slots past SPLIT_BYTES are made and used in further launch pairs: with 48 MB
 // the 64 heads took 74.2 us at 1000 tokens and 302 at 4096.
 constexpr int64_t SPLIT_HEADS = 64, SPLIT_ALWAYS = 48;
-constexpr int64_t SPLIT_MIN = 16, SPLIT_FROM = 25, SPLIT_TO = 160, SPLIT_TO32 = 96;
+constexpr int64_t SPLIT_MIN = 16, SPLIT_FROM = 25;
+template <typename TA> constexpr int64_t SPLIT_TO = std::is_same<TA, float>::value ? 96 : 256;
+template <> constexpr int64_t SPLIT_TO<__hip_bfloat16> = INT64_MAX;
 constexpr int64_t SPLIT_BYTES = 192 << 20;
 
 // what a producer wave of the two-kernel form keeps in LDS; the slots are global
@@ -830,10 +833,11 @@ __global__ __launch_bounds__(512, 1) void wkv7_chain_kernel(const ChunkSlot* __r
 }
 
 // chunks of one producer / chain launch pair: all of them up to SPLIT_BYTES of slots
-static int split_chunks(int64_t BH, int64_t T, bool f32) {
+template <typename TA>
+static int split_chunks(int64_t BH, int64_t T) {
   const int64_t n = (T + CH - 1) / CH;
   if (BH <= 0 || n < SPLIT_MIN || BH > SPLIT_HEADS) return 0;
-  if (BH > SPLIT_ALWAYS && (n < SPLIT_FROM || n > (f32 ? SPLIT_TO32 : SPLIT_TO))) return 0;
+  if (BH > SPLIT_ALWAYS && (n < SPLIT_FROM || n > SPLIT_TO<TA>)) return 0;
   const int64_t cap = std::max<int64_t>(1, SPLIT_BYTES / (BH * (int64_t)sizeof(ChunkSlot)));
   const int64_t segs = (n + cap - 1) / cap;
   return (int)((n + segs - 1) / segs);
@@ -847,7 +851,7 @@ template <typename TA, typename TW, int WMODE>
 static int chunk_go(int64_t B, int64_t T, int64_t H, void* stream, const void* r, const void* w, const void* k,
                     const void* v, const void* kk, const void* a, const float* state_in, float* state_out,
                     void* y, void* ws, int64_t ws_bytes) {
-  const int xn = split_chunks(B * H, T, std::is_same<TA, float>::value);
+  const int xn = split_chunks<TA>(B * H, T);
   if (xn > 0 && ws && ws_bytes >= B * H * xn * (int64_t)sizeof(ChunkSlot) && !(reinterpret_cast<uintptr_t>(ws) & 15)) {
     static std::atomic<uint64_t> chain_raised{0};
     if (int rc = raise_dynamic_lds(reinterpret_cast<const void*>(&wkv7_chain_kernel<TA>), (int)sizeof(ChainShared), chain_raised,
@@ -881,7 +885,7 @@ static int chunk_go(int64_t B, int64_t T, int64_t H, void* stream, const void* r
 
 extern "C" int64_t rwkv7mi_wkv7_chunk_workspace_bytes(int64_t B, int64_t T, int64_t H) {
   if (B <= 0 || T <= 0 || H <= 0 || B > INT32_MAX || H > INT32_MAX || T > INT32_MAX) return 0;
-  return B * H * split_chunks(B * H, T, false) * (int64_t)sizeof(ChunkSlot);  // (fp32 uses it up to SPLIT_TO32)
+  return B * H * split_chunks<__hip_bfloat16>(B * H, T) * (int64_t)sizeof(ChunkSlot);  // (the type with the longest range)
 }
 
 extern "C" int rwkv7mi_wkv7_chunk_prefill_ws(const void* r, const void* w, const void* k, const void* v,

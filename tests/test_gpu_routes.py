@@ -70,3 +70,16 @@ def test_dense_two_rows(Ns, dt, kernel):
 ])
 def test_dense_few_rows_of_many_short_outputs(rows, K, Ns, dt, kernel):
     assert _dense(rows, K, Ns, dt) == [kernel]
+
+
+@pytest.mark.parametrize("T,H,dt,two", [(320, 64, F16, False), (400, 64, F16, True), (1500, 64, torch.float32, True),
+                                        (2000, 64, torch.float32, False), (2000, 48, torch.float32, True),
+                                        (4200, 64, F16, False), (4200, 64, BF16, True)])
+def test_scan_one_launch_or_two(T, H, dt, two):
+    from rwkv7mi import dplr_chunk_scan
+
+    k = torch.nn.functional.normalize(_r(1, T, H, 64, dt=torch.float32), dim=-1).to(dt)
+    w = torch.full((1, T, H, 64), 0.6, device="cuda")
+    st = torch.zeros(1, H, 64, 64, device="cuda")
+    got = kernels(lambda: dplr_chunk_scan(_r(1, T, H, 64, dt=dt), w, k, k, k, k.abs(), st))
+    assert set(got) == ({"wkv7_chunk_kernel", "wkv7_chain_kernel"} if two else {"wkv7_chunk_kernel"})
