@@ -16,9 +16,9 @@
 //
 // Measured (fp16, time a call in a graph; operands straight into registers ->
 // the ring): 512 rows, three 768 -> 768 in one launch 20.0 -> 17.4 us, 768 ->
-// 3072 19.9 -> 17.1, 3072 -> 768 in K splits 21.8 -> 11.8; 64 rows, three 2048 ->
-// 2048 16.3 -> 10.6; 8 rows 3072 -> 768 7.3 -> 4.9; 1000 rows 8192 -> 2048 127 ->
-// 68.  (The 256 x 256 form and its copy of W took 38 us for 512 rows 768 -> 3072
+// 3072 19.9 -> 17.1, 3072 -> 768 (unsplit) 21.8 -> 11.8; 64 rows, three 2048 ->
+// 2048 16.3 -> 10.6; 8 rows 3072 -> 768 7.3 -> 4.9; 1000 rows 8192 -> 2048 (also
+// unsplit) 127 -> 68.  (The 256 x 256 form and its copy of W took 38 us for 512 rows 768 -> 3072
 // and 101 for 3072 -> 768.)
 #include <algorithm>
 

@@ -283,9 +283,10 @@ class DenseLinear:
 class QuantLinear:
     """MM8 Linear, all on HIP kernels: the fused blocked dequant GEMV for up to
     ``GEMV_ROWS`` rows, the 64-row MFMA tile GEMM (split K) up to ``GEMM_ROWS``
-    rows, and above that the prefill GEMM over the materialised fp16
-    dequantised weight (``mm8_many_rows_into``).  Modules whose bytes are not blocked
-    take MM8Linear's own route."""
+    rows, above that the prefill GEMM over the materialised fp16 dequantised
+    weight, and between them the 128-row tile kernel where it is faster
+    (``mm8_many_rows_into``).  Modules whose bytes are not blocked take
+    MM8Linear's own route."""
 
     GEMV_ROWS = GEMV_ROWS
     GEMM_ROWS = GEMM_ROWS

@@ -454,9 +454,10 @@ def _linear_into(x2, w, mx, rx, my, ry, bias, residual, out, epilogue) -> bool:
     calls that need the general route: mixed prefill dtypes or row chunks, an
     unaligned operand of the middle-row form, no room under graph capture.
     The general route's lists, pointer arrays and size queries cost more host
-    time than a small product's kernel runs: the 4096 -> 16384 -> 4096 FFN pair
-    took 49.4 us at 1 row with it and takes 30.2 us (31 us of kernels) on this
-    one, 58.3 -> 46.6 us at 16 rows, 63.4 -> 57.6 us at 200."""
+    time than a small product's kernel runs: called eagerly the 4096 -> 16384 ->
+    4096 FFN pair took 49.4 us at 1 row with it and takes 30.2 us on this one,
+    58.3 -> 46.6 us at 16 rows, the 2048 -> 8192 -> 2048 pair 50.7 -> 21.4 us at 1
+    row.  The kernels are the same: a captured step gains nothing."""
     rows, n = x2.shape
     m = out.shape[1]
     dt = _lib.dtype_code(x2)

@@ -7,8 +7,10 @@ chunk kernel (chunk 16, bf16x3 MFMA products, fp32 state in registers).
 divisible by chunk_size, chunk_size in {16, 32, 64}); ``dplr_chunk_scan``
 accepts any T like the reference's pure-torch oracle.  The kernel always uses
 16-token chunks internally (one workgroup of four state waves and four chunk
-producer waves per (batch, head)); ``chunk_size`` does not change the result
-beyond rounding.
+producer waves per (batch, head), or for few heads over many chunks a launch that
+makes the chunks' operands and one that moves the states, through up to 192 MB of
+scratch of the call's own); ``chunk_size`` does not change the result beyond
+rounding.
 """
 from __future__ import annotations
 

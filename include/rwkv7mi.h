@@ -149,7 +149,8 @@ int rwkv7mi_wkv7_chunk_prefill(const void* r, const void* w, const void* k,
 
 /* The same over a 16-byte aligned workspace of rwkv7mi_wkv7_chunk_workspace_bytes
  * (0: none is used): few heads then run as a launch that makes the chunks'
- * operands on the whole chip and one that moves the states over them.  Without
+ * operands on the whole chip and one that moves the states over them (up to 192
+ * MB of operands at a time).  Without
  * (or with a smaller) workspace: rwkv7mi_wkv7_chunk_prefill, the same results. */
 int64_t rwkv7mi_wkv7_chunk_workspace_bytes(int64_t B, int64_t T, int64_t H);
 int rwkv7mi_wkv7_chunk_prefill_ws(const void* r, const void* w, const void* k,
@@ -490,7 +491,7 @@ int rwkv7mi_mm8t_linear(int form, const void* x, const uint8_t* w_blk,
                         int64_t ws_bytes, void* stream);
 
 /* rwkv7mi_mm8t_gemm_multi (same arguments and results to rounding) for middle
- * row counts, fp16 / bf16 activations: 64-row x 256-column tiles, K split only
+ * row counts, fp16 / bf16 activations: 128-row x 256-column tiles, K split only
  * where they do not fill the chip.  The workspace (256-byte aligned) holds
  * rwkv7mi_mm8t_rows_workspace_bytes. */
 int64_t rwkv7mi_mm8t_rows_workspace_bytes(int nprob, int64_t rows, int64_t I, int64_t O);
@@ -679,9 +680,11 @@ int rwkv7mi_argmax_rows_ws(const void* x, int64_t rows, int64_t n, int64_t ld,
 
 /* ------------------------------------------------------------------ LoRA */
 
-/* Bytes of workspace rwkv7mi_lora_multi uses: fp32 split-K partials up to 32
- * rows (fp32: 64), the intermediate in the activation type above (rows x the ranks' sum;
- * more than 256 rows also run without one, on a slower kernel). */
+/* Bytes of workspace rwkv7mi_lora_multi uses: fp32 split-K partials of one
+ * 64-row chunk (every call of up to 256 rows needs room for them; fp16 / bf16
+ * use them up to 32 rows and for ranks above 128, fp32 up to 256), and above 32
+ * rows the intermediate in the activation type (rows x the ranks' sum).  More
+ * than 256 rows also run without a workspace. */
 size_t rwkv7mi_lora_workspace_bytes(int64_t nprob, const int64_t* ranks,
                                     int64_t rows, int64_t D);
 

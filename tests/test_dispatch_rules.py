@@ -80,7 +80,7 @@ def test_middle_row_kernel_against_the_64_row_tiles(lib, rows, I, O, pays):
 
 @pytest.mark.parametrize("rows,I,O,aff,dt,split", [
     (128, 1024, 1024, 0, 1, True), (512, 2048, 2048, 0, 1, True),      # 16.6 and 28.1 us unsplit, 11 and 20 split
-    (96, 2048, 8192, 1, 2, True),                                      # 46.9 us unsplit (start of the range), 24.6 split
+    (96, 2048, 8192, 1, 2, True),                                      # 46.9 us unsplit, 24.6 split
     (128, 768, 768, 0, 1, False),                                      # six blocks: 13.8 us in one launch
     (384, 4096, 16384, 0, 1, False), (1000, 4096, 4096, 0, 1, False),  # the tiles fill the chip
 ])
